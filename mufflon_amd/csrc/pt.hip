@@ -1,20 +1,23 @@
 // Path tracer megakernel for gfx950: the GPU device of Mufflon's pure path
-// tracer (GpuPathTracer, gpu_pt.cu:54-152), one iteration per launch.
+// tracer (GpuPathTracer, gpu_pt.cu:54-152), every iteration of a call in one
+// launch.
 //
-// One thread per pixel, 16x16 pixel tiles per 256-thread block (a wave covers
-// a 16x4 pixel patch, which keeps primary rays coherent). Per pixel it runs
-// pt_sample (pt_common.hpp:75-156): pinhole camera sample, BSDF sampling with
-// Russian roulette (random_walk.hpp:38-112), next-event estimation through the
-// light tree with MIS (light_tree_sampling.hpp:195-329, light_sampling.hpp),
-// emission hits weighted with light_pdf (:340-412), and accumulates the
-// iteration's Radiance and Hit ID into the running means of
-// output_handler_variance.hpp:7-31 in its epilogue (no separate update pass,
-// no atomics: each pixel belongs to one thread). The RNG is Mufflon's PCG64,
-// one 64-bit state per pixel, seeded as in gpu_pt.cu:140-152.
+// A lane owns a pixel and runs its iterations one after the other (each
+// continues the pixel's generator): pt_sample (pt_common.hpp:75-156) with the
+// pinhole camera sample, BSDF sampling with Russian roulette
+// (random_walk.hpp:38-112), next-event estimation through the light tree with
+// MIS (light_tree_sampling.hpp:195-329, light_sampling.hpp), emission hits
+// weighted with light_pdf (:340-412). At the end of each path it folds the
+// iteration's targets into the running means of
+// output_handler_variance.hpp:7-31 (no separate update pass, no atomics: each
+// pixel belongs to one lane). The RNG is Mufflon's PCG64, one 64-bit state per
+// pixel, seeded as in gpu_pt.cu:140-152.
 //
 // Float expressions keep the reference's operand order; transcendental
 // functions of the samplers are evaluated in double and rounded once
 // (correctly rounded sin/cos), the same definition as the CPU oracle's.
+#include <algorithm>
+
 #include "pt_path.hpp"
 
 namespace mfh {
@@ -24,74 +27,150 @@ namespace {
 using namespace shade;
 using namespace path;
 
-constexpr int kPtTile = 16;
+constexpr int kPtTile = 8;  // a wave starts on an 8x8 pixel tile
 constexpr int kPtThreads = kPtTile * kPtTile;
+// Fewest lanes of a wave that take pixels (Cornell box 256x256, 64 / 32 / 16
+// lanes: 14.1 / 12.7 / 10.6 ms; 200x151 room, 64 / 32 / 16 / 8: 0.72 / 0.63 /
+// 0.57 / 0.55 ms; the terrain image, which fills the chip, 24.5 / 34.4 / 47.5).
+constexpr int kPtMinLanes = 8;
 
+// Path regeneration. Paths end after very different numbers of segments (2.5
+// of 8 on average in the Cornell box), and a wave that runs one path per lane
+// works until its longest has ended, a launch per iteration until the longest
+// of the image has. So a turn of the loop below is one path segment (closest
+// hit, vertex, next-event estimate, walk), and a lane whose path has ended
+// starts its pixel's next iteration in the next turn, or takes another pixel
+// from the queue once the call's iterations are done. Against one path per
+// lane and one launch per iteration: Cornell box 256x256, 16 iterations 22.3
+// -> 10.6 ms; terrain of 2.1M triangles and 2048 instances, 1280x720, 4
+// iterations 31.5 -> 24.5 ms; one iteration of a 200x151 room 0.82 -> 0.55 ms.
+// What bounds it now is the traversal's chain of dependent loads (80 % of a
+// wave's time; about 1500 cycles a node or triangle step in the Cornell box).
+//
+// The shadow ray of a vertex is traced after the walk from it (the random
+// numbers of both are drawn before, in the order of pt_sample): through that
+// traversal the vertex, about 45 registers, is no longer live.
+//
 // kLeaf: triangles of a BVH leaf loaded ahead of their tests (1 or 8).
-// Three waves per SIMD: left to itself the compiler gives the whole path loop
-// 256 VGPRs + ~80 AGPRs (one wave per SIMD), too few waves to hide the
-// traversal's memory latency; at three it spills some state to scratch and
-// the 10M-triangle terrain iteration drops from 27.4 to 14.7 ms (leaf batch
-// 8; 34.8 -> 18.3 ms with 1), two waves 17.6 ms, four 17.6 ms (more spills).
+// Three waves per SIMD: left to itself the compiler takes 256 VGPRs and more
+// (one wave per SIMD), too few waves to hide the traversal's memory latency.
 // kMode: traversal specialization (trace_mode_of: one instance, instance
 // level, or a scene with quads or spheres).
-template <int kMode, int kLeaf>
-__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_pt_iterate(PtScene S) {
+// kNeeOne: at most one next-event estimate a vertex (several are traced one
+// after the other, before the walk).
+template <int kMode, int kLeaf, bool kNeeOne>
+__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_pt_iterate(PtScene S,
+                                                                                                  PtWork W) {
     __shared__ int sStack[kLdsDepth * kPtThreads];
-    const int px = blockIdx.x * kPtTile + (threadIdx.x % kPtTile);
-    const int py = blockIdx.y * kPtTile + (threadIdx.x / kPtTile);
-    if (px >= S.width || py >= S.height) return;
-    const size_t pixel = (size_t)px + (size_t)py * S.width;
     int* const lstack = sStack + threadIdx.x;
-    u64 rng = S.rngs[pixel];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *W.nextQueue = 0;
+    auto any_hit = [&](const NeeCandidate& c) {
+        return trace_mode<kMode, true, kPtThreads, kLdsDepth, kLeaf>(S.trace, c.a, c.dir, c.tmax, lstack).inst != -1;
+    };
+    const int lane = (int)threadIdx.x;
+    const int first = (int)gridDim.x * W.lanes;  // slots below are assigned by block index
+    bool start = true, more = first < W.slots;   // more: the queue may hold further slots
+    bool busy = false;                           // the lane owns a pixel
+    int px = 0, py = 0, done = 0;                // its position, its finished iterations
+    int pathLen = 0;
+    u64 rng = 0;
     Acc acc;
     acc.init(S.targetMask);
-    float guideWeight = 1.0f;
     float footA = 0.0f;  // FootprintV0::m_a (footprint.hpp:137-170)
-    V3 throughput = v3(1.0f, 1.0f, 1.0f);
-    Vertex vx;
-    pcg_next(rng);  // create_camera's RndSet2, unused by the pinhole
-    int pathLen = 0;
-    do {
-        if (pathLen > 0 && pathLen + 1 >= S.minPathLength && pathLen + 1 <= S.maxPathLength) {
-            const u64 neeSeed = pcg_next(rng);
-            for (int i = 0; i < S.neeCount; ++i) {
-                const u64 x = pcg_next(rng);
+    float pdfF = 1.0f;
+    V3 throughput = v3(1.0f, 1.0f, 1.0f), rayOrigin = throughput, dir = throughput, absorption = throughput;
+    V3 prevPos = throughput;
+    while (true) {
+        const unsigned long long idle = __ballot(!busy && lane < W.lanes);
+        if (idle != 0ull) {
+            int slot = -1;
+            if (start) {
+                if (lane < W.lanes) slot = (int)blockIdx.x * W.lanes + lane;
+            } else if (more && 4 * __popcll(idle) >= W.lanes) {
+                const int want = __popcll(idle), leader = __ffsll((long long)idle) - 1;
+                int base = 0;
+                if (lane == leader) base = atomicAdd(W.queue, want);
+                base = __shfl(base, leader) + first;
+                more = base + want < W.slots;
+                if (!busy && lane < W.lanes)
+                    slot = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(idle >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)idle, 0u));
+            }
+            start = false;
+            if (slot >= 0 && slot < W.slots) {
+                const int tile = slot / kPtThreads, in = slot % kPtThreads;
+                px = (tile % W.tilesX) * kPtTile + in % kPtTile;
+                py = (tile / W.tilesX) * kPtTile + in / kPtTile;
+                if (px < S.width && py < S.height) {
+                    busy = true;
+                    done = 0;
+                    pathLen = 0;
+                    rng = S.rngs[(size_t)px + (size_t)py * S.width];
+                }
+            }
+            if (__ballot(busy) == 0ull) {
+                if (!more) break;
+                continue;  // every lane took a slot outside the image
+            }
+        }
+        if (busy) {
+            if (pathLen == 0) {  // the camera's sample
+                acc.init(S.targetMask);
+                footA = 0.0f;
+                throughput = v3(1.0f, 1.0f, 1.0f);
+                pcg_next(rng);  // create_camera's RndSet2, unused by the pinhole
+                const u64 x0 = pcg_next(rng);
+                pcg_next(rng);
+                pcg_next(rng);  // the roulette always continues at throughput 1
+                camera_ray(S, px, py, x0, dir, pdfF);
+                rayOrigin = v3(S.camPos[0], S.camPos[1], S.camPos[2]);
+                absorption = v3(0.0f, 0.0f, 0.0f);
+                prevPos = rayOrigin;
+            }
+            const TraceHit hit =
+                trace_mode<kMode, false, kPtThreads, kLdsDepth, kLeaf>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
+            throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
+            footA += 1.0f / fsqrt(pdfF);
+            const float guideWeight = 1.f / (1.f + footA * footA / 1.0f);
+            Vertex vx;
+            make_vertex(S, rayOrigin, dir, pdfF, hit.t, hit.inst, hit.prim, hit.w0, hit.w1, vx);
+            ++pathLen;
+            vertex_targets(S, vx, pathLen, throughput, guideWeight, acc, prevPos);
+            bool ended = vx.isVoid || pathLen >= S.maxPathLength;
+            if (!ended) {
                 NeeCandidate c;
-                if (nee_candidate(S, vx, throughput, guideWeight, i, neeSeed, x, c)) {
-                    const TraceHit sh =
-                        trace_mode<kMode, true, kPtThreads, kLdsDepth, kLeaf>(S.trace, c.a, c.dir, c.tmax, lstack);
-                    if (sh.inst == -1) add_nee(c, acc);
+                bool shadow = false;
+                if (pathLen + 1 >= S.minPathLength) {
+                    const u64 neeSeed = pcg_next(rng);
+                    if constexpr (kNeeOne) {
+                        if (S.neeCount > 0)
+                            shadow = nee_candidate(S, vx, throughput, guideWeight, 0, neeSeed, pcg_next(rng), c);
+                    } else {
+                        for (int i = 0; i < S.neeCount; ++i)
+                            if (nee_candidate(S, vx, throughput, guideWeight, i, neeSeed, pcg_next(rng), c) &&
+                                !any_hit(c))
+                                add_nee(c, acc);
+                    }
+                }
+                const u64 x0 = pcg_next(rng);
+                const u64 x1 = pcg_next(rng);
+                const float rndRoulette = sample_uniform((u32)pcg_next(rng));
+                ended = !walk_surface(vx, x0, x1, rndRoulette, throughput, rayOrigin, dir, pdfF, absorption);
+                prevPos = vx.position;
+                if (shadow && !any_hit(c)) add_nee(c, acc);
+            }
+            if (ended) {
+                const size_t pixel = (size_t)px + (size_t)py * S.width;
+                accumulate(S, pixel, S.iteration + done, acc.v, acc.mask);
+                if (acc.nans) atomicAdd(S.nanCounter, acc.nans);
+                pathLen = 0;
+                if (++done == W.iterations) {
+                    S.rngs[pixel] = rng;
+                    busy = false;
                 }
             }
         }
-        const u64 x0 = pcg_next(rng);
-        const u64 x1 = pcg_next(rng);
-        const float rndRoulette = sample_uniform((u32)pcg_next(rng));
-        V3 rayOrigin, dir, absorption;
-        float pdfF;
-        if (pathLen == 0) {
-            camera_ray(S, px, py, x0, dir, pdfF);
-            rayOrigin = v3(S.camPos[0], S.camPos[1], S.camPos[2]);
-            absorption = v3(0.0f, 0.0f, 0.0f);
-        } else if (!walk_surface(vx, x0, x1, rndRoulette, throughput, rayOrigin, dir, pdfF, absorption)) {
-            break;
-        }
-        const TraceHit hit =
-            trace_mode<kMode, false, kPtThreads, kLdsDepth, kLeaf>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
-        throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
-        footA += 1.0f / fsqrt(pdfF);
-        guideWeight = 1.f / (1.f + footA * footA / 1.0f);
-        const V3 prevPos = pathLen == 0 ? rayOrigin : vx.position;
-        make_vertex(S, rayOrigin, dir, pdfF, hit.t, hit.inst, hit.prim, hit.w0, hit.w1, vx);
-        ++pathLen;
-        vertex_targets(S, vx, pathLen, throughput, guideWeight, acc, prevPos);
-        if (vx.isVoid) break;
-    } while (pathLen < S.maxPathLength);
-
-    S.rngs[pixel] = rng;
-    accumulate(S, pixel, S.iteration, acc.v, acc.mask);
-    if (acc.nans) atomicAdd(S.nanCounter, acc.nans);
+    }
 }
 
 // rngs[i] = PCG64(u32(i + seed)) (gpu_pt.cu:140-144, rng.hpp:76-81)
@@ -113,19 +192,45 @@ void launch_pt_init_rng(u64* rngs, int num, int seed, hipStream_t stream) {
     MFH_HIP(hipGetLastError());
 }
 
-void launch_pt_iterate(const PtScene& S, int leafBatch, hipStream_t stream) {
-    const dim3 grid((S.width + kPtTile - 1) / kPtTile, (S.height + kPtTile - 1) / kPtTile);
+namespace {
+
+using IterateFn = void (*)(PtScene, PtWork);
+
+template <int kMode>
+IterateFn iterate_kernel(bool leaf8, bool neeOne) {
+    if (neeOne) return leaf8 ? k_pt_iterate<kMode, 8, true> : k_pt_iterate<kMode, 1, true>;
+    return leaf8 ? k_pt_iterate<kMode, 8, false> : k_pt_iterate<kMode, 1, false>;
+}
+
+}  // namespace
+
+void launch_pt_iterate(const PtScene& S, int iterations, int leafBatch, PtQueue& queue, int numCUs,
+                       hipStream_t stream) {
     const int mode = trace_mode_of(S.trace);
-#define MFH_ITERATE(M, L) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pt_iterate<M, L>), grid, dim3(kPtThreads), 0, stream, S)
-    if (mode == kTraceSingle) {
-        if (leafBatch == 8) MFH_ITERATE(kTraceSingle, 8); else MFH_ITERATE(kTraceSingle, 1);
-    } else if (mode == kTraceMulti) {
-        if (leafBatch == 8) MFH_ITERATE(kTraceMulti, 8); else MFH_ITERATE(kTraceMulti, 1);
-    } else {
-        if (leafBatch == 8) MFH_ITERATE(kTraceMixed, 8); else MFH_ITERATE(kTraceMixed, 1);
-    }
-#undef MFH_ITERATE
+    const bool leaf8 = leafBatch == 8, neeOne = S.neeCount <= 1;
+    const IterateFn fn = mode == kTraceSingle  ? iterate_kernel<kTraceSingle>(leaf8, neeOne)
+                         : mode == kTraceMulti ? iterate_kernel<kTraceMulti>(leaf8, neeOne)
+                                               : iterate_kernel<kTraceMixed>(leaf8, neeOne);
+    int blocksPerCU = 0;
+    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocksPerCU, fn, kPtThreads, 0));
+    PtWork W;
+    W.tilesX = (S.width + kPtTile - 1) / kPtTile;
+    const int tiles = W.tilesX * ((S.height + kPtTile - 1) / kPtTile);
+    W.slots = tiles * kPtThreads;
+    W.iterations = iterations;
+    W.queue = queue.counters + queue.next;
+    W.nextQueue = queue.counters + (queue.next ^ 1);
+    // Lanes of a wave that take pixels: all 64, or for images too small to
+    // give every wave slot of the chip 64 pixels, half as many until they do.
+    // More waves of fewer pixels each hide one another's memory latency, and
+    // the segment of a wave waits for the longest of fewer rays.
+    const int resident = std::max(blocksPerCU, 1) * numCUs;
+    W.lanes = kPtThreads;
+    while (W.lanes > kPtMinLanes && W.slots / W.lanes < resident) W.lanes /= 2;
+    const int grid = std::min(W.slots / W.lanes, resident);
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(kPtThreads), 0, stream, S, W);
     MFH_HIP(hipGetLastError());
+    queue.next ^= 1;
 }
 
 }  // namespace mfh

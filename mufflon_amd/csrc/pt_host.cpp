@@ -21,7 +21,8 @@ struct PathTracer {
     BackgroundHost background;
     std::vector<HostPointLight> pointLights;
     DevBuf dMaterials, dPtLods, dLightMem, dMapKeys, dMapCodes, dTextures, dSat;
-    DevBuf dRngs, dNan;
+    DevBuf dRngs, dNan, dQueue;
+    PtQueue queue;  // over dQueue
     DevBuf dTargets[kNumTargets];
     DevBuf dVariance[kNumTargets];
     uint32_t targetMask = (1u << MFH_TARGET_RADIANCE) | (1u << MFH_TARGET_HIT_ID);
@@ -84,6 +85,9 @@ void release_wavefront(PathTracer& t) {
     t.wfMaxLen = t.wfNee = -1;
 }
 
+// Paths of one megakernel launch, at most (a fraction of a second on a large scene).
+constexpr int64_t kMaxLaunchPaths = 1 << 26;
+
 // Trace-stage forms the autotuners try: chunked queue walks with two chunk
 // sizes, and lane refill every 16 or 32 traversal steps.
 constexpr int kTraceModes = 4;
@@ -131,7 +135,7 @@ void destroy_tracers(Context& c) {
     for (PathTracer* t : c.tracers) {
         if (!t) continue;
         for (DevBuf* b : {&t->dMaterials, &t->dPtLods, &t->dLightMem, &t->dMapKeys, &t->dMapCodes, &t->dTextures,
-                          &t->dSat, &t->dRngs, &t->dNan})
+                          &t->dSat, &t->dRngs, &t->dNan, &t->dQueue})
             b->release();
         for (DevBuf& b : t->dTargets) b.release();
         for (DevBuf& b : t->dVariance) b.release();
@@ -598,11 +602,14 @@ int mfh_pt_create(mfh_context* ctx, int32_t sceneId, const mfh_material* materia
             const size_t num = (size_t)camera->width * camera->height;
             t->dRngs.reserve(8 * num);
             t->dNan.reserve(4);
+            t->dQueue.reserve(8);
+            MFH_HIP(hipMemsetAsync(t->dQueue.ptr, 0, 8, c.stream));
+            t->queue.counters = t->dQueue.as<int>();
             reset(c, *t);
             MFH_HIP(hipStreamSynchronize(c.stream));
         } catch (...) {
             for (DevBuf* b : {&t->dMaterials, &t->dPtLods, &t->dLightMem, &t->dMapKeys, &t->dMapCodes, &t->dTextures,
-                              &t->dSat, &t->dRngs, &t->dNan})
+                              &t->dSat, &t->dRngs, &t->dNan, &t->dQueue})
                 b->release();
             for (DevBuf& b : t->dTargets) b.release();
             for (DevBuf& b : t->dVariance) b.release();
@@ -661,9 +668,15 @@ int mfh_pt_iterate(mfh_context* ctx, int32_t ptId, int32_t iterations) {
             run_wavefront(c, t, S, iterations);
             return;
         }
-        for (int32_t k = 0; k < iterations; ++k) {
-            S.iteration = ++t.iteration;
-            launch_pt_iterate(S, kWfTraceShapes[t.tune.traceVariant].leafBatch, c.stream);
+        // all iterations in one launch, split only to bound its length (a pixel's iterations are a chain)
+        const int perLaunch = (int)std::max<int64_t>(1, kMaxLaunchPaths / ((int64_t)S.width * S.height));
+        const int cus = iterations > 0 ? num_cus(c) : 1;
+        for (int32_t k = 0; k < iterations;) {
+            const int n = std::min(iterations - k, perLaunch);
+            S.iteration = t.iteration + 1;
+            launch_pt_iterate(S, n, kWfTraceShapes[t.tune.traceVariant].leafBatch, t.queue, cus, c.stream);
+            t.iteration += n;
+            k += n;
         }
     });
 }
