@@ -375,10 +375,9 @@ typedef struct mfh_wavefront_tuning {
     int32_t stackDepth;
     int32_t queueChunk;
     int32_t sortBounces;
-    int32_t refillBudget; /* 0: chunked queue walk; n > 0: lanes whose ray ended take the next ray
-                             every n traversal steps once a quarter of the wave is idle */
-    int32_t leafBatch;    /* 1 or 8: triangles of a BVH leaf loaded ahead of their tests (long
-                             leaves); also used by the megakernel form; the refill kernels use 1 */
+    int32_t refillBudget; /* 0 .. 4096 and */
+    int32_t leafBatch;    /* 1 or 8: accepted and returned by mfh_pt_get_tuning; the traversal has one
+                             form, which loads a leaf's next primitive while it tests one */
     int32_t tailAfter;    /* 0: one launch per stage and bounce; k > 0: after the extension rays of
                              bounce k one launch finishes every remaining path (megakernel-style,
                              same bits), so the last bounces of a few long paths do not cost three
@@ -387,8 +386,7 @@ typedef struct mfh_wavefront_tuning {
 int mfh_pt_set_tuning(mfh_context* ctx, int32_t ptId, const mfh_wavefront_tuning* tuning);
 int mfh_pt_get_tuning(mfh_context* ctx, int32_t ptId, mfh_wavefront_tuning* outTuning);
 /* Times `iterations` wavefront iterations for every tuning candidate (block x
- * stack depth x leaf batch 1/8 x {chunk 256, chunk 1024, refill 16, refill 32}
- * x sorted bounces 0/1/2), then the tail bounce (never, 1, 2, 3, 4, 6) on the
+ * stack depth x chunk 256/1024 x sorted bounces 0/1/2), then the tail bounce (never, 1, 2, 3, 4, 6) on the
  * fastest of those, keeps the fastest and resets the path tracer. */
 int mfh_pt_autotune(mfh_context* ctx, int32_t ptId, int32_t iterations, mfh_wavefront_tuning* outBest,
                     float* outMsPerIteration);

@@ -45,15 +45,12 @@ void refresh_scene(Context& c, Scene& s) {
     for (size_t i = 0; !stale && i < c.lods.size(); ++i)
         stale = c.lods[i] && c.lods[i]->generation != s.lodGeneration[i];
     if (!stale) return;
-    std::vector<DevLod> lods(c.lods.size()), ref(c.lods.size());
+    std::vector<DevLod> lods(c.lods.size());
     s.lodGeneration.assign(c.lods.size(), 0);
     for (size_t i = 0; i < c.lods.size(); ++i) {
         std::memset(&lods[i], 0, sizeof(DevLod));
         const Lod* l = c.lods[i];
-        if (!l || !l->built) {
-            ref[i] = lods[i];
-            continue;
-        }
+        if (!l || !l->built) continue;
         s.lodGeneration[i] = l->generation;
         lods[i].triVerts = l->triVerts.as<float4>();
         lods[i].nodes = l->nodes.ptr;
@@ -62,11 +59,8 @@ void refresh_scene(Context& c, Scene& s) {
         lods[i].quadV3 = l->numQuads > 0 ? l->quadV3.as<float4>() : nullptr;
         std::memcpy(lods[i].box, l->box, sizeof(l->box));
         lods[i].coordMax = l->coordMax;
-        ref[i] = lods[i];
-        if (l->travNumInternal >= 0) {
-            lods[i].nodes = l->travNodes.ptr;
-            lods[i].numInternal = l->travNumInternal;
-        }
+        lods[i].wide = l->numPrims() > 1 ? l->wideNodes.as<float4>() : nullptr;
+        lods[i].leafBoxes = l->leafBoxes.as<float4>();
     }
     s.mixed = false;
     for (int32_t li : s.instLod) {
@@ -74,7 +68,6 @@ void refresh_scene(Context& c, Scene& s) {
         if (c.lods[li]->mixed()) s.mixed = true;
     }
     upload(c, s.dLods, lods.data(), sizeof(DevLod) * lods.size());
-    upload(c, s.dLodsRef, ref.data(), sizeof(DevLod) * ref.size());
     build_scene_bvh(c, s, nullptr);
     MFH_HIP(hipStreamSynchronize(c.stream));
 }
@@ -100,7 +93,13 @@ int mfh_create(int32_t deviceIndex, mfh_context** outCtx) {
             MFH_HIP(hipEventCreate(&ctx->c.evBegin));
             MFH_HIP(hipEventCreate(&ctx->c.evEnd));
             noalloc_scratch_init(deviceIndex);
+            MFH_HIP(hipDeviceGetAttribute(&ctx->c.numCUs, hipDeviceAttributeMultiprocessorCount, deviceIndex));
+            ctx->c.numCUs = std::max(ctx->c.numCUs, 1);
+            ctx->c.queueCounters.reserve(8);
+            MFH_HIP(hipMemsetAsync(ctx->c.queueCounters.ptr, 0, 8, ctx->c.stream));
+            ctx->c.traceQueue.counters = ctx->c.queueCounters.as<int>();
         } catch (...) {
+            ctx->c.queueCounters.release();
             delete ctx;
             throw;
         }
@@ -118,13 +117,13 @@ int mfh_destroy(mfh_context* ctx) {
             if (!l) continue;
             l->verts.release(); l->tris.release(); l->nodes.release(); l->primIds.release(); l->triVerts.release();
             l->quads.release(); l->spheres.release(); l->quadV3.release();
-            l->travNodes.release();
+            l->wideNodes.release(); l->leafBoxes.release();
             l->normals.release(); l->uvs.release(); l->matIdx.release();
             delete l;
         }
         for (Scene* s : c.scenes) {
             if (!s) continue;
-            s->dInstLod.release(); s->dWorldToInst.release(); s->dLods.release(); s->dLodsRef.release();
+            s->dInstLod.release(); s->dWorldToInst.release(); s->dLods.release();
             s->tlasNodes.release(); s->tlasPrimIds.release();
             delete s;
         }
@@ -139,6 +138,7 @@ int mfh_destroy(mfh_context* ctx) {
                           &b.boxes, &b.counters, &b.flags, &b.offsets, &b.offsets2, &b.hist, &b.partials,
                           &b.misc, &b.stage})
             d->release();
+        c.queueCounters.release();
         if (c.evBegin) (void)hipEventDestroy(c.evBegin);
         if (c.evEnd) (void)hipEventDestroy(c.evEnd);
         if (c.stream) (void)hipStreamDestroy(c.stream);
@@ -362,7 +362,7 @@ int mfh_scene_create(mfh_context* ctx, const int32_t* instLod, const float* worl
             refresh_scene(c, *s);
             MFH_HIP(hipStreamSynchronize(c.stream));
         } catch (...) {
-            s->dInstLod.release(); s->dWorldToInst.release(); s->dLods.release(); s->dLodsRef.release();
+            s->dInstLod.release(); s->dWorldToInst.release(); s->dLods.release();
             s->tlasNodes.release(); s->tlasPrimIds.release();
             delete s;
             throw;
@@ -397,7 +397,7 @@ int mfh_trace_closest(mfh_context* ctx, int32_t sceneId, const float* dRays, int
         MFH_REQUIRE(dRays && dHits, "null pointer");
         refresh_scene(c, s);
         launch_trace_closest(trace_params(s), dRays, numRays, static_cast<float4*>(dHits),
-                             reinterpret_cast<float2*>(dBary), nullptr, c.stream);
+                             reinterpret_cast<float2*>(dBary), c.traceQueue, c.numCUs, c.stream);
     });
 }
 
@@ -410,8 +410,8 @@ int mfh_trace_closest_stats(mfh_context* ctx, int32_t sceneId, const float* dRay
         if (numRays == 0) return;
         MFH_REQUIRE(dRays && dHits && dStats, "null pointer");
         refresh_scene(c, s);
-        launch_trace_closest(trace_params(s, true), dRays, numRays, static_cast<float4*>(dHits),
-                             reinterpret_cast<float2*>(dBary), reinterpret_cast<uint2*>(dStats), c.stream);
+        launch_trace_counts(trace_params(s), dRays, numRays, static_cast<float4*>(dHits),
+                            reinterpret_cast<float2*>(dBary), reinterpret_cast<uint2*>(dStats), c.stream);
     });
 }
 
@@ -423,7 +423,7 @@ int mfh_trace_any(mfh_context* ctx, int32_t sceneId, const float* dRays, int32_t
         if (numRays == 0) return;
         MFH_REQUIRE(dRays && dOccluded, "null pointer");
         refresh_scene(c, s);
-        launch_trace_any(trace_params(s), dRays, numRays, dOccluded, c.stream);
+        launch_trace_any(trace_params(s), dRays, numRays, dOccluded, c.traceQueue, c.numCUs, c.stream);
     });
 }
 

@@ -15,6 +15,7 @@
 //   k_mark      collapse decision per internal node      (build_lbvh.cu:417-463)
 //   scan        inclusive sum of the keep marks          (build_lbvh.cu:748-758)
 //   k_collapse  64-byte-node BVH with enlarged boxes     (build_lbvh.cu:503-566)
+//   k_wide      4-wide quantized nodes for the traversal kernels (LoDs)
 //
 // Determinism. The refit merges a node in a fixed operand order whatever
 // thread arrives second: box = min/max(right, left) and
@@ -732,12 +733,11 @@ __global__ __launch_bounds__(kLevelThreads) void k_refit_level(int n, int level,
 // traversal hierarchy: a node is also kept there when it holds more than
 // refineAbove primitives, so no traversal leaf is longer than that. Both mark
 // sets are closed under descendants (a removed node's subtree is removed).
-// *differ is set when the two sets differ.
 template <class C>
 __global__ __launch_bounds__(kThreads) void k_mark(int nInt, const i32* __restrict__ parents,
                                                   const uint8_t* __restrict__ flags, i32* __restrict__ marks,
                                                   const float4* __restrict__ boxes, int refineAbove,
-                                                  i32* __restrict__ marks2, u32* __restrict__ differ) {
+                                                  i32* __restrict__ marks2) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= nInt) return;
     int keep = 1;
@@ -752,25 +752,30 @@ __global__ __launch_bounds__(kThreads) void k_mark(int nInt, const i32* __restri
         y = parent_of(parents, y);
     }
     marks[x] = keep;
-    if (marks2) {
-        const int keep2 = (keep || C::sum(__float_as_int(boxes[2 * (size_t)x].w)) > refineAbove) ? 1 : 0;
-        marks2[x] = keep2;
-        if (keep2 != keep) *differ = 1u;
-    }
+    if (marks2) marks2[x] = (keep || C::sum(__float_as_int(boxes[2 * (size_t)x].w)) > refineAbove) ? 1 : 0;
 }
 
 __device__ __forceinline__ bool is_collapsed(const i32* offsets, int nInt, int node) {
     return node > 0 && node < nInt && (offsets[node] - offsets[node - 1]) == 0;
 }
 
-// The collapsed BVH's record of node `node` (its box enlarged, its index in
-// the collapsed numbering) under the keep scan `offsets`.
+// The box of a node as the BVHs hold it: enlarged by 1.0001 about its centre.
+__device__ __forceinline__ void enlarged_box(float4 a, float4 b, V3& bl, V3& bh) {
+    const V3 lo = v3(a.x, a.y, a.z), hi = v3(b.x, b.y, b.z);
+    const V3 c = (lo + hi) * 0.5f;
+    bl = (lo - c) * 1.0001f + c;
+    bh = (hi - c) * 1.0001f + c;
+}
+
+// The reference's collapsed BVH: each kept node and leaf writes its record
+// (enlarged box, index in the collapsed numbering) into its parent.
 template <class C>
-__device__ __forceinline__ void collapse_node(int node, int n, const i32* __restrict__ parents,
-                                              const float4* __restrict__ boxes, const i32* __restrict__ offsets,
-                                              BvhChild* __restrict__ out) {
+__global__ __launch_bounds__(kThreads) void k_collapse(int n, const i32* __restrict__ parents,
+                                                      const float4* __restrict__ boxes,
+                                                      const i32* __restrict__ offsets, BvhChild* __restrict__ out) {
+    const int node = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int nInt = n - 1;
-    if (is_collapsed(offsets, nInt, node)) return;
+    if (node >= 2 * n - 1 || is_collapsed(offsets, nInt, node)) return;
     const int nAfter = offsets[nInt - 1];
     int parent = parents[node];
     int off = parent < 0 ? 0 : 1;
@@ -789,10 +794,8 @@ __device__ __forceinline__ void collapse_node(int node, int n, const i32* __rest
     const i32 primCount = C::sum(__float_as_int(a.w));
     const int outIdx = (offsets[parent] - 1) * 2;
     const int outNode = (node >= nInt) ? node - nInt + nAfter : offsets[node] - 1;
-    const V3 lo = v3(a.x, a.y, a.z), hi = v3(b.x, b.y, b.z);
-    const V3 c = (lo + hi) * 0.5f;
-    const V3 bl = (lo - c) * 1.0001f + c;
-    const V3 bh = (hi - c) * 1.0001f + c;
+    V3 bl, bh;
+    enlarged_box(a, b, bl, bh);
     BvhChild r;
     r.lo[0] = bl.x; r.lo[1] = bl.y; r.lo[2] = bl.z;
     r.hi[0] = bh.x; r.hi[1] = bh.y; r.hi[2] = bh.z;
@@ -801,18 +804,134 @@ __device__ __forceinline__ void collapse_node(int node, int n, const i32* __rest
     out[outIdx + off] = r;
 }
 
-// The reference's collapsed BVH and, with offsets2, the traversal hierarchy
-// (written only when *differ is set) in one pass over the nodes.
+// ---- traversal hierarchy
+// One 64-byte node per kept binary node: up to four descendants of it (the
+// larger-surface inner child is opened twice), their boxes quantized to 8 bits
+// on a grid of the node's own.  {org.xyz, scale.x}, {scale.yz, lo.xy},
+// {lo.z, hi.xyz}, {child 0..3}: lo / hi hold the four children's byte
+// coordinates of one axis each, a child is another node's number or
+// kWideLeaf | position of a leaf's first primitive. A child never found (an
+// unused slot) has lo = 255, hi = 0 on every axis and child 0's reference, so
+// that a slab test that loses the inversion to rounding only revisits child 0.
+// The quantized boxes contain the enlarged boxes; a leaf's own box is kept in
+// full precision, so what a ray tests does not depend on the grid.
+struct WideChild {
+    V3 lo, hi;       // enlarged box
+    float area;      // surface of an inner child, -1 for a leaf (not opened)
+    int node;        // binary node of an inner child
+    u32 ref;
+};
+
+// Child c of binary node `parent`'s side (left or right) under the keep scan.
 template <class C>
-__global__ __launch_bounds__(kThreads) void k_collapse(int n, const i32* __restrict__ parents,
-                                                      const float4* __restrict__ boxes,
-                                                      const i32* __restrict__ offsets, BvhChild* __restrict__ out,
-                                                      const i32* __restrict__ offsets2, BvhChild* __restrict__ out2,
-                                                      const u32* __restrict__ differ) {
-    const int node = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (node >= 2 * n - 1) return;
-    collapse_node<C>(node, n, parents, boxes, offsets, out);
-    if (offsets2 && *differ != 0u) collapse_node<C>(node, n, parents, boxes, offsets2, out2);
+__device__ __forceinline__ WideChild wide_child(int c, bool left, int nInt, const float4* __restrict__ boxes,
+                                                const i32* __restrict__ offsets, i32& count) {
+    const float4 a = boxes[2 * (size_t)c], b = boxes[2 * (size_t)c + 1];
+    WideChild w;
+    enlarged_box(a, b, w.lo, w.hi);
+    w.node = c;
+    count = C::sum(__float_as_int(a.w));
+    if (c < nInt && !is_collapsed(offsets, nInt, c)) {
+        w.area = surface(w.lo, w.hi);
+        w.ref = (u32)(offsets[c] - 1);
+    } else {
+        // a removed left child's index is the last of its leaves, a right child's the first
+        const int first = c >= nInt ? c - nInt : (left ? c - count + 1 : c);
+        w.area = -1.0f;
+        w.ref = kWideLeaf | (u32)first;
+    }
+    return w;
+}
+
+template <class C>
+__global__ __launch_bounds__(kThreads) void k_wide(int n, const i32* __restrict__ children,
+                                                  const float4* __restrict__ boxes,
+                                                  const i32* __restrict__ offsets, float4* __restrict__ wide,
+                                                  float4* __restrict__ leafBoxes) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    const int nInt = n - 1;
+    if (x >= nInt || is_collapsed(offsets, nInt, x)) return;
+    WideChild ch[4];
+    int used = 2;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        i32 count;
+        ch[k] = wide_child<C>(children[2 * x + k], k == 0, nInt, boxes, offsets, count);
+        if (ch[k].area < 0.0f) {  // the leaf's own record, from its binary parent
+            const size_t at = 2 * (size_t)(ch[k].ref & ~kWideLeaf);
+            leafBoxes[at] = make_float4(ch[k].lo.x, ch[k].lo.y, ch[k].lo.z, ch[k].hi.x);
+            leafBoxes[at + 1] = make_float4(ch[k].hi.y, ch[k].hi.z, __int_as_float(count), 0.0f);
+        }
+    }
+#pragma unroll
+    for (int open = 2; open < 4; ++open) {  // open the inner child with the largest surface
+        int best = -1;
+        float area = -1.0f;
+#pragma unroll
+        for (int k = 0; k < open; ++k)
+            if (k < used && ch[k].area > area) {
+                area = ch[k].area;
+                best = k;
+            }
+        if (best < 0) break;
+        int node = ch[0].node;
+#pragma unroll
+        for (int k = 1; k < open; ++k)
+            if (k == best) node = ch[k].node;
+        i32 count;
+        const WideChild l = wide_child<C>(children[2 * node], true, nInt, boxes, offsets, count);
+        const WideChild r = wide_child<C>(children[2 * node + 1], false, nInt, boxes, offsets, count);
+#pragma unroll
+        for (int k = 0; k < open; ++k)
+            if (k == best) ch[k] = l;
+        ch[open] = r;
+        used = open + 1;
+    }
+    float org[3], scale[3];
+    u32 qlo[3], qhi[3];
+#pragma unroll
+    for (int axis = 0; axis < 3; ++axis) {
+        float lo[4], hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int c = k < used ? k : 0;
+            const V3 bl = ch[c].lo, bh = ch[c].hi;
+            lo[k] = axis == 0 ? bl.x : (axis == 1 ? bl.y : bl.z);
+            hi[k] = axis == 0 ? bh.x : (axis == 1 ? bh.y : bh.z);
+        }
+        float mnv = lo[0], mxv = hi[0];
+#pragma unroll
+        for (int k = 1; k < 4; ++k) {
+            mnv = __builtin_fminf(mnv, lo[k]);
+            mxv = __builtin_fmaxf(mxv, hi[k]);
+        }
+        // slack for the rounding of the grid coordinates (a few ulps of the
+        // largest coordinate), also where the node is flat
+        const float slack = __builtin_fmaxf(fabsf(mnv), fabsf(mxv)) * 0x1p-21f + 1e-36f;
+        org[axis] = mnv - 2.0f * slack;
+        scale[axis] = __builtin_fmaxf((mxv + 2.0f * slack - org[axis]) / 254.0f, 1e-38f);
+        u32 l = 0, h = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            u32 ql = 255u, qh = 0u;
+            if (k < used) {
+                ql = (u32)clampf(floorf((lo[k] - slack - org[axis]) / scale[axis]), 0.0f, 255.0f);
+                qh = (u32)clampf(ceilf((hi[k] + slack - org[axis]) / scale[axis]), 0.0f, 255.0f);
+            }
+            l |= ql << (8 * k);
+            h |= qh << (8 * k);
+        }
+        qlo[axis] = l;
+        qhi[axis] = h;
+    }
+    float4* o = wide + 4 * (size_t)(offsets[x] - 1);
+    o[0] = make_float4(org[0], org[1], org[2], scale[0]);
+    o[1] = make_float4(scale[1], scale[2], __uint_as_float(qlo[0]), __uint_as_float(qlo[1]));
+    o[2] = make_float4(__uint_as_float(qlo[2]), __uint_as_float(qhi[0]), __uint_as_float(qhi[1]),
+                       __uint_as_float(qhi[2]));
+    o[3] = make_float4(__uint_as_float(ch[0].ref), __uint_as_float(ch[1].ref),
+                       __uint_as_float(used > 2 ? ch[2].ref : ch[0].ref),
+                       __uint_as_float(used > 3 ? ch[3].ref : ch[0].ref));
 }
 
 // Zero fill and count hand-off of the build (kernels, not memsets, so that a
@@ -824,16 +943,6 @@ __global__ void k_fill_u32(u32* p, int n, u32 v) {
 __global__ void k_num_internal(const i32* offsets, int n, i32* out) {
     if (threadIdx.x == 0) *out = n > 1 ? offsets[n - 2] : 0;
 }
-// Internal node counts of the reference BVH and of the traversal hierarchy,
-// and whether the two differ, for one copy to the host.
-__global__ void k_build_counts(const i32* offsets, const i32* offsets2, const u32* differ, int n, i32* out) {
-    if (threadIdx.x == 0) {
-        out[0] = offsets[n - 2];
-        out[1] = offsets2 ? offsets2[n - 2] : 0;
-        out[2] = differ ? (i32)*differ : 0;
-    }
-}
-
 // World box of each instance (feeds the scene box of the instance level).
 __global__ __launch_bounds__(kThreads) void k_inst_boxes(InstPrims set, int n, float* out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -868,16 +977,16 @@ void fill_u32(void* p, int n, u32 v, hipStream_t st) {
     MFH_HIP(hipGetLastError());
 }
 
-// The traversal hierarchy of a build: the reference's collapsed BVH with
-// every collapsed subtree of more than refineAbove primitives kept split
-// (leaves of at most refineAbove primitives), over the same sorted primitive
-// records. Closest and any hit do not depend on the hierarchy they are found
-// through (the closest hit is the lowest (t, instance, primitive)), so the
-// traversal kernels use it while the exported BVH stays the reference's.
-struct Refinement {
-    int refineAbove = 0;  // 0: none
-    DevBuf* nodes = nullptr;
-    int numInternal = -1;  // -1: equal to the reference (no subtree was split)
+// The traversal hierarchy of a build (k_wide): over the reference's collapsed
+// BVH with every collapsed subtree of more than refineAbove primitives kept
+// split (0: none), and the same sorted primitive records. Closest and any hit
+// do not depend on the hierarchy they are found through (the closest hit is
+// the lowest (t, instance, primitive)), so the traversal kernels use it while
+// the exported BVH stays the reference's.
+struct WideOut {
+    int refineAbove;
+    DevBuf* nodes;
+    DevBuf* leafBoxes;
 };
 
 // Shared orchestration (build_lbvh.cu:586-780). Returns the number of
@@ -887,7 +996,7 @@ struct Refinement {
 template <class P, class C>
 int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const float* bbox, DevBuf& nodes,
                   DevBuf& primIds, float4* triVerts, StageSink* sink, i32* dNumInternal = nullptr,
-                  Refinement* refine = nullptr, float4* stage = nullptr) {
+                  const WideOut* wideOut = nullptr, float4* stage = nullptr) {
     hipStream_t st = ctx.stream;
     MFH_REQUIRE(n < kMaxPrims, "an LBVH build holds fewer than 2^29 primitives");
     s.keysA.reserve(8 * (size_t)n);
@@ -952,45 +1061,37 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
         return 0;
     }
     i32* offsets = s.offsets.as<i32>();
-    const bool refining = refine && refine->refineAbove > 0 && !dNumInternal;
+    const bool refining = wideOut && wideOut->refineAbove > 0;
     i32* offsets2 = nullptr;
-    u32* differ = nullptr;
     if (refining) {
-        s.offsets2.reserve(4 * (size_t)(n - 1) + 4);
+        s.offsets2.reserve(4 * (size_t)(n - 1));
         offsets2 = s.offsets2.as<i32>();
-        differ = reinterpret_cast<u32*>(offsets2 + (n - 1));
-        fill_u32(differ, 1, 0u, st);
     }
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mark<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n - 1, parents,
-                       s.flags.as<uint8_t>(), offsets, boxes, refining ? refine->refineAbove : 0, offsets2, differ);
-    // the reference's BVH and the traversal hierarchy (collapsed whether or
-    // not it differs, so that the build waits for the device once; its
-    // records are written only when it differs)
+                       s.flags.as<uint8_t>(), offsets, boxes, refining ? wideOut->refineAbove : 0, offsets2);
     if (refining)
         scan_inclusive_i32_pair(offsets, offsets2, n - 1, s, st);
     else
         scan_inclusive_i32(offsets, offsets, n - 1, s, st);
     nodes.reserve(64 * (size_t)(n - 1));
-    if (refining) refine->nodes->reserve(64 * (size_t)(n - 1));
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_collapse<C>), dim3(blocks_for(2 * n - 2)), dim3(kThreads), 0, st, n,
-                       parents, boxes, offsets, nodes.as<BvhChild>(), offsets2,
-                       refining ? refine->nodes->as<BvhChild>() : nullptr, differ);
+                       parents, boxes, offsets, nodes.as<BvhChild>());
+    if (wideOut) {
+        wideOut->nodes->reserve(64 * (size_t)(n - 1));
+        wideOut->leafBoxes->reserve(32 * (size_t)n);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wide<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n, children,
+                           boxes, refining ? offsets2 : offsets, wideOut->nodes->as<float4>(),
+                           wideOut->leafBoxes->as<float4>());
+    }
     MFH_HIP(hipGetLastError());
     if (dNumInternal) {
         hipLaunchKernelGGL(k_num_internal, dim3(1), dim3(64), 0, st, offsets, n, dNumInternal);
         MFH_HIP(hipGetLastError());
         return -1;
     }
-    s.misc.reserve(16);
-    i32* dCounts = s.misc.as<i32>();
-    hipLaunchKernelGGL(k_build_counts, dim3(1), dim3(64), 0, st, offsets, refining ? offsets2 : nullptr, differ, n,
-                       dCounts);
-    MFH_HIP(hipGetLastError());
-    i32 counts[3] = {0, 0, 0};
-    MFH_HIP(hipMemcpyAsync(counts, dCounts, sizeof(counts), hipMemcpyDeviceToHost, st));
+    i32 nAfter = 0;
+    MFH_HIP(hipMemcpyAsync(&nAfter, offsets + (n - 2), sizeof(nAfter), hipMemcpyDeviceToHost, st));
     MFH_HIP(hipStreamSynchronize(st));
-    const i32 nAfter = counts[0];
-    if (refining) refine->numInternal = counts[2] ? counts[1] : -1;
     if (sink) {
         d2h(st, sink->parents, parents, 2 * (size_t)n - 1);
         d2h(st, sink->boxes, boxes, 8 * (size_t)(2 * n - 1));
@@ -1006,24 +1107,21 @@ void build_lod_bvh(Context& ctx, Lod& lod, const float* bbox, StageSink* sink) {
     MFH_REQUIRE(n >= 1, "LoD has no primitives");
     if (bbox) std::memcpy(lod.box, bbox, sizeof(lod.box));
     lod.triVerts.reserve(48 * (size_t)n);
-    Refinement refine;
-    refine.refineAbove = ctx.traversalLeafLimit;
-    refine.nodes = &lod.travNodes;
+    const WideOut wide{ctx.traversalLeafLimit, &lod.wideNodes, &lod.leafBoxes};
     if (lod.mixed()) {
         if (lod.numQuads > 0) lod.quadV3.reserve(16 * (size_t)n);
         MixedPrims set{lod.verts.as<float>(), lod.tris.as<u32>(),  lod.quads.as<u32>(), lod.spheres.as<float4>(),
                        lod.numQuads > 0 ? lod.quadV3.as<float4>() : nullptr, lod.numTris, lod.numQuads};
         lod.numInternal = build_generic<MixedPrims, LodCost>(ctx, ctx.scratch, set, n, lod.box, lod.nodes,
                                                              lod.primIds, lod.triVerts.as<float4>(), sink, nullptr,
-                                                             &refine);
+                                                             &wide);
     } else {
         TriPrims set{lod.verts.as<float>(), lod.tris.as<u32>()};
         ctx.scratch.stage.reserve(48 * (size_t)n);
         lod.numInternal = build_generic<TriPrims, LodCost>(ctx, ctx.scratch, set, n, lod.box, lod.nodes,
                                                            lod.primIds, lod.triVerts.as<float4>(), sink, nullptr,
-                                                           &refine, ctx.scratch.stage.as<float4>());
+                                                           &wide, ctx.scratch.stage.as<float4>());
     }
-    lod.travNumInternal = refine.numInternal;
     lod.built = true;
 }
 

@@ -75,7 +75,8 @@ __device__ LtEmitter light_position(const PtScene& S, uint16_t type, u32 offset,
         const float cosTheta = u0 * 2.0f - 1.0f;
         const float sinTheta = fsqrt((1.0f - cosTheta) * (1.0f + cosTheta));
         const float phi = u1 * 2.0f * kPi;
-        const V3 n = v3(sinTheta * fsin(phi), sinTheta * fcos(phi), cosTheta);
+        const SinCos sc = fsincos(phi);
+        const V3 n = v3(sinTheta * sc.s, sinTheta * sc.c, cosTheta);
         // the emitter's uv is (u1, acos(n.z)), the polar angle unnormalized
         // (light_sampling.hpp:181)
         const MatParams m = fetch(S, matIdx, u1, facos(n.z));
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(kLtThreads) void k_lt_iterate(PtScene S, float* __r
                     const V3 d = b - a;
                     const float tmax = len(d);
                     const TraceHit sh =
-                        trace_mode<kMode, true, kLtThreads, kLdsDepth, 1>(S.trace, a, d / tmax, tmax, lstack);
+                        trace_mode<kMode, true, kLtThreads, kLdsDepth>(S.trace, a, d / tmax, tmax, lstack);
                     if (sh.inst == -1) {
                         bxdfProd = bxdfProd / distSq;
                         const V3 rad = throughput * cosProd * bxdfProd;
@@ -258,7 +259,8 @@ __global__ __launch_bounds__(kLtThreads) void k_lt_iterate(PtScene S, float* __r
                 const float cosT = fsqrt(u0);
                 const float sinT = fsqrt(1.0f - u0);
                 const float phi = u1 * 2 * kPi;
-                const float lx = sinT * fsin(phi), ly = sinT * fcos(phi);
+                const SinCos sc = fsincos(phi);
+                const float lx = sinT * sc.s, ly = sinT * sc.c;
                 const V3 tx = normalize(perpendicular(light.normal));
                 const V3 ty = cross(light.normal, tx);
                 dirOut = smul(lx, tx) + smul(ly, ty) + smul(cosT, light.normal);
@@ -268,7 +270,8 @@ __global__ __launch_bounds__(kLtThreads) void k_lt_iterate(PtScene S, float* __r
                 const float cosT = u0 * 2.0f - 1.0f;
                 const float sinT = fsqrt((1.0f - cosT) * (1.0f + cosT));
                 const float phi = u1 * 2.0f * kPi;
-                dirOut = v3(sinT * fsin(phi), sinT * fcos(phi), cosT);
+                const SinCos sc = fsincos(phi);
+                dirOut = v3(sinT * sc.s, sinT * sc.c, cosT);
                 sThroughput = light.intensity * 4 * kPi;
                 geoOut = v3(0, 0, 0);
             }
@@ -288,7 +291,7 @@ __global__ __launch_bounds__(kLtThreads) void k_lt_iterate(PtScene S, float* __r
         if (rndRoulette >= cont) break;
         throughput = throughput / cont;
         rayOrigin = add_epsilon(rayOrigin, dirOut, geoOut);
-        const TraceHit hit = trace_mode<kMode, false, kLtThreads, kLdsDepth, 1>(S.trace, rayOrigin, dirOut,
+        const TraceHit hit = trace_mode<kMode, false, kLtThreads, kLdsDepth>(S.trace, rayOrigin, dirOut,
                                                                                  kMaxSceneSize, lstack);
         throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
         if (hit.inst == -1) break;

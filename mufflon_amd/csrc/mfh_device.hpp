@@ -119,13 +119,20 @@ __device__ __forceinline__ bool ray_triangle(const FastRay& r, V3 v0, V3 v1, V3 
     const V3 e2 = v2 - v0;
     const V3 p = cross(r.d, e2);
     const float det = dot(e1, p);
+    const V3 s = r.o - v0;
+    const V3 q = cross(s, e1);
+    const float us = dot(s, p), vs = dot(r.d, q);
+    // Most tests miss: reject with the hardware's approximate reciprocal what
+    // the correctly rounded quotients below reject too (they agree to a few
+    // ulps wherever that reciprocal is not flushed).
+    const float approx = __builtin_amdgcn_rcpf(det);
+    const float ua = us * approx, va = vs * approx;
+    if (fabsf(det) > 1e-30f && (ua < -1e-20f || va < -1e-20f || ua + va > 1.00001f)) return false;
     if (det == 0.0f) return false;
     const float invDet = 1.0f / det;
-    const V3 s = r.o - v0;
-    const float u = dot(s, p) * invDet;
+    const float u = us * invDet;
     if (u < 0.0f || u > 1.0f) return false;
-    const V3 q = cross(s, e1);
-    const float v = dot(r.d, q) * invDet;
+    const float v = vs * invDet;
     if (v < 0.0f || u + v > 1.0f) return false;
     t = dot(e2, q) * invDet;
     w0 = 1.0f - u - v;
@@ -290,5 +297,7 @@ struct __attribute__((packed)) BvhChild {
     i32 primCount;
 };
 static_assert(sizeof(BvhChild) == 32, "BvhChild must be 32 bytes");
+// Leaf flag of a wide node's child reference (the rest: a sorted position).
+constexpr u32 kWideLeaf = 0x80000000u;
 
 }  // namespace mfh

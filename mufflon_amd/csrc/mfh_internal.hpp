@@ -88,7 +88,7 @@ struct BuildScratch {
     DevBuf counters;                  // n-1 arrival counters (refit levels past their LDS capacity)
     DevBuf flags;                     // n-1 bytes: bit0 count capped, bit1 leaf cheaper than split
     DevBuf offsets;                   // n-1 inclusive scan of the keep marks
-    DevBuf offsets2;                  // n-1 (+1 flag) the same for the traversal hierarchy
+    DevBuf offsets2;                  // n-1 the same for the traversal hierarchy
     DevBuf hist;                      // radix digit counts
     DevBuf partials;                  // scan partial sums
     DevBuf misc;                      // small values (scene box, counts)
@@ -139,10 +139,11 @@ struct Lod {
     // {radius, 0, 0, 2}, {0}. The kind is the int bits of the second .w.
     DevBuf triVerts;
     DevBuf quadV3;            // float4 per sorted position (LoDs with quads only)
-    // traversal hierarchy: the collapsed BVH with its long leaves kept split
-    // (travNumInternal = -1: none was, traversal uses nodes)
-    DevBuf travNodes;
-    int32_t travNumInternal = -1;
+    // traversal hierarchy (WideNode): 4-wide nodes over the collapsed BVH with
+    // its long leaves kept split, and at the sorted position of each of its
+    // leaves' first primitive that leaf's box and primitive count (32 bytes)
+    DevBuf wideNodes;
+    DevBuf leafBoxes;
     int32_t numPrims() const { return numTris + numQuads + numSpheres; }
     bool mixed() const { return numQuads > 0 || numSpheres > 0; }
 };
@@ -153,7 +154,6 @@ struct Scene {
     std::vector<int32_t> instLod;
     std::vector<float> worldToInst;
     DevBuf dInstLod, dWorldToInst, dLods;
-    DevBuf dLodsRef;  // the LoD table over the reference BVHs (visit counts of the reference order)
     float box[6] = {0, 0, 0, 0, 0, 0};
     int32_t tlasNumInternal = 0;
     DevBuf tlasNodes, tlasPrimIds;
@@ -171,8 +171,19 @@ struct Texture {
     DevBuf dev;
 };
 
+// Work queue of persistent kernels: two device counters that start at 0. A
+// launch takes work through one and clears the other for the launch after it
+// (all launches of a queue go to one stream).
+struct LaunchQueue {
+    int* counters = nullptr;
+    int next = 0;
+};
+
 struct Context {
     int device = 0;
+    int numCUs = 1;
+    DevBuf queueCounters;
+    LaunchQueue traceQueue;  // over queueCounters
     hipStream_t stream = nullptr;
     hipEvent_t evBegin = nullptr, evEnd = nullptr;
     std::vector<Lod*> lods;
@@ -190,7 +201,9 @@ struct Context {
 // Device view of one LoD, as the traversal kernels read it.
 struct DevLod {
     const float4* triVerts;
-    const void* nodes;
+    const void* nodes;       // the reference's collapsed BVH
+    const float4* wide;      // WideNode, four float4 each (null for one primitive)
+    const float4* leafBoxes; // two float4 per sorted position
     const float4* quadV3;  // fourth quad vertices per sorted position (null without quads)
     int32_t numInternal;
     int32_t numPrims;
@@ -202,7 +215,8 @@ struct DevLod {
 void destroy_tracers(Context& ctx);
 void upload(Context& c, DevBuf& b, const void* src, size_t bytes);
 
-// LBVH over a triangle LoD; fills lod.nodes / primIds / triVerts / numInternal.
+// LBVH over a triangle LoD; fills lod.nodes / primIds / triVerts / numInternal
+// and the traversal hierarchy (wideNodes / leafBoxes).
 void build_lod_bvh(Context& ctx, Lod& lod, const float* bbox, StageSink* sink);
 // LBVH over the instances of a scene (instance-level hierarchy).
 void build_scene_bvh(Context& ctx, Scene& sc, StageSink* sink);
@@ -243,12 +257,13 @@ struct TraceParams {
     float tlasCoordMax;  // largest |coordinate| of the scene box (bounds the instance-level node boxes)
     int32_t mixed;       // an instance's LoD holds quads or spheres (kernels with kMixed)
 };
-// Traversal over the LoDs' traversal hierarchies, or (reference = true) over
-// the reference BVHs, whose visit counts follow the reference's order.
-TraceParams trace_params(const Scene& sc, bool reference = false);
-void launch_trace_closest(const TraceParams& p, const float* rays, int n, float4* hits, float2* bary, uint2* stats,
-                          hipStream_t stream);
-void launch_trace_any(const TraceParams& p, const float* rays, int n, int32_t* occluded, hipStream_t stream);
+TraceParams trace_params(const Scene& sc);
+void launch_trace_closest(const TraceParams& p, const float* rays, int n, float4* hits, float2* bary,
+                          LaunchQueue& queue, int numCUs, hipStream_t stream);
+void launch_trace_counts(const TraceParams& p, const float* rays, int n, float4* hits, float2* bary, uint2* stats,
+                         hipStream_t stream);
+void launch_trace_any(const TraceParams& p, const float* rays, int n, int32_t* occluded, LaunchQueue& queue,
+                      int numCUs, hipStream_t stream);
 // Re-upload the LoD table of a scene (and rebuild its instance level) when a
 // LoD was rebuilt after the scene was created.
 void refresh_scene(Context& ctx, Scene& sc);

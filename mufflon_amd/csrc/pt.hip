@@ -51,21 +51,20 @@ constexpr int kPtMinLanes = 8;
 // numbers of both are drawn before, in the order of pt_sample): through that
 // traversal the vertex, about 45 registers, is no longer live.
 //
-// kLeaf: triangles of a BVH leaf loaded ahead of their tests (1 or 8).
 // Three waves per SIMD: left to itself the compiler takes 256 VGPRs and more
 // (one wave per SIMD), too few waves to hide the traversal's memory latency.
 // kMode: traversal specialization (trace_mode_of: one instance, instance
 // level, or a scene with quads or spheres).
 // kNeeOne: at most one next-event estimate a vertex (several are traced one
 // after the other, before the walk).
-template <int kMode, int kLeaf, bool kNeeOne>
+template <int kMode, bool kNeeOne>
 __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_pt_iterate(PtScene S,
                                                                                                   PtWork W) {
     __shared__ int sStack[kLdsDepth * kPtThreads];
     int* const lstack = sStack + threadIdx.x;
     if (blockIdx.x == 0 && threadIdx.x == 0) *W.nextQueue = 0;
     auto any_hit = [&](const NeeCandidate& c) {
-        return trace_mode<kMode, true, kPtThreads, kLdsDepth, kLeaf>(S.trace, c.a, c.dir, c.tmax, lstack).inst != -1;
+        return trace_mode<kMode, true, kPtThreads, kLdsDepth>(S.trace, c.a, c.dir, c.tmax, lstack).inst != -1;
     };
     const int lane = (int)threadIdx.x;
     const int first = (int)gridDim.x * W.lanes;  // slots below are assigned by block index
@@ -128,7 +127,7 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(3)))
                 prevPos = rayOrigin;
             }
             const TraceHit hit =
-                trace_mode<kMode, false, kPtThreads, kLdsDepth, kLeaf>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
+                trace_mode<kMode, false, kPtThreads, kLdsDepth>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
             throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
             footA += 1.0f / fsqrt(pdfF);
             const float guideWeight = 1.f / (1.f + footA * footA / 1.0f);
@@ -197,20 +196,18 @@ namespace {
 using IterateFn = void (*)(PtScene, PtWork);
 
 template <int kMode>
-IterateFn iterate_kernel(bool leaf8, bool neeOne) {
-    if (neeOne) return leaf8 ? k_pt_iterate<kMode, 8, true> : k_pt_iterate<kMode, 1, true>;
-    return leaf8 ? k_pt_iterate<kMode, 8, false> : k_pt_iterate<kMode, 1, false>;
+IterateFn iterate_kernel(bool neeOne) {
+    return neeOne ? k_pt_iterate<kMode, true> : k_pt_iterate<kMode, false>;
 }
 
 }  // namespace
 
-void launch_pt_iterate(const PtScene& S, int iterations, int leafBatch, PtQueue& queue, int numCUs,
-                       hipStream_t stream) {
+void launch_pt_iterate(const PtScene& S, int iterations, LaunchQueue& queue, int numCUs, hipStream_t stream) {
     const int mode = trace_mode_of(S.trace);
-    const bool leaf8 = leafBatch == 8, neeOne = S.neeCount <= 1;
-    const IterateFn fn = mode == kTraceSingle  ? iterate_kernel<kTraceSingle>(leaf8, neeOne)
-                         : mode == kTraceMulti ? iterate_kernel<kTraceMulti>(leaf8, neeOne)
-                                               : iterate_kernel<kTraceMixed>(leaf8, neeOne);
+    const bool neeOne = S.neeCount <= 1;
+    const IterateFn fn = mode == kTraceSingle  ? iterate_kernel<kTraceSingle>(neeOne)
+                         : mode == kTraceMulti ? iterate_kernel<kTraceMulti>(neeOne)
+                                               : iterate_kernel<kTraceMixed>(neeOne);
     int blocksPerCU = 0;
     MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocksPerCU, fn, kPtThreads, 0));
     PtWork W;

@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_pt_adjoint(PtScene S, AdjointSt
                     const u64 x = pcg_next(rng);
                     NeeCandidate c;
                     if (nee_candidate(S, vx, throughput, guideWeight, i, neeSeed, x, c)) {
-                        const TraceHit sh = trace_mode<kMode, true, kAdjThreads, kLdsDepth, kPtLeafBatch, false>(
+                        const TraceHit sh = trace_mode<kMode, true, kAdjThreads, kLdsDepth>(
                             S.trace, c.a, c.dir, c.tmax, lstack);
                         if (sh.inst == -1) {
                             AdjVertex& r = rec[pathLen];
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_pt_adjoint(PtScene S, AdjointSt
                 r.tp = r.astar == 0 ? tPrime.x : (r.astar == 1 ? tPrime.y : tPrime.z);
                 if (!ok) break;
             }
-            const TraceHit hit = trace_mode<kMode, false, kAdjThreads, kLdsDepth, kPtLeafBatch, false>(
+            const TraceHit hit = trace_mode<kMode, false, kAdjThreads, kLdsDepth>(
                 S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
             throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
             footA += 1.0f / fsqrt(pdfF);

@@ -124,13 +124,6 @@ struct PtScene {
 };
 
 void launch_pt_init_rng(uint64_t* rngs, int num, int seed, hipStream_t stream);
-// Pixel queue of the megakernel: two device counters that start at 0. A launch
-// takes pixels through one and clears the other for the launch after it (on
-// the same stream).
-struct PtQueue {
-    int* counters = nullptr;
-    int next = 0;
-};
 // Work of one launch: `iterations` iterations of the pixels in 8x8 tile order
 // (`slots` = tiles * 64, `tilesX` tiles a row), taken by the first `lanes`
 // lanes of each wave. Blocks start on the slots of their index, later slots
@@ -141,8 +134,7 @@ struct PtWork {
     int* nextQueue;
 };
 // `iterations` iterations from index S.iteration on.
-void launch_pt_iterate(const PtScene& S, int iterations, int leafBatch, PtQueue& queue, int numCUs,
-                       hipStream_t stream);
+void launch_pt_iterate(const PtScene& S, int iterations, LaunchQueue& queue, int numCUs, hipStream_t stream);
 // One iteration of the wireframe renderer into S.cum[MFH_TARGET_RADIANCE]
 // (and S.var[...] when recorded), S.iteration the iteration index.
 void launch_wireframe(const PtScene& S, const uint32_t* seeds, float lineWidth, int maxTraceDepth,

@@ -22,7 +22,7 @@ struct PathTracer {
     std::vector<HostPointLight> pointLights;
     DevBuf dMaterials, dPtLods, dLightMem, dMapKeys, dMapCodes, dTextures, dSat;
     DevBuf dRngs, dNan, dQueue;
-    PtQueue queue;  // over dQueue
+    LaunchQueue queue;  // over dQueue
     DevBuf dTargets[kNumTargets];
     DevBuf dVariance[kNumTargets];
     uint32_t targetMask = (1u << MFH_TARGET_RADIANCE) | (1u << MFH_TARGET_HIT_ID);
@@ -88,11 +88,9 @@ void release_wavefront(PathTracer& t) {
 // Paths of one megakernel launch, at most (a fraction of a second on a large scene).
 constexpr int64_t kMaxLaunchPaths = 1 << 26;
 
-// Trace-stage forms the autotuners try: chunked queue walks with two chunk
-// sizes, and lane refill every 16 or 32 traversal steps.
-constexpr int kTraceModes = 4;
-constexpr int kTraceModeChunk[kTraceModes] = {256, 1024, 256, 256};
-constexpr int kTraceModeRefill[kTraceModes] = {0, 0, 16, 32};
+// Queue chunks the autotuners try.
+constexpr int kTraceModes = 2;
+constexpr int kTraceModeChunk[kTraceModes] = {256, 1024};
 
 // A batch of path tracers iterated together by the wavefront stages.
 struct PtBatch {
@@ -391,12 +389,6 @@ void reset(Context& c, PathTracer& t) {
     t.iteration = -1;
 }
 
-int num_cus(const Context& c) {
-    int n = 0;
-    MFH_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, c.device));
-    return std::max(n, 1);
-}
-
 // Buffers of the wavefront form for the current resolution, path length and
 // NEE count; the counter block holds queue lengths, shadow counts, work
 // counters and the device iteration counter.
@@ -471,18 +463,18 @@ WfState wavefront_state(Context& c, PathTracer& t) {
     t.wfSortScratch.hist.reserve(radix_sort_hist_bytes(N, 0, 32));
     t.wfSortScratch.partials.reserve(radix_sort_partials_bytes(N));
     if (t.tune.traceGrid <= 0 || t.tune.shadeGrid <= 0) {
-        const int cus = num_cus(c);
+        const int cus = c.numCUs;
         t.tune.traceGrid = 0;
         t.tune.shadeGrid = wf_shade_grid(cus);
     }
-    if (t.tune.tailGrid <= 0) t.tune.tailGrid = wf_tail_grid(num_cus(c));
+    if (t.tune.tailGrid <= 0) t.tune.tailGrid = wf_tail_grid(c.numCUs);
     return W;
 }
 
 // Runs `iterations` wavefront iterations, replaying a captured graph when enabled.
 void run_wavefront(Context& c, PathTracer& t, PtScene& S, int32_t iterations) {
     WfState W = wavefront_state(c, t);
-    if (t.tune.traceGrid <= 0) t.tune.traceGrid = wf_grid(S, t.tune, num_cus(c));
+    if (t.tune.traceGrid <= 0) t.tune.traceGrid = wf_grid(S, t.tune, c.numCUs);
     // the device iteration counter continues from the host's
     const int32_t it = t.iteration;
     MFH_HIP(hipMemcpyAsync(W.iteration, &it, 4, hipMemcpyHostToDevice, c.stream));
@@ -670,11 +662,10 @@ int mfh_pt_iterate(mfh_context* ctx, int32_t ptId, int32_t iterations) {
         }
         // all iterations in one launch, split only to bound its length (a pixel's iterations are a chain)
         const int perLaunch = (int)std::max<int64_t>(1, kMaxLaunchPaths / ((int64_t)S.width * S.height));
-        const int cus = iterations > 0 ? num_cus(c) : 1;
         for (int32_t k = 0; k < iterations;) {
             const int n = std::min(iterations - k, perLaunch);
             S.iteration = t.iteration + 1;
-            launch_pt_iterate(S, n, kWfTraceShapes[t.tune.traceVariant].leafBatch, t.queue, cus, c.stream);
+            launch_pt_iterate(S, n, t.queue, c.numCUs, c.stream);
             t.iteration += n;
             k += n;
         }
@@ -1011,9 +1002,9 @@ WfState batch_state(Context& c, PtBatch& b, std::vector<PtScene>& scenes) {
     W.scenes = b.dScenes.as<PtScene>();
     W.sceneOffset = b.dOffsets.as<int>();
     W.numScenes = (int)b.tracers.size();
-    if (b.tune.traceGrid <= 0) b.tune.traceGrid = wf_grid_batch(b.tune, num_cus(c));
-    if (b.tune.shadeGrid <= 0) b.tune.shadeGrid = wf_shade_grid(num_cus(c));
-    if (b.tune.tailGrid <= 0) b.tune.tailGrid = wf_tail_grid(num_cus(c));
+    if (b.tune.traceGrid <= 0) b.tune.traceGrid = wf_grid_batch(b.tune, c.numCUs);
+    if (b.tune.shadeGrid <= 0) b.tune.shadeGrid = wf_shade_grid(c.numCUs);
+    if (b.tune.tailGrid <= 0) b.tune.tailGrid = wf_tail_grid(c.numCUs);
     return W;
 }
 
@@ -1111,12 +1102,11 @@ int mfh_batch_iterate(mfh_context* ctx, int32_t batchId, int32_t iterations) {
 namespace mfh {
 namespace {
 
-// Trace variant of a tuning record (block, LDS stack depth, leaf batch); -1 if none matches.
+// Trace variant of a tuning record (block, LDS stack depth); -1 if none matches.
 int trace_variant_of(const mfh_wavefront_tuning& tuning) {
+    if (tuning.leafBatch != 1 && tuning.leafBatch != 8) return -1;
     for (int k = 0; k < kWfNumTraceVariants; ++k)
-        if (kWfTraceShapes[k].block == tuning.traceBlock && kWfTraceShapes[k].lds == tuning.stackDepth &&
-            kWfTraceShapes[k].leafBatch == tuning.leafBatch)
-            return k;
+        if (kWfTraceShapes[k].block == tuning.traceBlock && kWfTraceShapes[k].lds == tuning.stackDepth) return k;
     return -1;
 }
 
@@ -1126,7 +1116,7 @@ void tuning_record(const WfTuning& tune, mfh_wavefront_tuning* out) {
     out->queueChunk = tune.chunk;
     out->sortBounces = tune.sortBounces;
     out->refillBudget = tune.refill;
-    out->leafBatch = kWfTraceShapes[tune.traceVariant].leafBatch;
+    out->leafBatch = tune.leafBatch;
     out->tailAfter = tune.tailAfter;
 }
 
@@ -1151,6 +1141,7 @@ int mfh_batch_set_tuning(mfh_context* ctx, int32_t batchId, const mfh_wavefront_
         b.tune.traceVariant = v;
         b.tune.chunk = tuning->queueChunk;
         b.tune.refill = tuning->refillBudget;
+        b.tune.leafBatch = tuning->leafBatch;
         b.tune.tailAfter = tuning->tailAfter;
         b.tune.traceGrid = 0;
         drop_batch_graph(b);
@@ -1167,10 +1158,8 @@ int mfh_batch_autotune(mfh_context* ctx, int32_t batchId, int32_t iterations, mf
         WfTuning bestTune = b.tune;
         for (int v = 0; v < kWfNumTraceVariants; ++v) {
             for (int m = 0; m < kTraceModes; ++m) {
-                if (kTraceModeRefill[m] > 0 && kWfTraceShapes[v].leafBatch != 1) continue;  // same kernels as leaf 1
                 b.tune.traceVariant = v;
                 b.tune.chunk = kTraceModeChunk[m];
-                b.tune.refill = kTraceModeRefill[m];
                 b.tune.traceGrid = 0;
                 drop_batch_graph(b);
                 run_batch(c, b, 1);
@@ -1245,6 +1234,7 @@ int mfh_pt_set_tuning(mfh_context* ctx, int32_t ptId, const mfh_wavefront_tuning
         t.tune.chunk = tuning->queueChunk;
         t.tune.sortBounces = tuning->sortBounces;
         t.tune.refill = tuning->refillBudget;
+        t.tune.leafBatch = tuning->leafBatch;
         t.tune.tailAfter = tuning->tailAfter;
         t.tune.traceGrid = 0;
         drop_graph(t);
@@ -1275,10 +1265,8 @@ int mfh_pt_autotune(mfh_context* ctx, int32_t ptId, int32_t iterations, mfh_wave
         for (int v = 0; v < kWfNumTraceVariants; ++v) {
             for (int cs = 0; cs < 3 * kTraceModes; ++cs) {
                 const int m = cs % kTraceModes;
-                if (kTraceModeRefill[m] > 0 && kWfTraceShapes[v].leafBatch != 1) continue;  // same kernels as leaf 1
                 t.tune.traceVariant = v;
                 t.tune.chunk = kTraceModeChunk[m];
-                t.tune.refill = kTraceModeRefill[m];
                 t.tune.sortBounces = sorts[cs / kTraceModes];
                 t.tune.traceGrid = 0;
                 drop_graph(t);

@@ -27,13 +27,23 @@ __device__ __forceinline__ V3 neg(V3 v) { return {-v.x, -v.y, -v.z}; }
 __device__ __forceinline__ V3 smul(float s, V3 a) { return {s * a.x, s * a.y, s * a.z}; }
 __device__ __forceinline__ float sdiv(float x, float d) { return x / (d + 1e-20f * sgnf(d)); }
 __device__ __forceinline__ bool nonzero(V3 v) { return v.x != 0.0f || v.y != 0.0f || v.z != 0.0f; }
-__device__ __forceinline__ float fsin(float x) { return (float)sin((double)x); }
-__device__ __forceinline__ float fcos(float x) { return (float)cos((double)x); }
-__device__ __forceinline__ float facos(float x) { return (float)acos((double)x); }
-__device__ __forceinline__ float fatan2(float y, float x) { return (float)atan2((double)y, (double)x); }
-__device__ __forceinline__ float fexp(float x) { return (float)exp((double)x); }
-__device__ __forceinline__ float flog(float x) { return (float)log((double)x); }
-__device__ __forceinline__ float fpow(float x, float y) { return (float)pow((double)x, (double)y); }
+// The double evaluations are calls, one copy each: inlined at their about
+// twenty uses they made 55 of a path kernel's 128 KB of code, and their
+// temporaries most of its spilled registers.
+#define MFH_CALL __device__ __attribute__((noinline))
+struct SinCos {
+    float s, c;
+};
+MFH_CALL SinCos fsincos(float x) {
+    double s, c;
+    sincos((double)x, &s, &c);
+    return {(float)s, (float)c};
+}
+MFH_CALL float facos(float x) { return (float)acos((double)x); }
+MFH_CALL float fatan2(float y, float x) { return (float)atan2((double)y, (double)x); }
+MFH_CALL float fexp(float x) { return (float)exp((double)x); }
+MFH_CALL float flog(float x) { return (float)log((double)x); }
+MFH_CALL float fpow(float x, float y) { return (float)pow((double)x, (double)y); }
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_sqrtf(x); }
 __device__ __forceinline__ int ifloor(float x) { return (int)floorf(x); }
 __device__ __forceinline__ int imod(int a, int m) {
@@ -74,7 +84,7 @@ __device__ __forceinline__ u64 percentage_of(u64 num, float p) {
     return ((pfix * (num & 0x7fffffff)) >> 31) + (pfix * (num >> 31));
 }
 // sampling.hpp:72-85 (an empty interval maps to its left end)
-__device__ __forceinline__ u64 rescale_sample(u64 x, u64 pLeft, u64 pRight) {
+MFH_CALL u64 rescale_sample(u64 x, u64 pLeft, u64 pRight) {
     const u64 interval = pRight - pLeft;
     const u64 xrel = x - pLeft;
     if (interval == 0) return 0;
@@ -87,7 +97,7 @@ __device__ __forceinline__ float4 texel(const DevTexture& t, int x, int y) {
 }
 // CPU texture sampling (cputexture.cpp:372-411): nearest, linear without
 // half-texel offset, 1x1 textures return their texel.
-__device__ __forceinline__ float4 tex_sample(const DevTexture& t, float u, float v) {
+MFH_CALL float4 tex_sample(const DevTexture& t, float u, float v) {
     if (t.width == 1 && t.height == 1) return t.texels[0];
     if (t.sampling == 0) return texel(t, ifloor(u * (float)t.width), ifloor(v * (float)t.height));
     float fx = u * (float)t.width, fy = v * (float)t.height;
@@ -124,6 +134,7 @@ struct Medium {
 // Medium::get_transmission (medium.hpp:40-42)
 __device__ __forceinline__ V3 transmission(const Medium& m, float distance) {
     const V3 e = m.absorption * -distance;
+    if (e.x == 0.0f && e.y == 0.0f && e.z == 0.0f) return {1.0f, 1.0f, 1.0f};  // exp(+-0), most media
     return {fexp(e.x), fexp(e.y), fexp(e.z)};
 }
 
@@ -253,8 +264,9 @@ __device__ V3 sample_half(const MatParams& p, V3 in, float u0, float u1, u64& rn
         if (tanTheta < 0.0001f) {
             const float r = fsqrt(sdiv(u0, (1.f - u0)));
             const float phi = 6.28318530718f * u1;
-            sx = r * fcos(phi);
-            sy = r * fsin(phi);
+            const SinCos sc = fsincos(phi);
+            sx = r * sc.c;
+            sy = r * sc.s;
         } else {
             const float a1 = 1.0f / tanTheta;
             const float g1 = 2.f / (1.f + fsqrt(1.0f + 1.0f / (a1 * a1)));
@@ -285,8 +297,9 @@ __device__ V3 sample_half(const MatParams& p, V3 in, float u0, float u1, u64& rn
     if (p.ndf == kNdfGgx) {
         const float phi = 2.0f * kPi * u0;
         const float e = fsqrt(u1 / (1.0f - u1));
-        float slopeX = e * fcos(phi);
-        float slopeY = e * fsin(phi);
+        const SinCos sc = fsincos(phi);
+        float slopeX = e * sc.c;
+        float slopeY = e * sc.s;
         const float norm = kPi * p.rx * p.ry;
         const float tmp = 1.0f + slopeX * slopeX + slopeY * slopeY;
         slopeX *= p.rx;
@@ -297,8 +310,9 @@ __device__ V3 sample_half(const MatParams& p, V3 in, float u0, float u1, u64& rn
         const float phi = 2 * kPi * u0;
         const float xi = u1 + 1e-20f;
         const float e = fsqrt(-flog(xi));
-        const float slopeX = e * fcos(phi);
-        const float slopeY = e * fsin(phi);
+        const SinCos sc = fsincos(phi);
+        const float slopeX = e * sc.c;
+        const float slopeY = e * sc.s;
         cav = normalize(v3(-p.rx * slopeX, -p.ry * slopeY, 1.0f));
         cavityPdf = xi / mx(kPi * p.rx * p.ry * cav.z * cav.z * cav.z, 1e-20f);
     }
@@ -336,7 +350,8 @@ __device__ bool sample_ts(const MatParams& p, V3 in, float u0, float u1, u64 rnd
         const float sinT = fsqrt(1.0f - u0);
         const float phi = u1 * 2 * kPi;
         const float sg = sgnf(in.z);
-        ex = v3(sinT * fsin(phi) * sg, sinT * fcos(phi) * sg, cosT * sg);
+        const SinCos sc = fsincos(phi);
+        ex = v3(sinT * sc.s * sg, sinT * sc.c * sg, cosT * sg);
         throughput = p.albedo;
         pdfF = cosT / kPi;
         return true;
@@ -648,7 +663,8 @@ __device__ void background_sample_dir(const PtScene& S, float u0, float u1, V3& 
         const float cosTheta = u0 * 2.0f - 1.0f;
         const float sinTheta = fsqrt((1.0f - cosTheta) * (1.0f + cosTheta));
         const float phi = u1 * 2.0f * kPi;
-        dir = v3(sinTheta * fsin(phi), sinTheta * fcos(phi), cosTheta);
+        const SinCos sc = fsincos(phi);
+        dir = v3(sinTheta * sc.s, sinTheta * sc.c, cosTheta);
         pdf = 1.f / (4.f * kPi);
         radiance = v3(bg.color[0], bg.color[1], bg.color[2]) * v3(bg.scale[0], bg.scale[1], bg.scale[2]);
         return;
@@ -670,9 +686,10 @@ __device__ void background_sample_dir(const PtScene& S, float u0, float u1, V3& 
     const float texPdf = (vc1 - vc0) * (float)W * (float)H / highestRowwise;
     const float phi = columnVal * 2.f * kPi;
     const float theta = (1.f - rowVal) * kPi;
-    const float sinTheta = fsin(theta);
-    const float cosTheta = fcos(theta);
-    dir = v3(sinTheta * fcos(phi), cosTheta, sinTheta * fsin(phi));
+    const SinCos th = fsincos(theta), ph = fsincos(phi);
+    const float sinTheta = th.s;
+    const float cosTheta = th.c;
+    dir = v3(sinTheta * ph.c, cosTheta, sinTheta * ph.s);
     pdf = texPdf / (2.f * kPi * kPi * sinTheta);
     const float4 t = texel(env, column, row);
     radiance = v3(t.x, t.y, t.z) * v3(bg.scale[0], bg.scale[1], bg.scale[2]);
@@ -696,7 +713,7 @@ __device__ V3 evaluate_background(const PtScene& S, V3 direction, float& pdfBack
     const float cdf = bg.sat[(size_t)(H - 1) * W + (W - 1)] / (float)(H * W);
     float pdfScale = dot(v3(0.212671f, 0.715160f, 0.072169f), radiance);
     const int pixelY = ifloor(v * (float)H);
-    const float sinPixel = fsin(kPi * (float)((float)pixelY + 0.5f) / (float)H);
+    const float sinPixel = fsincos(kPi * (float)((float)pixelY + 0.5f) / (float)H).s;
     const float sinJac = fsqrt(1.0f - direction.y * direction.y);
     pdfScale *= sinPixel / (2.0f * kPi * kPi * sinJac);
     pdfBack = pdfScale / cdf;
@@ -796,7 +813,8 @@ __device__ Nee connect_sphere(const PtScene& S, const uint8_t* light, V3 pos, fl
     const float cosTheta = (1.f - u0) + u0 * cosSphere;
     const float sinTheta = fsqrt(1.f - cosTheta * cosTheta);
     const float phi = 2.f * u1 * kPi;
-    const float lx = fcos(phi) * sinTheta, ly = fsin(phi) * sinTheta;
+    const SinCos sc = fsincos(phi);
+    const float lx = sc.c * sinTheta, ly = sc.s * sinTheta;
     const float conePdf = 1.f / (2.f * kPi * (1.f - cosSphere));
     const V3 tangentX = normalize(perpendicular(centerDir));
     const V3 tangentY = cross(centerDir, tangentX);

@@ -147,9 +147,8 @@ __global__ void k_wf_begin(WfState W) {
 
 // Camera rays and their closest hits, one thread per pixel: 16x16 tiles for
 // one scene, one path per thread in path order for a batch (kMode 2).
-// kLeaf: triangles of a leaf loaded ahead of their tests (trace_ray's kBatch).
-template <int kMode, int kLeaf>
-__global__ __launch_bounds__(256) void k_wf_primary(PtScene S0, WfState W) {
+template <int kMode>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMode == 1 ? 5 : 4))) void k_wf_primary(PtScene S0, WfState W) {
     __shared__ int sStack[kLdsDepth * 256];
     constexpr bool kBatch = kMode == 2;
     int px, py, p, local, s = 0;
@@ -177,7 +176,7 @@ __global__ __launch_bounds__(256) void k_wf_primary(PtScene S0, WfState W) {
     camera_ray(S, px, py, x0, dir, pdfF);
     const V3 o = v3(S.camPos[0], S.camPos[1], S.camPos[2]);
     const TraceHit h =
-        trace_mode<kMode, false, 256, kLdsDepth, kLeaf>(S.trace, o, dir, kMaxSceneSize, sStack + threadIdx.x);
+        trace_mode<kMode, false, 256, kLdsDepth>(S.trace, o, dir, kMaxSceneSize, sStack + threadIdx.x);
     S.rngs[local] = rng;
     W.rayO[0][p] = float4{o.x, o.y, o.z, pdfF};
     W.rayD[0][p] = float4{dir.x, dir.y, dir.z, __int_as_float(p)};
@@ -191,46 +190,102 @@ __global__ __launch_bounds__(256) void k_wf_primary(PtScene S0, WfState W) {
 }
 
 // Closest hit of queue `buf` (length at counters[count]).
-template <int kMode, int kBlock, int kLds, int kLeaf>
-__global__ __launch_bounds__(kBlock) void k_wf_extend(PtScene S0, WfState W, int buf, int count, int work,
-                                                      const int* perm) {
+template <int kMode, int kBlock, int kLds>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMode == 1 ? 5 : 4))) void k_wf_extend(
+    PtScene S0, WfState W, int buf, int count, int work, const int* perm) {
     __shared__ int sStack[kLds * kBlock];
     constexpr bool kBatch = kMode == 2;
+    using T = ModeTrav<kMode, false, kBlock, kLds>;
     const int n = W.counters[count];
-    int* const lstack = sStack + threadIdx.x;
-    for (QueueWalk wk(n, W.chunk); wk.base < n; wk.next(W.counters + work)) {
-        const int end = min(wk.base + wk.chunk, n);
-        for (int qs = wk.base + lane_id(); qs < end; qs += 64) {
+    const int waves = (int)(gridDim.x * blockDim.x) / 64;
+    int s = 0;  // this lane's scene (batches)
+    const int lanes = queue_lanes(n, waves);
+    WaveQueue wq(n, lanes, queue_chunk(n, W.chunk), (int)(blockIdx.x * blockDim.x + threadIdx.x) / 64, waves,
+                 W.counters + work);
+    trace_queue<T>(
+        wq, sStack + threadIdx.x,
+        [&](int) -> const TraceParams& { return scene_ref<kBatch>(S0, W, s).trace; },
+        [&](int qs, V3& o, V3& d, float& tmax) {
             const int q = perm ? perm[qs] : qs;
-            const float4 o = W.rayO[buf][q];
-            const float4 d = W.rayD[buf][q];
+            const float4 ro = W.rayO[buf][q];
+            const float4 rd = W.rayD[buf][q];
             int local;
-            const int s = locate<kBatch>(W, __float_as_int(d.w), local);
-            const PtScene& S = scene_ref<kBatch>(S0, W, s);
-            const TraceHit h = trace_mode<kMode, false, kBlock, kLds, kLeaf>(S.trace, v3(o.x, o.y, o.z),
-                                                                             v3(d.x, d.y, d.z), kMaxSceneSize, lstack);
+            s = locate<kBatch>(W, __float_as_int(rd.w), local);
+            o = v3(ro.x, ro.y, ro.z);
+            d = v3(rd.x, rd.y, rd.z);
+            tmax = kMaxSceneSize;
+            return true;
+        },
+        [&](int qs, const TraceHit& h) {
+            const int q = perm ? perm[qs] : qs;
             W.hit[buf][q] = float4{h.t, __int_as_float(h.inst), __int_as_float(h.prim), h.w0};
             W.rayM[buf][q].w = h.w1;
-        }
-    }
+        });
 }
 
 // Any hit of the shadow candidates of one bounce; visible ones are added to
-// their path's accumulator in candidate order.
-template <int kMode, int kBlock, int kLds, int kLeaf>
-__global__ __launch_bounds__(kBlock) void k_wf_shadow(PtScene S0, WfState W, int count, int work, const int* perm) {
+// their path's accumulator in candidate order. An entry of the queue is one
+// candidate's ray when every slot holds at most one (neeStride 1); otherwise
+// the candidates of a slot are traced in turn.
+template <int kMode, int kBlock, int kLds>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMode == 1 ? 5 : 4))) void k_wf_shadow(
+    PtScene S0, WfState W, int count, int work, const int* perm) {
     __shared__ int sStack[kLds * kBlock];
     constexpr bool kBatch = kMode == 2;
+    using T = ModeTrav<kMode, true, kBlock, kLds>;
     const int n = W.counters[count];
+    const int waves = (int)(gridDim.x * blockDim.x) / 64;
     int* const lstack = sStack + threadIdx.x;
-    for (QueueWalk wk(n, W.chunk); wk.base < n; wk.next(W.counters + work)) {
-        const int end = min(wk.base + wk.chunk, n);
-        for (int ss = wk.base + lane_id(); ss < end; ss += 64) {
+    int si = 0;  // this lane's scene (batches)
+    auto add = [&](int path, int sl, u32 visible) {
+        const PtScene& S = scene_ref<kBatch>(S0, W, si);
+        Acc acc;
+        load_acc(W, S.targetMask, path, acc);
+        for (int i = 0; i < S.neeCount; ++i) {
+            if (!((visible >> i) & 1u)) continue;
+            const float4 c = W.shC[(size_t)sl * W.neeStride + i];
+            NeeCandidate nc;
+            nc.radiance = v3(c.x, c.y, c.z);
+            nc.lightness = c.w;
+            add_nee(nc, acc);
+        }
+        store_acc(W, S.targetMask, path, acc);
+        if (acc.nans) atomicAdd(S.nanCounter, acc.nans);
+    };
+    const int lanes = queue_lanes(n, waves);
+    WaveQueue wq(n, lanes, queue_chunk(n, W.chunk), (int)(blockIdx.x * blockDim.x + threadIdx.x) / 64, waves,
+                 W.counters + work);
+    if (W.neeStride == 1) {
+        trace_queue<T>(
+            wq, lstack, [&](int) -> const TraceParams& { return scene_ref<kBatch>(S0, W, si).trace; },
+            [&](int ss, V3& o, V3& d, float& tmax) {
+                const int sl = perm ? perm[ss] : ss;
+                const int2 pm = W.shPath[sl];
+                if (!(pm.y & 1)) return false;
+                int local;
+                si = locate<kBatch>(W, pm.x, local);
+                const float4 ro = W.shO[sl];
+                const float4 rd = W.shD[sl];
+                o = v3(ro.x, ro.y, ro.z);
+                d = v3(rd.x, rd.y, rd.z);
+                tmax = ro.w;
+                return true;
+            },
+            [&](int ss, const TraceHit& h) {
+                if (h.inst != -1) return;
+                const int sl = perm ? perm[ss] : ss;
+                add(W.shPath[sl].x, sl, 1u);
+            });
+        return;
+    }
+    while (wq.left()) {
+        const int ss = wq.take(wq.takers(true));
+        if (ss >= 0) {
             const int sl = perm ? perm[ss] : ss;
             const int2 pm = W.shPath[sl];
             const u32 cand = (u32)pm.y;
             int local;
-            const int si = locate<kBatch>(W, pm.x, local);
+            si = locate<kBatch>(W, pm.x, local);
             const PtScene& S = scene_ref<kBatch>(S0, W, si);
             u32 visible = 0;
             for (int i = 0; i < S.neeCount; ++i) {
@@ -238,154 +293,11 @@ __global__ __launch_bounds__(kBlock) void k_wf_shadow(PtScene S0, WfState W, int
                 const size_t e = (size_t)sl * W.neeStride + i;
                 const float4 a = W.shO[e];
                 const float4 d = W.shD[e];
-                const TraceHit h = trace_mode<kMode, true, kBlock, kLds, kLeaf>(S.trace, v3(a.x, a.y, a.z),
-                                                                                v3(d.x, d.y, d.z), a.w, lstack);
+                const TraceHit h =
+                    trace_mode<kMode, true, kBlock, kLds>(S.trace, v3(a.x, a.y, a.z), v3(d.x, d.y, d.z), a.w, lstack);
                 if (h.inst == -1) visible |= 1u << i;
             }
-            if (visible) {  // add the unoccluded estimates in candidate order
-                Acc acc;
-                load_acc(W, S.targetMask, pm.x, acc);
-                for (int i = 0; i < S.neeCount; ++i) {
-                    if (!((visible >> i) & 1u)) continue;
-                    const float4 c = W.shC[(size_t)sl * W.neeStride + i];
-                    NeeCandidate nc;
-                    nc.radiance = v3(c.x, c.y, c.z);
-                    nc.lightness = c.w;
-                    add_nee(nc, acc);
-                }
-                store_acc(W, S.targetMask, pm.x, acc);
-                if (acc.nans) atomicAdd(S.nanCounter, acc.nans);
-            }
-        }
-    }
-}
-
-// ---- trace stages with lane refill
-// The persistent trace kernels above give each lane whole rays from the
-// wave's chunk; a lane whose ray ends early idles until the wave's longest
-// traversal in the chunk is done. The refill forms below traverse in rounds
-// of `budget` steps (Traversal::run) and, between rounds, hand new rays to
-// idle lanes as soon as a quarter of the wave is idle: one atomic on the
-// queue's work counter per refill, lanes ranked with mbcnt. The queue is
-// consumed in order of the grabs, and a ray's result does not depend on the
-// rounds it took.
-constexpr int kRefillMinIdle = 16;
-
-__device__ __forceinline__ int lane_rank(unsigned long long mask) {
-    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-}
-
-// Refill of the idle lanes (mask `idle`, wave-uniform): first queue index of
-// this lane or -1; drained is set once the queue has been handed out.
-__device__ __forceinline__ int refill_slot(int* work, int n, unsigned long long idle, bool& drained) {
-    const int want = __popcll(idle);
-    const int leader = __ffsll((long long)idle) - 1;
-    int base = 0;
-    if (lane_id() == leader) base = atomicAdd(work, want);
-    base = __shfl(base, leader);
-    if (base + want >= n) drained = true;
-    if (!((idle >> lane_id()) & 1ull)) return -1;
-    const int slot = base + lane_rank(idle);
-    return slot < n ? slot : -1;
-}
-
-template <int kMode, int kBlock, int kLds>
-__global__ __launch_bounds__(kBlock) void k_wf_extend_refill(PtScene S0, WfState W, int buf, int count, int work,
-                                                             const int* perm, int budget) {
-    __shared__ int sStack[kLds * kBlock];
-    constexpr bool kBatch = kMode == 2;
-    using T = Traversal<false, false, traversal_mode<kMode>(), kBlock, kLds, kMode == kTraceMixed>;
-    const int n = W.counters[count];
-    int* const lstack = sStack + threadIdx.x;
-    int spill[T::kSpill];
-    T tr;
-    int q = -1, si = 0;
-    bool drained = false;
-    while (true) {
-        const unsigned long long idle = __ballot(q < 0);
-        if (!drained && __popcll(idle) >= kRefillMinIdle) {
-            const int slot = refill_slot(W.counters + work, n, idle, drained);
-            if (slot >= 0) {
-                q = perm ? perm[slot] : slot;
-                const float4 o = W.rayO[buf][q];
-                const float4 d = W.rayD[buf][q];
-                int local;
-                si = locate<kBatch>(W, __float_as_int(d.w), local);
-                tr.init(scene_ref<kBatch>(S0, W, si).trace, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), kMaxSceneSize);
-            }
-        }
-        if (__ballot(q >= 0) == 0) break;  // nothing in flight: the queue is drained
-        if (q >= 0 && tr.template run<true>(scene_ref<kBatch>(S0, W, si).trace, lstack, spill, budget)) {
-            const TraceHit h = tr.result();
-            W.hit[buf][q] = float4{h.t, __int_as_float(h.inst), __int_as_float(h.prim), h.w0};
-            W.rayM[buf][q].w = h.w1;
-            q = -1;
-        }
-    }
-}
-
-template <int kMode, int kBlock, int kLds>
-__global__ __launch_bounds__(kBlock) void k_wf_shadow_refill(PtScene S0, WfState W, int count, int work,
-                                                             const int* perm, int budget) {
-    __shared__ int sStack[kLds * kBlock];
-    constexpr bool kBatch = kMode == 2;
-    using T = Traversal<true, false, traversal_mode<kMode>(), kBlock, kLds, kMode == kTraceMixed>;
-    const int n = W.counters[count];
-    int* const lstack = sStack + threadIdx.x;
-    int spill[T::kSpill];
-    T tr;
-    int sl = -1, si = 0, path = 0, cur = 0;
-    u32 remaining = 0, visible = 0;
-    bool drained = false;
-    // next candidate of the slot, or its result once every candidate is traced
-    auto advance = [&]() {
-        while (sl >= 0) {
-            if (remaining) {
-                cur = __ffs(remaining) - 1;
-                remaining &= remaining - 1;
-                const size_t e = (size_t)sl * W.neeStride + cur;
-                const float4 a = W.shO[e];
-                const float4 d = W.shD[e];
-                tr.init(scene_ref<kBatch>(S0, W, si).trace, v3(a.x, a.y, a.z), v3(d.x, d.y, d.z), a.w);
-                return;
-            }
-            if (visible) {  // add the unoccluded estimates in candidate order
-                const PtScene& S = scene_ref<kBatch>(S0, W, si);
-                Acc acc;
-                load_acc(W, S.targetMask, path, acc);
-                for (int i = 0; i < S.neeCount; ++i) {
-                    if (!((visible >> i) & 1u)) continue;
-                    const float4 c = W.shC[(size_t)sl * W.neeStride + i];
-                    NeeCandidate nc;
-                    nc.radiance = v3(c.x, c.y, c.z);
-                    nc.lightness = c.w;
-                    add_nee(nc, acc);
-                }
-                store_acc(W, S.targetMask, path, acc);
-                if (acc.nans) atomicAdd(S.nanCounter, acc.nans);
-            }
-            sl = -1;
-        }
-    };
-    while (true) {
-        const unsigned long long idle = __ballot(sl < 0);
-        if (!drained && __popcll(idle) >= kRefillMinIdle) {
-            const int slot = refill_slot(W.counters + work, n, idle, drained);
-            if (slot >= 0) {
-                sl = perm ? perm[slot] : slot;
-                const int2 pm = W.shPath[sl];
-                path = pm.x;
-                remaining = (u32)pm.y;
-                visible = 0;
-                int local;
-                si = locate<kBatch>(W, path, local);
-                advance();
-            }
-        }
-        if (__ballot(sl >= 0) == 0) break;
-        if (sl >= 0 && tr.template run<true>(scene_ref<kBatch>(S0, W, si).trace, lstack, spill, budget)) {
-            if (tr.result().inst == -1) visible |= 1u << cur;
-            advance();
+            if (visible) add(pm.x, sl, visible);
         }
     }
 }
@@ -489,7 +401,7 @@ __global__ __launch_bounds__(256) void k_wf_shade(PtScene S0, WfState W, int k, 
 // ray. Random numbers are drawn, and contributions reach the accumulator, in
 // the order of the staged kernels and of the megakernel (emission of a vertex,
 // its next-event estimates, the next vertex), so the bits are the same.
-template <int kMode, int kLeaf>
+template <int kMode>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_wf_tail(PtScene S0, WfState W, int k,
                                                                                        int buf, int count, int work) {
     __shared__ int sStack[kLdsDepth * 256];
@@ -543,7 +455,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                         NeeCandidate c;
                         if (nee_candidate(S, vx, throughput, guideWeight, i, neeSeed, x, c)) {
                             const TraceHit sh =
-                                trace_mode<kMode, true, 256, kLdsDepth, kLeaf>(S.trace, c.a, c.dir, c.tmax, lstack);
+                                trace_mode<kMode, true, 256, kLdsDepth>(S.trace, c.a, c.dir, c.tmax, lstack);
                             if (sh.inst == -1) add_nee(c, acc);
                         }
                     }
@@ -553,7 +465,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                 const float rndRoulette = sample_uniform((u32)pcg_next(rng));
                 if (!walk_surface(vx, x0, x1, rndRoulette, throughput, rayOrigin, dir, pdfF, absorption)) break;
                 prevPos = vx.position;
-                hit = trace_mode<kMode, false, 256, kLdsDepth, kLeaf>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
+                hit = trace_mode<kMode, false, 256, kLdsDepth>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
             }
             S.rngs[local] = rng;
             store_acc(W, S.targetMask, p, acc);
@@ -626,46 +538,29 @@ __global__ void k_wf_finish(PtScene S0, WfState W) {
     accumulate(S, (size_t)local, *W.iteration, v, S.targetMask);
 }
 
-template <int kMode, int kBlock, int kLds, int kLeaf>
+template <int kMode, int kBlock, int kLds>
 struct TraceKernels {
     static void extend(const PtScene& S, const WfState& W, int grid, int buf, int count, int work, const int* perm,
-                       int refill, hipStream_t st) {
-        if (refill > 0)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_extend_refill<kMode, kBlock, kLds>), dim3(grid), dim3(kBlock), 0,
-                               st, S, W, buf, count, work, perm, refill);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_extend<kMode, kBlock, kLds, kLeaf>), dim3(grid), dim3(kBlock), 0,
-                               st, S, W, buf, count, work, perm);
-    }
-    static void shadow(const PtScene& S, const WfState& W, int grid, int count, int work, const int* perm, int refill,
                        hipStream_t st) {
-        if (refill > 0)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_shadow_refill<kMode, kBlock, kLds>), dim3(grid), dim3(kBlock), 0,
-                               st, S, W, count, work, perm, refill);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_shadow<kMode, kBlock, kLds, kLeaf>), dim3(grid), dim3(kBlock), 0,
-                               st, S, W, count, work, perm);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_extend<kMode, kBlock, kLds>), dim3(grid), dim3(kBlock), 0, st, S, W,
+                           buf, count, work, perm);
     }
-    static int occupancy(bool refill) {
+    static void shadow(const PtScene& S, const WfState& W, int grid, int count, int work, const int* perm,
+                       hipStream_t st) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_shadow<kMode, kBlock, kLds>), dim3(grid), dim3(kBlock), 0, st, S, W,
+                           count, work, perm);
+    }
+    static int occupancy() {
         int a = 0, b = 0;
-        if (refill) {
-            MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_wf_extend_refill<kMode, kBlock, kLds>, kBlock,
-                                                                 0));
-            MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_shadow_refill<kMode, kBlock, kLds>, kBlock,
-                                                                 0));
-        } else {
-            MFH_HIP(
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_wf_extend<kMode, kBlock, kLds, kLeaf>, kBlock, 0));
-            MFH_HIP(
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_shadow<kMode, kBlock, kLds, kLeaf>, kBlock, 0));
-        }
+        MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_wf_extend<kMode, kBlock, kLds>, kBlock, 0));
+        MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_shadow<kMode, kBlock, kLds>, kBlock, 0));
         return std::max(1, std::min(a, b));
     }
 };
 
-using ExtendFn = void (*)(const PtScene&, const WfState&, int, int, int, int, const int*, int, hipStream_t);
-using ShadowFn = void (*)(const PtScene&, const WfState&, int, int, int, const int*, int, hipStream_t);
-using OccFn = int (*)(bool);
+using ExtendFn = void (*)(const PtScene&, const WfState&, int, int, int, int, const int*, hipStream_t);
+using ShadowFn = void (*)(const PtScene&, const WfState&, int, int, int, const int*, hipStream_t);
+using OccFn = int (*)();
 
 struct TraceVariant {
     ExtendFn extend;
@@ -673,48 +568,35 @@ struct TraceVariant {
     OccFn occupancy;
 };
 
-template <int kMode, int kBlock, int kLds, int kLeaf>
+template <int kMode, int kBlock, int kLds>
 constexpr TraceVariant variant() {
-    return {&TraceKernels<kMode, kBlock, kLds, kLeaf>::extend, &TraceKernels<kMode, kBlock, kLds, kLeaf>::shadow,
-            &TraceKernels<kMode, kBlock, kLds, kLeaf>::occupancy};
+    return {&TraceKernels<kMode, kBlock, kLds>::extend, &TraceKernels<kMode, kBlock, kLds>::shadow,
+            &TraceKernels<kMode, kBlock, kLds>::occupancy};
 }
 
-// Tuning space of the trace stages: block size x LDS stack depth x leaf
-// batch (1 or 8 triangles loaded ahead; the lane-refill kernels test one at a
-// time), for multi-instance scenes (0), single-instance scenes (1), batches
-// (2) and scenes with quads or spheres (3).
-template <int kMode, int kLeaf>
-constexpr std::array<TraceVariant, 7> shapes() {
-    return {variant<kMode, 64, 8, kLeaf>(),   variant<kMode, 64, 16, kLeaf>(),  variant<kMode, 128, 8, kLeaf>(),
-            variant<kMode, 128, 16, kLeaf>(), variant<kMode, 256, 8, kLeaf>(),  variant<kMode, 256, 16, kLeaf>(),
-            variant<kMode, 256, 24, kLeaf>()};
-}
+// Tuning space of the trace stages: block size x LDS stack depth, for
+// multi-instance scenes (0), single-instance scenes (1), batches (2) and
+// scenes with quads or spheres (3).
 template <int kMode>
-std::array<TraceVariant, kWfNumTraceVariants> variants() {
-    const std::array<TraceVariant, 7> a = shapes<kMode, 1>(), b = shapes<kMode, 8>();
-    std::array<TraceVariant, kWfNumTraceVariants> v{};
-    for (int i = 0; i < 7; ++i) {
-        v[i] = a[i];
-        v[7 + i] = b[i];
-    }
-    return v;
+constexpr std::array<TraceVariant, kWfNumTraceVariants> variants() {
+    return {variant<kMode, 64, 8>(),   variant<kMode, 64, 16>(), variant<kMode, 128, 8>(), variant<kMode, 128, 16>(),
+            variant<kMode, 256, 8>(), variant<kMode, 256, 16>(), variant<kMode, 256, 24>()};
 }
 const std::array<TraceVariant, kWfNumTraceVariants> kVariants[4] = {variants<0>(), variants<1>(), variants<2>(),
                                                                      variants<3>()};
 
 }  // namespace
 
-const WfTraceShape kWfTraceShapes[kWfNumTraceVariants] = {
-    {64, 8, 1}, {64, 16, 1}, {128, 8, 1}, {128, 16, 1}, {256, 8, 1}, {256, 16, 1}, {256, 24, 1},
-    {64, 8, 8}, {64, 16, 8}, {128, 8, 8}, {128, 16, 8}, {256, 8, 8}, {256, 16, 8}, {256, 24, 8}};
+const WfTraceShape kWfTraceShapes[kWfNumTraceVariants] = {{64, 8},  {64, 16},  {128, 8}, {128, 16},
+                                                          {256, 8}, {256, 16}, {256, 24}};
 
 int wf_grid(const PtScene& S, const WfTuning& tune, int numCUs) {
     const TraceVariant& v = kVariants[trace_mode_of(S.trace)][tune.traceVariant];
-    return v.occupancy(tune.refill > 0) * numCUs;
+    return v.occupancy() * numCUs;
 }
 
 int wf_grid_batch(const WfTuning& tune, int numCUs) {
-    return kVariants[2][tune.traceVariant].occupancy(tune.refill > 0) * numCUs;
+    return kVariants[2][tune.traceVariant].occupancy() * numCUs;
 }
 
 int wf_shade_grid(int numCUs) {
@@ -726,28 +608,18 @@ int wf_shade_grid(int numCUs) {
 
 int wf_tail_grid(int numCUs) {
     int a = 0, b = 0, c = 0, d = 0;
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_wf_tail<0, 1>, 256, 0));
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_tail<1, 8>, 256, 0));
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, k_wf_tail<2, 1>, 256, 0));
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&d, k_wf_tail<3, 8>, 256, 0));
+    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_wf_tail<0>, 256, 0));
+    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_tail<1>, 256, 0));
+    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, k_wf_tail<2>, 256, 0));
+    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&d, k_wf_tail<3>, 256, 0));
     return std::max(1, std::min(std::min(a, d), std::min(b, c))) * numCUs;
 }
 
 namespace {
-void launch_tail(int mode, bool leaf8, const PtScene& S, const WfState& W, int grid, int k, int buf, int count,
-                 int work, hipStream_t st) {
-#define MFH_TAIL(M, L) \
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_tail<M, L>), dim3(grid), dim3(256), 0, st, S, W, k, buf, count, work)
-    if (mode == 0) {
-        if (leaf8) MFH_TAIL(0, 8); else MFH_TAIL(0, 1);
-    } else if (mode == 1) {
-        if (leaf8) MFH_TAIL(1, 8); else MFH_TAIL(1, 1);
-    } else if (mode == 2) {
-        if (leaf8) MFH_TAIL(2, 8); else MFH_TAIL(2, 1);
-    } else {
-        if (leaf8) MFH_TAIL(3, 8); else MFH_TAIL(3, 1);
-    }
-#undef MFH_TAIL
+void launch_tail(int mode, const PtScene& S, const WfState& W, int grid, int k, int buf, int count, int work,
+                 hipStream_t st) {
+    auto* const fn = mode == 0 ? k_wf_tail<0> : (mode == 1 ? k_wf_tail<1> : (mode == 2 ? k_wf_tail<2> : k_wf_tail<3>));
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, st, S, W, k, buf, count, work);
     MFH_HIP(hipGetLastError());
 }
 }  // namespace
@@ -766,16 +638,9 @@ void launch_pt_wavefront(const PtScene& S, const WfState& W, const WfTuning& tun
     const TraceVariant& v = kVariants[mode][tune.traceVariant];
     hipLaunchKernelGGL(k_wf_begin, dim3((W.numCounters + 255) / 256), dim3(256), 0, stream, W);
     const dim3 pgrid((S.width + 15) / 16, (S.height + 15) / 16);
-    const bool leaf8 = kWfTraceShapes[tune.traceVariant].leafBatch == 8;
-#define MFH_PRIMARY(M, L) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_primary<M, L>), pgrid, dim3(256), 0, stream, S, W)
-    if (mode == kTraceSingle) {
-        if (leaf8) MFH_PRIMARY(1, 8); else MFH_PRIMARY(1, 1);
-    } else if (mode == kTraceMulti) {
-        if (leaf8) MFH_PRIMARY(0, 8); else MFH_PRIMARY(0, 1);
-    } else {
-        if (leaf8) MFH_PRIMARY(3, 8); else MFH_PRIMARY(3, 1);
-    }
-#undef MFH_PRIMARY
+    auto* const primary =
+        mode == kTraceSingle ? k_wf_primary<1> : (mode == kTraceMulti ? k_wf_primary<0> : k_wf_primary<3>);
+    hipLaunchKernelGGL(primary, pgrid, dim3(256), 0, stream, S, W);
     // pt_sample's loop is a do-while: the first hit is shaded even at maximum path length 0
     const int L = S.maxPathLength > 1 ? S.maxPathLength : 1;
     int work = W.workBase;
@@ -785,13 +650,12 @@ void launch_pt_wavefront(const PtScene& S, const WfState& W, const WfTuning& tun
                            buf, W.qBase + k, W.qBase + k + 1, W.shBase + k, work++);
         const bool sortNow = k < tune.sortBounces;
         if (sortNow) sort_queue(S, W, 0, W.shBase + k, true, scratch, stream);
-        v.shadow(S, W, tune.traceGrid, W.shBase + k, work++, sortNow ? W.sortIds[0] : nullptr, tune.refill, stream);
+        v.shadow(S, W, tune.traceGrid, W.shBase + k, work++, sortNow ? W.sortIds[0] : nullptr, stream);
         if (k + 1 < L) {
             if (sortNow) sort_queue(S, W, buf ^ 1, W.qBase + k + 1, false, scratch, stream);
-            v.extend(S, W, tune.traceGrid, buf ^ 1, W.qBase + k + 1, work++, sortNow ? W.sortIds[0] : nullptr,
-                     tune.refill, stream);
+            v.extend(S, W, tune.traceGrid, buf ^ 1, W.qBase + k + 1, work++, sortNow ? W.sortIds[0] : nullptr, stream);
             if (tune.tailAfter > 0 && k + 1 == tune.tailAfter) {  // the rest of every path in one launch
-                launch_tail(mode, leaf8, S, W, tune.tailGrid, k + 1, buf ^ 1, W.qBase + k + 1, work++, stream);
+                launch_tail(mode, S, W, tune.tailGrid, k + 1, buf ^ 1, W.qBase + k + 1, work++, stream);
                 break;
             }
         }
@@ -806,24 +670,18 @@ void launch_pt_wavefront_batch(const WfState& W, const WfTuning& tune, int maxLe
     std::memset(&none, 0, sizeof(none));
     const TraceVariant& v = kVariants[2][tune.traceVariant];
     hipLaunchKernelGGL(k_wf_begin, dim3((W.numCounters + 255) / 256), dim3(256), 0, stream, W);
-    if (kWfTraceShapes[tune.traceVariant].leafBatch == 8)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_primary<2, 8>), dim3((W.numPaths + 255) / 256), dim3(256), 0, stream,
-                           none, W);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_primary<2, 1>), dim3((W.numPaths + 255) / 256), dim3(256), 0, stream,
-                           none, W);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_primary<2>), dim3((W.numPaths + 255) / 256), dim3(256), 0, stream, none, W);
     const int L = maxLen > 1 ? maxLen : 1;
     int work = W.workBase;
     for (int k = 0; k < L; ++k) {
         const int buf = k & 1;
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_shade<true>), dim3(tune.shadeGrid), dim3(256), 0, stream, none, W, k,
                            buf, W.qBase + k, W.qBase + k + 1, W.shBase + k, work++);
-        v.shadow(none, W, tune.traceGrid, W.shBase + k, work++, nullptr, tune.refill, stream);
+        v.shadow(none, W, tune.traceGrid, W.shBase + k, work++, nullptr, stream);
         if (k + 1 < L) {
-            v.extend(none, W, tune.traceGrid, buf ^ 1, W.qBase + k + 1, work++, nullptr, tune.refill, stream);
+            v.extend(none, W, tune.traceGrid, buf ^ 1, W.qBase + k + 1, work++, nullptr, stream);
             if (tune.tailAfter > 0 && k + 1 == tune.tailAfter) {
-                launch_tail(2, kWfTraceShapes[tune.traceVariant].leafBatch == 8, none, W, tune.tailGrid, k + 1,
-                            buf ^ 1, W.qBase + k + 1, work++, stream);
+                launch_tail(2, none, W, tune.tailGrid, k + 1, buf ^ 1, W.qBase + k + 1, work++, stream);
                 break;
             }
         }

@@ -39,16 +39,17 @@ struct WfState {
 };
 
 struct WfTraceShape {
-    int block, lds, leafBatch;
+    int block, lds;
 };
-constexpr int kWfNumTraceVariants = 14;
+constexpr int kWfNumTraceVariants = 7;
 extern const WfTraceShape kWfTraceShapes[kWfNumTraceVariants];
 
 struct WfTuning {
-    int traceVariant = 5;  // 256 threads, 16 LDS stack entries, leaf batch 1
+    int traceVariant = 5;  // 256 threads, 16 LDS stack entries
     int chunk = 256;
     int sortBounces = 0;   // extension / shadow queues of the first bounces traced in sorted order
-    int refill = 0;        // > 0: trace stages refill idle lanes every `refill` traversal steps
+    int refill = 0;        // recorded for the caller: the traversal has one form
+    int leafBatch = 1;     // likewise
     int tailAfter = 0;     // > 0: after the extension rays of this bounce, one launch finishes every path
     int traceGrid = 0;
     int shadeGrid = 0;

@@ -2,20 +2,23 @@
 // kernels and the path tracer: the GPU device of Mufflon's first_intersection /
 // any_intersection (intersection.cu:366-753).
 //
-// One ray per lane. The stack keeps its lowest kLdsDepth entries in LDS (one
-// column per lane, so the 64 lanes of a wave touch 64 consecutive dwords) and
-// spills deeper entries to a per-lane private array. Nodes are Mufflon's
-// 64-byte collapsed LBVH nodes, read as four 16-byte loads; the primitives of
+// One ray per lane, through two levels: the instances over Mufflon's 64-byte
+// collapsed LBVH nodes in the reference's order, the primitives of an object
+// over its 4-wide traversal hierarchy (k_wide in lbvh.hip). The primitives of
 // a leaf are contiguous 48-byte records in BVH order ({v0, primId}, {v1, kind},
 // {v2} for triangles and quads, {center, primId}, {radius, .., kind} for
-// spheres).
+// spheres). The stack keeps its lowest kLdsDepth entries in LDS (one column
+// per lane, so the 64 lanes of a wave touch 64 consecutive dwords) and spills
+// deeper entries to a per-lane private array.
 //
-// Visiting order and box test are those of the reference CPU path: the slab
-// test of intersection.cu:57-75 (computed without its early outs, which give
-// the same accept/reject and entry distance), nearer child first with ties to
-// the left, the farther child pushed, leaves pushed as (count, index), and the
-// two-level instance transition of intersection.cu:321-361. Closest hit is the
-// lexicographic minimum of (t, instance, primitive).
+// A primitive is tested where its leaf's box, in full precision, passes the
+// slab test of the reference CPU path (intersection.cu:57-75); the quantized
+// boxes above contain that box and are tested with an error margin, so they
+// only cull. (A node step replaces two binary ones, with half their dependent
+// loads; 44 -> 23.5 steps a ray on a 1M-triangle mesh, 8.3 triangle tests.) Closest hit is the lexicographic minimum of (t, instance,
+// primitive), which does not depend on the order inside an object; the order
+// of the objects, whose entry and exit round the hit distance
+// (intersection.cu:321-361), is the reference's.
 #pragma once
 #include "mfh_device.hpp"
 #include "mfh_internal.hpp"
@@ -23,14 +26,9 @@
 namespace mfh {
 
 constexpr int kSentinel = (int)0xFFFFFFFF;
-constexpr int kStackCap = 128;
-constexpr int kTraceThreads = 256;
+constexpr int kStackCap = 128;  // entries of the binary traversals
+constexpr int kWideCap = 64;    // entries of the wide traversal; fuller stacks take reference_ray
 constexpr int kLdsDepth = 16;
-// Leaf batch (trace_ray's kBatch) of the path-tracing kernels: on scenes with
-// long leaves (a 10M-triangle heightfield leaves up to ~1400 triangle tests on
-// one ray) the slowest rays of a launch are bound by one memory latency per
-// triangle; the plain trace kernels keep 1, which is faster on small leaves.
-constexpr int kPtLeafBatch = 8;
 
 // A load of BVH-node or triangle data as a global-memory load: the pointers
 // arrive in structs as generic pointers, whose loads would compile to flat
@@ -199,254 +197,38 @@ struct TraceHit {
     unsigned nodeVisits, primTests;
 };
 
-// Resumable traversal of one ray: trace_ray's loops (below) with their state
-// kept in a struct, so that run() can stop after a budget of steps (node
-// visits and primitive tests) and continue later. The persistent wavefront
-// kernels use it to refill lanes whose ray has finished while the rest of
-// the wave is still traversing. It takes the same steps as trace_ray, so the
-// result of a ray does not depend on how its traversal is split; trace_ray
-// stays a separate straight-line form because the resumable one needs more
-// registers.
-// kSingleMode: 1 = one instance (no instance level), 0 = instance level,
-// 2 = chosen per ray at init (batches mix both kinds of scenes).
-// The stack's deeper entries live in a private array of the caller
-// (kSpill ints), passed to run() so that the struct itself holds only
-// scalars and stays in registers.
-template <bool kAny, bool kStats, int kSingleMode, int kStride, int kLds = kLdsDepth, bool kMixed = false>
-struct Traversal {
-    static constexpr int kSpill = kStackCap - kLds;
-    FastRay cur;
-    V3 wo, wd;
-    float hitT, hw0, hw1, scale;
-    int hInst, hPrim;
-    const BvhChild* bvh;
-    const float4* tris;
-    int numInternal, objPrims, curInst;
-    int nodeAddr, primCount, primOffset, sp;
-    bool inObj, overflow, done, single;
-    unsigned nodeVisits, primTests;
-
-    __device__ __forceinline__ bool is_single() const {
-        if constexpr (kSingleMode == 2)
-            return single;
-        else
-            return kSingleMode == 1;
-    }
-    __device__ __forceinline__ void push(int* lstack, int* spill, int v) {
-        if (sp < kLds)
-            lds_at(lstack, sp * kStride) = v;
-        else if (sp < kStackCap)
-            spill[sp - kLds] = v;
-        if (sp < kStackCap)
-            ++sp;
-        else
-            overflow = true;
-    }
-    __device__ __forceinline__ int pop(const int* lstack, const int* spill) {
-        --sp;
-        return sp < kLds ? lds_at(lstack, sp * kStride) : spill[sp - kLds];
-    }
-
-    __device__ __forceinline__ void init(const TraceParams& p, V3 o, V3 d, float tmax) {
-        wo = o;
-        wd = d;
-        sp = 0;
-        overflow = done = false;
-        cur = make_fast_ray(wo, wd);
-        hitT = tmax;
-        hInst = hPrim = -1;
-        hw0 = hw1 = 0.0f;
-        scale = 1.0f;
-        nodeVisits = primTests = 0;
-        bvh = (const BvhChild*)p.tlasNodes;
-        tris = nullptr;
-        numInternal = p.tlasNumInternal;
-        objPrims = 0;
-        inObj = false;
-        curInst = -1;
-        nodeAddr = 0;
-        primCount = 2;
-        primOffset = 0;
-        if constexpr (kSingleMode == 2) single = p.numInstances == 1;
-        if (is_single()) {
-            DevLod lod;
-            const ObjectEntry e = enter_object(p, 0, wo, wd, hitT, lod);
-            if (kStats) ++nodeVisits;
-            if (!e.hit) {
-                primCount = 0;
-            } else {
-                cur = e.ray;
-                scale = e.scale;
-                hitT = e.tmax;
-                bvh = (const BvhChild*)lod.nodes;
-                tris = lod.triVerts;
-                numInternal = lod.numInternal;
-                inObj = true;
-                curInst = 0;
-                if (lod.numPrims == 1) primCount = 1;
-            }
-        }
-    }
-
-    // Advance by at most `budget` steps (kBudget) or to the end; true when
-    // the ray is finished.
-    template <bool kBudget>
-    __device__ __forceinline__ bool run(const TraceParams& p, int* lstack, int* spill, int budget) {
-        while (true) {
-            // descend through internal nodes, nearer child first, farther pushed
-            while (nodeAddr < numInternal && primCount > 0) {
-                if (kBudget && budget-- <= 0) return false;
-                const float4* nd = reinterpret_cast<const float4*>(bvh + 2 * (size_t)nodeAddr);
-                const float4 q0 = gload(nd), q1 = gload(nd + 1), q2 = gload(nd + 2), q3 = gload(nd + 3);
-                if (kStats) ++nodeVisits;
-                const float lLo[3] = {q0.x, q0.y, q0.z}, lHi[3] = {q0.w, q1.x, q1.y};
-                const float rLo[3] = {q2.x, q2.y, q2.z}, rHi[3] = {q2.w, q3.x, q3.y};
-                const int lIdx = __float_as_int(q1.z), lCnt = __float_as_int(q1.w);
-                const int rIdx = __float_as_int(q3.z), rCnt = __float_as_int(q3.w);
-                float c0, c1;
-                const bool t0 = slab(lLo, lHi, cur, hitT, c0);
-                const bool t1 = slab(rLo, rHi, cur, hitT, c1);
-                if (!t0) c0 = 1e38f;
-                if (!t1) c1 = 1e38f;
-                if (t0 && t1) {
-                    const bool farLeft = c1 < c0;
-                    const int pushed = farLeft ? lIdx : rIdx;
-                    if (pushed >= numInternal) push(lstack, spill, farLeft ? lCnt : rCnt);
-                    push(lstack, spill, pushed);
-                }
-                const bool nearLeft = c0 <= c1;
-                nodeAddr = nearLeft ? lIdx : rIdx;
-                primCount = (nodeAddr >= numInternal) ? (nearLeft ? lCnt : rCnt) : 2;
-                primOffset = 0;
-                if (!t0 && !t1) primCount = 0;
-            }
-            if (overflow) return true;
-            // the primitives of a leaf, one after the other
-            bool descend = false;
-            while (nodeAddr >= numInternal && primCount > 0) {
-                if (kBudget && budget-- <= 0) return false;
-                const int leafId = nodeAddr - numInternal + primOffset;
-                ++primOffset;
-                --primCount;
-                if (!is_single() && !inObj) {
-                    const int inst = p.tlasPrimIds[leafId];
-                    DevLod lod;
-                    const ObjectEntry e = enter_object(p, inst, wo, wd, hitT, lod);
-                    if (kStats) ++nodeVisits;
-                    if (!e.hit) continue;
-                    if (lod.numPrims == 1) {
-                        // single-primitive object: test it and return to the instance level
-                        const float4 a = lod.triVerts[0], b = lod.triVerts[1], c = lod.triVerts[2];
-                        float t, w0, w1;
-                        if (kStats) ++primTests;
-                        const float objT = e.tmax;
-                        float ht = objT;
-                        if (prim_hit<kMixed>(e.ray, a, b, c, 0, [&] { return lod.quadV3; }, t, w0, w1) &&
-                            better(t, inst, __float_as_int(a.w), ht, hInst, hPrim)) {
-                            ht = t;
-                            hInst = inst;
-                            hPrim = __float_as_int(a.w);
-                            hw0 = w0;
-                            hw1 = w1;
-                            if (kAny) done = true;
-                        }
-                        hitT = ht / e.scale;
-                        if (done) return true;
-                        continue;
-                    }
-                    if (primCount > 0) {
-                        push(lstack, spill, primCount);
-                        push(lstack, spill, nodeAddr + primOffset);
-                    }
-                    push(lstack, spill, kSentinel);
-                    cur = e.ray;
-                    scale = e.scale;
-                    hitT = e.tmax;
-                    bvh = (const BvhChild*)lod.nodes;
-                    tris = lod.triVerts;
-                    numInternal = lod.numInternal;
-                    objPrims = lod.numPrims;
-                    inObj = true;
-                    curInst = inst;
-                    nodeAddr = 0;
-                    primCount = objPrims == 1 ? 1 : 2;
-                    primOffset = 0;
-                    descend = true;
-                    break;
-                }
-                const float4 a = gload(tris + 3 * (size_t)leafId), b = gload(tris + 3 * (size_t)leafId + 1),
-                             c = gload(tris + 3 * (size_t)leafId + 2);
-                float t, w0, w1;
-                const int prim = __float_as_int(a.w);
-                if (kStats) ++primTests;
-                if (prim_hit<kMixed>(cur, a, b, c, leafId, [&] { return p.lods[p.instLod[curInst]].quadV3; }, t, w0,
-                                     w1) &&
-                    better(t, curInst, prim, hitT, hInst, hPrim)) {
-                    hitT = t;
-                    hInst = curInst;
-                    hPrim = prim;
-                    hw0 = w0;
-                    hw1 = w1;
-                    if (kAny) {
-                        done = true;
-                        return true;
-                    }
-                }
-            }
-            if (overflow) return true;
-            if (descend) continue;
-            // pop the next subtree (or return from an object to the instance level)
-            if (sp == 0) return true;
-            nodeAddr = pop(lstack, spill);
-            if (!is_single() && nodeAddr == kSentinel) {
-                if (sp == 0) return true;
-                cur = make_fast_ray(wo, wd);
-                hitT /= scale;
-                scale = 1.0f;
-                bvh = (const BvhChild*)p.tlasNodes;
-                numInternal = p.tlasNumInternal;
-                inObj = false;
-                nodeAddr = pop(lstack, spill);
-            }
-            primCount = (nodeAddr >= numInternal) ? pop(lstack, spill) : 2;
-            primOffset = 0;
-        }
-    }
-
-    // On return t is the world-space distance (or the round-tripped tmax on
-    // a miss) and inst/prim are -1 on a miss.
-    __device__ __forceinline__ TraceHit result() const {
-        TraceHit h;
-        h.t = (!kAny && inObj) ? hitT / scale : hitT;  // object_to_world_space
-        h.inst = hInst;
-        h.prim = hPrim;
-        h.w0 = hw0;
-        h.w1 = hw1;
-        h.overflow = overflow;
-        h.nodeVisits = nodeVisits;
-        h.primTests = primTests;
-        return h;
-    }
-};
-
-// Traverse from (wo, wd) up to tmax. lstack: this lane's LDS stack column
-// (stride kStride ints). On return t is the world-space distance (or the
-// round-tripped tmax on a miss) and inst/prim are -1 on a miss.
-template <bool kAny, bool kStats, bool kSingle, int kStride, int kLds = kLdsDepth, int kBatch = 1,
-          bool kMixed = false>
-__device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd, float tmax, int* const lstack) {
-    int spill[kStackCap - kLds];
+// Closest or any hit over the reference's BVHs in its order (nearer child
+// first with ties to the left, the farther child pushed, leaves pushed as
+// (count, index)) with its compare-select slab test. The visit counts come
+// from it (kCount: internal nodes visited, an object-box test at instance
+// entry among them, and primitives tested), and it takes the rays that the
+// wide traversals hand over: rays whose slab values may be NaN (slab_finite)
+// and rays that fill the wide stack. Both are rare, so it is a call: its
+// registers and its stack burden no kernel's main path.
+template <bool kAny, bool kCount, bool kMixed>
+__device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstances, const float* worldToInst,
+                                                             const int32_t* instLod, const DevLod* lods,
+                                                             const void* tlasNodes, const int32_t* tlasPrimIds,
+                                                             int tlasNumInternal, V3 wo, V3 wd, float tmax) {
+    TraceParams p;
+    p.numInstances = numInstances;
+    p.worldToInst = worldToInst;
+    p.instLod = instLod;
+    p.lods = lods;
+    p.tlasNodes = tlasNodes;
+    p.tlasPrimIds = tlasPrimIds;
+    p.tlasNumInternal = tlasNumInternal;
+    const bool single = p.numInstances == 1;
+    int stack[kStackCap];
     int sp = 0;
     bool overflow = false;
-#define MFH_PUSH(v)                                     \
-    do {                                                \
-        if (sp < kLds)                                  \
-            lds_at(lstack, sp * kStride) = (v);                 \
-        else if (sp < kStackCap)                        \
-            spill[sp - kLds] = (v);                     \
-        if (sp < kStackCap) ++sp; else overflow = true; \
-    } while (0)
-#define MFH_POP() (--sp, (sp < kLds) ? lds_at(lstack, sp * kStride) : spill[sp - kLds])
+    auto push = [&](int v) {
+        if (sp < kStackCap)
+            stack[sp++] = v;
+        else
+            overflow = true;
+    };
+    auto pop = [&]() { return stack[--sp]; };
 
     FastRay cur = make_fast_ray(wo, wd);
     float hitT = tmax;
@@ -464,18 +246,15 @@ __device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd
     int curInst = -1;
     int nodeAddr = 0, primCount = 2, primOffset = 0;
     bool done = false;
-    // no NaN can reach this lane's slab tests at the current level
-    bool finite = slab_finite(cur, p.tlasCoordMax);
 
-    if (kSingle) {
+    if (single) {
         DevLod lod;
         const ObjectEntry e = enter_object(p, 0, wo, wd, hitT, lod);
-        if (kStats) ++nodeVisits;
+        if (kCount) ++nodeVisits;
         if (!e.hit) {
             primCount = 0;
         } else {
             cur = e.ray;
-            finite = slab_finite(cur, lod.coordMax);
             scale = e.scale;
             hitT = e.tmax;
             bvh = (const BvhChild*)lod.nodes;
@@ -492,21 +271,20 @@ __device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd
         while (nodeAddr < numInternal && primCount > 0) {
             const float4* nd = reinterpret_cast<const float4*>(bvh + 2 * (size_t)nodeAddr);
             const float4 q0 = gload(nd), q1 = gload(nd + 1), q2 = gload(nd + 2), q3 = gload(nd + 3);
-            if (kStats) ++nodeVisits;
+            if (kCount) ++nodeVisits;
             const float lLo[3] = {q0.x, q0.y, q0.z}, lHi[3] = {q0.w, q1.x, q1.y};
             const float rLo[3] = {q2.x, q2.y, q2.z}, rHi[3] = {q2.w, q3.x, q3.y};
             const int lIdx = __float_as_int(q1.z), lCnt = __float_as_int(q1.w);
             const int rIdx = __float_as_int(q3.z), rCnt = __float_as_int(q3.w);
             float c0, c1;
-            bool t0, t1;
-            slab_pair(__all(finite), lLo, lHi, rLo, rHi, cur, hitT, t0, t1, c0, c1);
+            const bool t0 = slab(lLo, lHi, cur, hitT, c0), t1 = slab(rLo, rHi, cur, hitT, c1);
             if (!t0) c0 = 1e38f;
             if (!t1) c1 = 1e38f;
             if (t0 && t1) {
                 const bool farLeft = c1 < c0;
-                const int push = farLeft ? lIdx : rIdx;
-                if (push >= numInternal) MFH_PUSH(farLeft ? lCnt : rCnt);
-                MFH_PUSH(push);
+                const int far = farLeft ? lIdx : rIdx;
+                if (far >= numInternal) push(farLeft ? lCnt : rCnt);
+                push(far);
             }
             const bool nearLeft = c0 <= c1;
             nodeAddr = nearLeft ? lIdx : rIdx;
@@ -518,61 +296,21 @@ __device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd
         // the primitives of a leaf, one after the other
         bool descend = false;
         while (nodeAddr >= numInternal && primCount > 0) {
-            if (kBatch > 1 && (kSingle || inObj)) {
-                // Triangles in batches of kBatch: every load of the batch is
-                // issued before the first test, so a long leaf costs one memory
-                // latency per batch instead of one per triangle. The tests and
-                // hit updates still run in leaf order (the result and the counts
-                // are those of testing one at a time).
-                const int nb = primCount < kBatch ? primCount : kBatch;
-                const int first = nodeAddr - numInternal + primOffset;
-                float4 ta[kBatch], tb[kBatch], tc[kBatch];
-#pragma unroll
-                for (int j = 0; j < kBatch; ++j) {
-                    if (j < nb) {
-                        const size_t id = (size_t)(first + j);
-                        ta[j] = gload(tris + 3 * id);
-                        tb[j] = gload(tris + 3 * id + 1);
-                        tc[j] = gload(tris + 3 * id + 2);
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < kBatch; ++j) {
-                    if (j >= nb || done) continue;
-                    float t, w0, w1;
-                    const int prim = __float_as_int(ta[j].w);
-                    if (kStats) ++primTests;
-                    if (prim_hit<kMixed>(cur, ta[j], tb[j], tc[j], first + j,
-                                 [&] { return p.lods[p.instLod[kSingle ? 0 : curInst]].quadV3; }, t, w0, w1) &&
-                        better(t, curInst, prim, hitT, hInst, hPrim)) {
-                        hitT = t;
-                        hInst = curInst;
-                        hPrim = prim;
-                        hw0 = w0;
-                        hw1 = w1;
-                        if (kAny) done = true;
-                    }
-                }
-                primOffset += nb;
-                primCount -= nb;
-                if (done) break;
-                continue;
-            }
             const int leafId = nodeAddr - numInternal + primOffset;
             ++primOffset;
             --primCount;
-            if (!kSingle && !inObj) {
+            if (!single && !inObj) {
                 // an instance of the top level: enter its object
                 const int inst = p.tlasPrimIds[leafId];
                 DevLod lod;
                 const ObjectEntry e = enter_object(p, inst, wo, wd, hitT, lod);
-                if (kStats) ++nodeVisits;
+                if (kCount) ++nodeVisits;
                 if (!e.hit) continue;
                 if (lod.numPrims == 1) {
                     // single-primitive object: test it and return to the instance level
                     const float4 a = lod.triVerts[0], b = lod.triVerts[1], c = lod.triVerts[2];
                     float t, w0, w1;
-                    if (kStats) ++primTests;
+                    if (kCount) ++primTests;
                     const float objT = e.tmax;
                     float ht = objT;
                     if (prim_hit<kMixed>(e.ray, a, b, c, 0, [&] { return lod.quadV3; }, t, w0, w1) &&
@@ -589,12 +327,11 @@ __device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd
                     continue;
                 }
                 if (primCount > 0) {
-                    MFH_PUSH(primCount);
-                    MFH_PUSH(nodeAddr + primOffset);
+                    push(primCount);
+                    push(nodeAddr + primOffset);
                 }
-                MFH_PUSH(kSentinel);
+                push(kSentinel);
                 cur = e.ray;
-                finite = slab_finite(cur, lod.coordMax);
                 scale = e.scale;
                 hitT = e.tmax;
                 bvh = (const BvhChild*)lod.nodes;
@@ -609,13 +346,12 @@ __device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd
                 descend = true;
                 break;
             }
-            // one triangle at a time (kBatch == 1)
             const float4 a = gload(tris + 3 * (size_t)leafId), b = gload(tris + 3 * (size_t)leafId + 1),
                          c = gload(tris + 3 * (size_t)leafId + 2);
             float t, w0, w1;
             const int prim = __float_as_int(a.w);
-            if (kStats) ++primTests;
-            if (prim_hit<kMixed>(cur, a, b, c, leafId, [&] { return p.lods[p.instLod[kSingle ? 0 : curInst]].quadV3; },
+            if (kCount) ++primTests;
+            if (prim_hit<kMixed>(cur, a, b, c, leafId, [&] { return p.lods[p.instLod[curInst]].quadV3; },
                                  t, w0, w1) &&
                 better(t, curInst, prim, hitT, hInst, hPrim)) {
                 hitT = t;
@@ -633,23 +369,20 @@ __device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd
         if (descend) continue;
         // pop the next subtree (or return from an object to the instance level)
         if (sp == 0) break;
-        nodeAddr = MFH_POP();
-        if (!kSingle && nodeAddr == kSentinel) {
+        nodeAddr = pop();
+        if (!single && nodeAddr == kSentinel) {
             if (sp == 0) break;
             cur = make_fast_ray(wo, wd);
-            finite = slab_finite(cur, p.tlasCoordMax);
             hitT /= scale;
             scale = 1.0f;
             bvh = (const BvhChild*)p.tlasNodes;
             numInternal = p.tlasNumInternal;
             inObj = false;
-            nodeAddr = MFH_POP();
+            nodeAddr = pop();
         }
-        primCount = (nodeAddr >= numInternal) ? MFH_POP() : 2;
+        primCount = (nodeAddr >= numInternal) ? pop() : 2;
         primOffset = 0;
     }
-#undef MFH_PUSH
-#undef MFH_POP
     if (!kAny && inObj) hitT /= scale;  // object_to_world_space
     TraceHit h;
     h.t = hitT;
@@ -663,66 +396,256 @@ __device__ __forceinline__ TraceHit trace_ray(const TraceParams& p, V3 wo, V3 wd
     return h;
 }
 
-// Closest hit of a single-instance scene with postponed leaves (Aila and
-// Laine 2009, "speculative while-while"): a lane that reaches a leaf keeps it
-// and goes on descending through inner nodes until it reaches a second leaf
-// or half of the active lanes of its wave hold one; then the held leaves are
-// tested (kBatch triangles loaded at a time, as in trace_ray). Node steps and
-// leaf tests of a wave thus run with more lanes active. (1M-triangle
-// benchmark, test when: every lane holds 976, 7/8 994, 3/4 1041, 5/8 1086,
-// 1/2 1122, 3/8 1106, 1/4 1073 Mrays/s. On the two-level terrain, holding
-// inside objects was slower, so two-level scenes keep trace_ray.)
-// The visiting order differs from trace_ray's, which does not change the
-// result: inside one object the closest hit is the lexicographic minimum of
-// (t, primitive) over every triangle whose box path passes the slab tests,
-// and a box is culled only when its entry distance exceeds the current best
-// (the collapse enlarges boxes, so a triangle never lies closer than its
-// box's entry). No counts (the stats kernels use trace_ray).
-template <int kStride, int kLds = kLdsDepth, int kBatch = 1, bool kMixed = false>
-__device__ __forceinline__ TraceHit trace_closest_held(const TraceParams& p, V3 wo, V3 wd, float tmax,
-                                                       int* const lstack) {
-    int spill[kStackCap - kLds];
-    int sp = 0;
-    bool overflow = false;
-    auto push = [&](int v) {
+// The call takes the scene's pointers one by one: a reference would make the
+// kernels keep their argument block in private memory.
+template <bool kAny, bool kCount, bool kMixed>
+__device__ __forceinline__ TraceHit reference_ray(const TraceParams& p, V3 wo, V3 wd, float tmax) {
+    return reference_call<kAny, kCount, kMixed>(p.numInstances, p.worldToInst, p.instLod, p.lods, p.tlasNodes,
+                                                p.tlasPrimIds, p.tlasNumInternal, wo, wd, tmax);
+}
+
+// A ray in an object's space for the wide nodes: the margin (in distance along
+// the ray, per axis) covers the rounding of a quantized plane's distance and
+// of the full-precision slab test it stands for, each below 2^-23 (|origin| +
+// |coordinate|) / |direction|.
+struct WideRay {
+    V3 o, inv, eps;
+};
+__device__ __forceinline__ WideRay make_wide_ray(const FastRay& r, float coordMax) {
+    WideRay w;
+    w.o = r.o;
+    w.inv = r.inv;
+    w.eps = v3((fabsf(r.o.x) + coordMax) * fabsf(r.inv.x) * 0x1p-21f,
+               (fabsf(r.o.y) + coordMax) * fabsf(r.inv.y) * 0x1p-21f,
+               (fabsf(r.o.z) + coordMax) * fabsf(r.inv.z) * 0x1p-21f);
+    return w;
+}
+
+// Byte k of q as a float (v_cvt_f32_ubyte).
+template <int k>
+__device__ __forceinline__ float ubyte(u32 q) {
+    return (float)((q >> (8 * k)) & 0xFFu);
+}
+
+// One step through wide node `node`: the children that the ray may enter
+// before hitT as sort keys (entry distance with the child's number in the two
+// lowest bits, top bit set; 0: not entered) in descending order, so that the
+// entered children come first, the farthest leading.
+constexpr u32 kWideNone = 0xFFFFFFFFu;
+struct WideStep {
+    u32 key[4];
+    u32 child[4];
+    __device__ __forceinline__ u32 ref(u32 k) const {
+        const u32 lo = (k & 1u) ? child[1] : child[0], hi = (k & 1u) ? child[3] : child[2];
+        return (k & 2u) ? hi : lo;
+    }
+};
+template <int k>
+__device__ __forceinline__ u32 wide_key(u32 nx, u32 ny, u32 nz, u32 fx, u32 fy, u32 fz, V3 a, V3 bn, V3 bf,
+                                        float hitT) {
+    const float tn = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(__builtin_fmaf(ubyte<k>(nx), a.x, bn.x),
+                                                                     __builtin_fmaf(ubyte<k>(ny), a.y, bn.y)),
+                                                     __builtin_fmaf(ubyte<k>(nz), a.z, bn.z)),
+                                     0.0f);
+    const float tf = __builtin_fminf(__builtin_fminf(__builtin_fminf(__builtin_fmaf(ubyte<k>(fx), a.x, bf.x),
+                                                                     __builtin_fmaf(ubyte<k>(fy), a.y, bf.y)),
+                                                     __builtin_fmaf(ubyte<k>(fz), a.z, bf.z)),
+                                     hitT);
+    return tn <= tf ? ((__float_as_uint(tn) & 0x7FFFFFFCu) | (0x80000000u | (u32)k)) : 0u;
+}
+__device__ __forceinline__ WideStep wide_step(const float4* __restrict__ nodes, u32 node, const WideRay& w,
+                                              float hitT) {
+    const float4* nd = nodes + 4 * (size_t)node;
+    const float4 n0 = gload(nd), n1 = gload(nd + 1), n2 = gload(nd + 2), n3 = gload(nd + 3);
+    const V3 inv = w.inv;
+    const V3 a = v3(n0.w * inv.x, n1.x * inv.y, n1.y * inv.z);
+    const V3 off = v3(n0.x - w.o.x, n0.y - w.o.y, n0.z - w.o.z);
+    const V3 bn = v3(__builtin_fmaf(off.x, inv.x, -w.eps.x), __builtin_fmaf(off.y, inv.y, -w.eps.y),
+                     __builtin_fmaf(off.z, inv.z, -w.eps.z));
+    const V3 bf = v3(__builtin_fmaf(off.x, inv.x, w.eps.x), __builtin_fmaf(off.y, inv.y, w.eps.y),
+                     __builtin_fmaf(off.z, inv.z, w.eps.z));
+    const u32 lx = __float_as_uint(n1.z), ly = __float_as_uint(n1.w), lz = __float_as_uint(n2.x);
+    const u32 hx = __float_as_uint(n2.y), hy = __float_as_uint(n2.z), hz = __float_as_uint(n2.w);
+    const bool sx = inv.x < 0.0f, sy = inv.y < 0.0f, sz = inv.z < 0.0f;
+    const u32 nx = sx ? hx : lx, ny = sy ? hy : ly, nz = sz ? hz : lz;
+    const u32 fx = sx ? lx : hx, fy = sy ? ly : hy, fz = sz ? lz : hz;
+    WideStep r;
+    r.key[0] = wide_key<0>(nx, ny, nz, fx, fy, fz, a, bn, bf, hitT);
+    r.key[1] = wide_key<1>(nx, ny, nz, fx, fy, fz, a, bn, bf, hitT);
+    r.key[2] = wide_key<2>(nx, ny, nz, fx, fy, fz, a, bn, bf, hitT);
+    r.key[3] = wide_key<3>(nx, ny, nz, fx, fy, fz, a, bn, bf, hitT);
+    auto order = [&](int x, int y) {
+        const u32 hi = r.key[x] > r.key[y] ? r.key[x] : r.key[y], lo = r.key[x] > r.key[y] ? r.key[y] : r.key[x];
+        r.key[x] = hi;
+        r.key[y] = lo;
+    };
+    order(0, 1);
+    order(2, 3);
+    order(0, 2);
+    order(1, 3);
+    order(1, 2);
+    r.child[0] = __float_as_uint(n3.x);
+    r.child[1] = __float_as_uint(n3.y);
+    r.child[2] = __float_as_uint(n3.z);
+    r.child[3] = __float_as_uint(n3.w);
+    return r;
+}
+
+// Stack of a lane: its LDS column (stride kStride), deeper entries in the
+// private array `spill` of the caller.
+template <int kStride, int kLds>
+struct WideStack {
+    int* lds;
+    int sp;
+    bool overflow;  // a push found the stack full
+    __device__ __forceinline__ void push(int* spill, int v) {
         if (sp < kLds)
-            lds_at(lstack, sp * kStride) = v;
-        else if (sp < kStackCap)
+            lds_at(lds, sp * kStride) = v;
+        else if (sp < kWideCap)
             spill[sp - kLds] = v;
-        if (sp < kStackCap)
+        if (sp < kWideCap)
             ++sp;
         else
             overflow = true;
-    };
-    auto pop = [&]() {
-        --sp;
-        return sp < kLds ? lds_at(lstack, sp * kStride) : spill[sp - kLds];
-    };
-    TraceHit h;
-    h.inst = h.prim = -1;
-    h.w0 = h.w1 = 0.0f;
-    h.nodeVisits = h.primTests = 0;
-    DevLod lod;
-    const ObjectEntry e = enter_object(p, 0, wo, wd, tmax, lod);
-    if (!e.hit) {
-        h.t = tmax;
-        h.overflow = false;
-        return h;
     }
-    const FastRay cur = e.ray;
-    // every lane of the wave that traverses is active here: the choice holds for the whole traversal
-    const bool fast = __all(slab_finite(cur, lod.coordMax));
-    float hitT = e.tmax;
-    const BvhChild* const bvh = (const BvhChild*)lod.nodes;
-    const float4* const tris = lod.triVerts;
-    const int numInternal = lod.numInternal;
-    // current node (count 2 = inner node, n = leaf of n triangles, 0 = none)
-    int nodeAddr = 0, primCount = lod.numPrims == 1 ? 1 : 2;
-    int heldAddr = 0, heldCount = 0;  // the postponed leaf
-    while (true) {
+    __device__ __forceinline__ int pop(const int* spill) {
+        --sp;
+        int v = lds_at(lds, (sp < kLds ? sp : kLds - 1) * kStride);
+        if (sp >= kLds) v = spill[sp - kLds];
+        return v;
+    }
+    // The entered children of a step: the nearest is returned (kWideNone:
+    // none), the others go on the stack, the farthest first. The column takes
+    // three entries at once, entered or not (what lies above sp is free).
+    __device__ __forceinline__ u32 take(int* spill, const WideStep& r) {
+        const bool e0 = r.key[0] != 0u, e1 = r.key[1] != 0u, e2 = r.key[2] != 0u, e3 = r.key[3] != 0u;
+        const u32 c0 = r.ref(r.key[0]), c1 = r.ref(r.key[1]), c2 = r.ref(r.key[2]), c3 = r.ref(r.key[3]);
+        if (sp + 3 <= kLds) {
+            lds_at(lds, sp * kStride) = (int)c0;
+            lds_at(lds, (sp + 1) * kStride) = (int)c1;
+            lds_at(lds, (sp + 2) * kStride) = (int)c2;
+            sp += (e1 ? 1 : 0) + (e2 ? 1 : 0) + (e3 ? 1 : 0);
+        } else {
+            if (e1) push(spill, (int)c0);
+            if (e2) push(spill, (int)c1);
+            if (e3) push(spill, (int)c2);
+        }
+        return e3 ? c3 : (e2 ? c2 : (e1 ? c1 : (e0 ? c0 : kWideNone)));
+    }
+};
+
+// What the traversal of an object reads of its LoD.
+struct ObjectData {
+    const float4 *wide, *leafBoxes, *triVerts, *quadV3;
+};
+__device__ __forceinline__ ObjectData object_data(const DevLod& lod) {
+    return {lod.wide, lod.leafBoxes, lod.triVerts, lod.quadV3};
+}
+
+// The traversal of one ray, resumable: run() returns when the ray is done or
+// when fewer than `minActive` lanes of the wave are still under way, so that
+// the caller can hand new rays to the lanes that are done. kSingle: one
+// instance (else the instance level, or one instance found at run time).
+//
+// (1M-triangle mesh, 2.1M camera and 2.1M incoherent rays: 2.96 ms with a ray
+// per lane over binary nodes, 2.15 over wide nodes, 1.65 with the lanes handed
+// new rays: 22 -> 39 % of the lanes active. What bounds it now is instruction
+// issue, 70 % of the time, at that utilization.)
+//
+// A turn of run() takes the lanes between objects to their next one (over the
+// binary nodes of the instances, in the reference's order), and the lanes
+// inside one through node steps with postponed leaves (Aila and Laine 2009,
+// "speculative while-while"): a lane that reaches a leaf keeps it and goes on
+// descending until it reaches a second one or half of the active lanes hold
+// one; then the held leaves are tested, so node steps and leaf tests run with
+// more lanes active.
+template <bool kAny, bool kSingle, bool kMixed, int kStride, int kLds>
+struct Trav {
+    static constexpr int kSpill = kWideCap - kLds;
+    WideStack<kStride, kLds> st;
+    V3 wo, wd;         // the ray in world space (kSingle: unused)
+    V3 dir;            // in the entered object's space, with w
+    WideRay w;
+    float hitT, scale;
+    int hInst, hPrim;
+    float hw0, hw1;
+    ObjectData data;   // of the entered object (kSingle: see object())
+    int inst, base;    // the entered object, the stack height at its entry
+    int node, count, offset;  // instance level: node (count 2) or the rest of a leaf
+    u32 cur, held;     // node or leaf to do next, the postponed leaf
+    bool inObj, done, exact;  // exact: the ray is reference_ray's
+
+    __device__ __forceinline__ void enter(const ObjectEntry& e, const DevLod& lod, int instance) {
+        inst = instance;
+        hitT = e.tmax;
+        scale = e.scale;
+        if (!slab_finite(e.ray, lod.coordMax)) {
+            exact = done = true;
+            return;
+        }
+        w = make_wide_ray(e.ray, lod.coordMax);
+        dir = e.ray.d;
+        if (!kSingle) data = object_data(lod);
+        base = st.sp;
+        inObj = true;
+        cur = 0u;
+        held = kWideNone;
+    }
+    // An object of a single primitive: tested at once. The hit distance takes
+    // the way through the object's space and back as for any entered object.
+    __device__ __forceinline__ void single_prim(const ObjectEntry& e, const DevLod& lod, int instance) {
+        const float4 a = lod.triVerts[0], b = lod.triVerts[1], c = lod.triVerts[2];
+        float t, w0, w1, ht = e.tmax;
+        if (prim_hit<kMixed>(e.ray, a, b, c, 0, [&] { return lod.quadV3; }, t, w0, w1) &&
+            better(t, instance, __float_as_int(a.w), ht, hInst, hPrim)) {
+            ht = t;
+            hInst = instance;
+            hPrim = __float_as_int(a.w);
+            hw0 = w0;
+            hw1 = w1;
+        }
+        hitT = ht / e.scale;
+    }
+    __device__ __forceinline__ void init(const TraceParams& p, V3 o, V3 d, float maxT, int* lstack) {
+        st.lds = lstack;
+        st.sp = 0;
+        st.overflow = false;
+        if (!kSingle) {
+            wo = o;
+            wd = d;
+        }
+        hitT = maxT;
+        hInst = hPrim = -1;
+        hw0 = hw1 = 0.0f;
+        scale = 1.0f;
+        inObj = done = exact = false;
+        cur = held = kWideNone;
+        node = count = offset = 0;
+        base = 0;
+        if (kSingle || p.numInstances == 1) {
+            DevLod lod;
+            const ObjectEntry e = enter_object(p, 0, o, d, maxT, lod);
+            done = true;
+            if (!e.hit) return;
+            if (lod.numPrims == 1) {
+                single_prim(e, lod, 0);
+                return;
+            }
+            done = false;
+            enter(e, lod, 0);
+        } else {
+            count = 2;
+        }
+    }
+    // Instance level: to the next object, or done.
+    __device__ __forceinline__ void next_object(const TraceParams& p, int* spill) {
+        const BvhChild* const tlas = (const BvhChild*)p.tlasNodes;
+        const int tlasInternal = p.tlasNumInternal;
+        const FastRay world = make_fast_ray(wo, wd);
+        const bool finite = slab_finite(world, p.tlasCoordMax);
         while (true) {
-            if (primCount > 0 && nodeAddr < numInternal) {
-                const float4* nd = reinterpret_cast<const float4*>(bvh + 2 * (size_t)nodeAddr);
+            while (node < tlasInternal && count > 0) {
+                const float4* nd = reinterpret_cast<const float4*>(tlas + 2 * (size_t)node);
                 const float4 q0 = gload(nd), q1 = gload(nd + 1), q2 = gload(nd + 2), q3 = gload(nd + 3);
                 const float lLo[3] = {q0.x, q0.y, q0.z}, lHi[3] = {q0.w, q1.x, q1.y};
                 const float rLo[3] = {q2.x, q2.y, q2.z}, rHi[3] = {q2.w, q3.x, q3.y};
@@ -730,70 +653,156 @@ __device__ __forceinline__ TraceHit trace_closest_held(const TraceParams& p, V3 
                 const int rIdx = __float_as_int(q3.z), rCnt = __float_as_int(q3.w);
                 float c0, c1;
                 bool t0, t1;
-                slab_pair(fast, lLo, lHi, rLo, rHi, cur, hitT, t0, t1, c0, c1);
+                slab_pair(__all(finite), lLo, lHi, rLo, rHi, world, hitT, t0, t1, c0, c1);
                 if (!t0) c0 = 1e38f;
                 if (!t1) c1 = 1e38f;
                 if (t0 && t1) {
                     const bool farLeft = c1 < c0;
                     const int far = farLeft ? lIdx : rIdx;
-                    if (far >= numInternal) push(farLeft ? lCnt : rCnt);
-                    push(far);
+                    if (far >= tlasInternal) st.push(spill, farLeft ? lCnt : rCnt);
+                    st.push(spill, far);
                 }
                 const bool nearLeft = c0 <= c1;
-                nodeAddr = nearLeft ? lIdx : rIdx;
-                primCount = (!t0 && !t1) ? 0 : (nodeAddr >= numInternal ? (nearLeft ? lCnt : rCnt) : 2);
-                if (overflow) break;
+                node = nearLeft ? lIdx : rIdx;
+                count = (!t0 && !t1) ? 0 : (node >= tlasInternal ? (nearLeft ? lCnt : rCnt) : 2);
+                offset = 0;
             }
-            if (primCount > 0 && nodeAddr >= numInternal) {
-                if (heldCount > 0) break;  // a second leaf: test the held one first
-                heldAddr = nodeAddr;
-                heldCount = primCount;
-                primCount = 0;
-            }
-            if (primCount == 0) {
-                if (sp == 0) break;
-                nodeAddr = pop();
-                primCount = nodeAddr >= numInternal ? pop() : 2;
-            }
-            // half of the active lanes hold a leaf: test them together
-            if (2 * __popcll(__ballot(heldCount > 0)) >= __popcll(__builtin_amdgcn_read_exec())) break;
-        }
-        if (overflow) break;
-        for (int k = 0; k < heldCount; k += kBatch) {
-            const int nb = heldCount - k < kBatch ? heldCount - k : kBatch;
-            const int first = heldAddr - numInternal + k;
-            float4 ta[kBatch], tb[kBatch], tc[kBatch];
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j) {
-                if (j < nb) {
-                    const size_t id = (size_t)(first + j);
-                    ta[j] = gload(tris + 3 * id);
-                    tb[j] = gload(tris + 3 * id + 1);
-                    tc[j] = gload(tris + 3 * id + 2);
+            while (count > 0 && !inObj && !done) {
+                const int instance = p.tlasPrimIds[node - tlasInternal + offset];
+                ++offset;
+                --count;
+                DevLod lod;
+                const ObjectEntry e = enter_object(p, instance, wo, wd, hitT, lod);
+                if (!e.hit) continue;
+                if (lod.numPrims == 1) {
+                    single_prim(e, lod, instance);
+                    if (kAny && hInst != -1) done = true;
+                } else {
+                    enter(e, lod, instance);
                 }
             }
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j) {
-                if (j >= nb) continue;
-                float t, w0, w1;
-                const int prim = __float_as_int(ta[j].w);
-                if (prim_hit<kMixed>(cur, ta[j], tb[j], tc[j], first + j, [&] { return lod.quadV3; }, t, w0, w1) &&
-                    better(t, 0, prim, hitT, h.inst, h.prim)) {
-                    hitT = t;
-                    h.inst = 0;
-                    h.prim = prim;
-                    h.w0 = w0;
-                    h.w1 = w1;
-                }
+            if (st.overflow) exact = done = true;
+            if (inObj || done) return;
+            if (st.sp == 0) {
+                done = true;
+                return;
             }
+            node = st.pop(spill);
+            count = node >= tlasInternal ? st.pop(spill) : 2;
+            offset = 0;
         }
-        heldCount = 0;
-        if (primCount == 0 && sp == 0) break;
     }
-    h.t = hitT / e.scale;  // object_to_world_space
-    h.overflow = overflow;
-    return h;
-}
+    // The primitives of the held leaf: its box, then its records, the next one
+    // loaded while one is tested.
+    __device__ __forceinline__ void test_leaf(const ObjectData& od) {
+        const u32 first = held & ~kWideLeaf;
+        held = kWideNone;
+        const float4* bx = od.leafBoxes + 2 * (size_t)first;
+        const float4 b0 = gload(bx), b1 = gload(bx + 1);
+        const float4* rec = od.triVerts + 3 * (size_t)first;
+        float4 a = gload(rec), b = gload(rec + 1), c = gload(rec + 2);
+        const float lo[3] = {b0.x, b0.y, b0.z}, hi[3] = {b0.w, b1.x, b1.y};
+        const FastRay r{w.o, dir, w.inv, w.o * w.inv};
+        float entry;
+        if (!slab_fast(lo, hi, r, hitT, entry)) return;
+        const int n = __float_as_int(b1.z);
+        for (int k = 0;;) {
+            float4 na = a, nb = b, nc = c;
+            if (k + 1 < n) {
+                rec += 3;
+                na = gload(rec);
+                nb = gload(rec + 1);
+                nc = gload(rec + 2);
+            }
+            float t, w0, w1;
+            const int prim = __float_as_int(a.w);
+            if (prim_hit<kMixed>(r, a, b, c, (int)first + k, [&] { return od.quadV3; }, t, w0, w1) &&
+                better(t, inst, prim, hitT, hInst, hPrim)) {
+                hitT = t;
+                hInst = inst;
+                hPrim = prim;
+                hw0 = w0;
+                hw1 = w1;
+                if (kAny) {
+                    done = true;
+                    return;
+                }
+            }
+            if (++k >= n) return;
+            a = na;
+            b = nb;
+            c = nc;
+        }
+    }
+    // The data of the entered object; with one instance the same for every
+    // lane, so that it stays in scalar registers.
+    __device__ __forceinline__ ObjectData object(const TraceParams& p) const {
+        if constexpr (kSingle) return object_data(p.lods[p.instLod[0]]);
+        return data;
+    }
+    __device__ __forceinline__ void run(const TraceParams& p, int* spill, int minActive) {
+        ObjectData one;
+        if (kSingle) one = object(p);
+        while (!done) {
+            const ObjectData& od = kSingle ? one : data;
+            if (!kSingle) {
+                // the instance level, once a quarter of the lanes is there
+                const u64 between = __ballot(!inObj), active = __builtin_amdgcn_read_exec();
+                if (4 * __popcll(between) >= __popcll(active) && !inObj) next_object(p, spill);
+            }
+            if (kSingle || (inObj && !done)) {
+                while (true) {
+                    if (!(cur & kWideLeaf)) cur = st.take(spill, wide_step(od.wide, cur, w, hitT));
+                    if ((cur & kWideLeaf) && cur != kWideNone) {
+                        if (held != kWideNone) break;  // a second leaf: test the held one first
+                        held = cur;
+                        cur = kWideNone;
+                    }
+                    if (cur == kWideNone) {
+                        if (st.sp == base) break;
+                        cur = (u32)st.pop(spill);
+                    }
+                    if (2 * __popcll(__ballot(held != kWideNone)) >= __popcll(__builtin_amdgcn_read_exec())) break;
+                }
+                if (st.overflow) {
+                    exact = done = true;
+                } else {
+                    if (held != kWideNone) test_leaf(od);
+                    if (cur == kWideNone && st.sp == base && !done) {  // the object is through
+                        hitT /= scale;
+                        scale = 1.0f;
+                        inObj = false;
+                        if (kSingle) {
+                            done = true;
+                        } else if (count == 0) {
+                            if (st.sp == 0)
+                                done = true;
+                            else {
+                                node = st.pop(spill);
+                                count = node >= p.tlasNumInternal ? st.pop(spill) : 2;
+                                offset = 0;
+                            }
+                        }
+                    }
+                }
+            }
+            if (__popcll(__ballot(!done)) < minActive) break;
+        }
+    }
+    // The hit of a ray that is done (o, d, maxT: as given to init).
+    __device__ __forceinline__ TraceHit result(const TraceParams& p, V3 o, V3 d, float maxT) const {
+        if (__builtin_expect(exact, 0)) return reference_ray<kAny, false, kMixed>(p, o, d, maxT);
+        TraceHit h;
+        h.t = hitT;
+        h.inst = hInst;
+        h.prim = hPrim;
+        h.w0 = hw0;
+        h.w1 = hw1;
+        h.overflow = false;
+        h.nodeVisits = h.primTests = 0;
+        return h;
+    }
+};
 
 // Traversal specializations of the kernels that trace (their kMode): fixed
 // for one scene, or chosen per ray (a batch of scenes mixes single- and
@@ -807,27 +816,121 @@ constexpr int kTraceMixed = 3;   // per ray, LoDs with quads and spheres
 inline int trace_mode_of(const TraceParams& p) {
     return p.mixed ? kTraceMixed : (p.numInstances == 1 ? kTraceSingle : kTraceMulti);
 }
-// Traversal kind of the resumable Traversal for a mode.
-template <int kMode>
-constexpr int traversal_mode() {
-    return kMode == kTraceSingle ? 1 : (kMode == kTraceMulti ? 0 : 2);
+// Lanes of each wave that take entries of a queue of n: all 64, or where that
+// would leave more than three quarters of the `waves` resident waves without
+// any, half as many until it does not (at least 8). A wave with fewer rays
+// waits less for its longest, and more waves hide one another's memory latency. (Closest + any hit
+// of 12,765 rays through 924 instances: 457 us with 64 lanes, 204 with 8.)
+__host__ __device__ __forceinline__ int queue_lanes(int n, int waves) {
+    int lanes = 64;
+    while (lanes > 8 && n / lanes < waves / 4) lanes /= 2;
+    return lanes;
 }
 
-// Closest (kAny = false) or any hit in mode kMode; closest hits of
-// single-instance scenes hold leaves (trace_closest_held) unless kHeld is
-// false.
-template <int kMode, bool kAny, int kStride, int kLds, int kLeaf, bool kHeld = true>
-__device__ __forceinline__ TraceHit trace_mode(const TraceParams& tp, V3 o, V3 d, float tmax, int* lstack) {
-    constexpr bool kMixed = kMode == kTraceMixed;
-    if constexpr (kMode == kTraceSingle && !kAny && kHeld)
-        return trace_closest_held<kStride, kLds, kLeaf>(tp, o, d, tmax, lstack);
-    if constexpr (kMode == kTraceSingle) return trace_ray<kAny, false, true, kStride, kLds, kLeaf>(tp, o, d, tmax, lstack);
-    if constexpr (kMode == kTraceMulti) return trace_ray<kAny, false, false, kStride, kLds, kLeaf>(tp, o, d, tmax, lstack);
-    if (tp.numInstances == 1) {
-        if constexpr (!kAny && kHeld) return trace_closest_held<kStride, kLds, kLeaf, kMixed>(tp, o, d, tmax, lstack);
-        return trace_ray<kAny, false, true, kStride, kLds, kLeaf, kMixed>(tp, o, d, tmax, lstack);
+// A wave's part of a queue of `n` entries, taken by its first `lanes` lanes: a
+// chunk of `chunk` entries by wave index, later chunks from *counter (which
+// starts at 0) once every wave has its first. Queues of fewer than four chunks
+// a wave are dealt out in turn instead: every wave asks the counter once more
+// than it gets, and thousands of atomics on one address take longer than such
+// a queue's work may (341,000 rays through a sparse mesh of 3343 triangles: 52 us with the
+// counter, 27 dealt out). Entries go to the lanes in order.
+struct WaveQueue {
+    int n, lanes, chunk, at, end, first;
+    u32 base;  // of the current chunk (the counter may run past n)
+    int* counter;
+    bool more;  // further chunks may be left
+    __device__ __forceinline__ WaveQueue(int n_, int lanes_, int maxChunk, int wave, int waves, int* counter_)
+        : n(n_), lanes(lanes_), counter(counter_) {
+        const bool deal = n < 4 * 64 * waves;
+        chunk = deal ? lanes : maxChunk;
+        if (deal) counter = nullptr;
+        first = waves * chunk;
+        start((u32)(wave * chunk));
+        more = counter ? first < n : base + (u32)first < (u32)n;
     }
-    return trace_ray<kAny, false, false, kStride, kLds, kLeaf, kMixed>(tp, o, d, tmax, lstack);
+    __device__ __forceinline__ void start(u32 b) {
+        base = b;
+        at = b < (u32)n ? (int)b : n;
+        end = min(chunk, n - at) + at;
+    }
+    __device__ __forceinline__ bool left() const { return at < end || more; }
+    // The lanes that may take entries, of those with `idle` set.
+    __device__ __forceinline__ u64 takers(bool idle) const { return __ballot(idle && (int)__lane_id() < lanes); }
+    // Entries for the lanes of `mask`, -1 where there is none.
+    __device__ __forceinline__ int take(u64 mask) {
+        if (at >= end && more) {
+            if (counter) {
+                const int leader = __ffsll((long long)mask) - 1;
+                int got = 0;
+                if ((int)__lane_id() == leader) got = atomicAdd(counter, chunk);
+                start((u32)__shfl(got, leader) + (u32)first);
+                more = base + (u32)chunk < (u32)n;
+            } else {
+                start(base + (u32)first);
+                more = base + (u32)first < (u32)n;
+            }
+        }
+        const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+        const int e = at + rank;
+        const bool mine = ((mask >> __lane_id()) & 1ull) && e < end;
+        at = min(at + __popcll(mask), end);
+        return mine ? e : -1;
+    }
+};
+
+// Traces the rays of a wave's queue: load(entry, o, d, tmax) yields an entry's
+// ray (false: nothing to trace), store(entry, hit) takes its hit. Rays end
+// after very different numbers of steps, so a lane whose ray has ended takes
+// the next one as soon as fewer than 5/8 of the lanes are under way; a wave
+// that runs one ray per lane spends most of its steps on its few longest.
+template <class T, class Params, class Load, class Store>
+__device__ __forceinline__ void trace_queue(WaveQueue& q, int* lstack, Params params, Load load, Store store) {
+    T t;
+    int spill[T::kSpill];
+    t.done = true;
+    int entry = -1;
+    while (true) {
+        const u64 idle = q.takers(entry < 0);
+        if (idle != 0ull && q.left()) {
+            const int e = q.take(idle);
+            V3 o, d;
+            float tmax;
+            if (e >= 0 && load(e, o, d, tmax)) {
+                entry = e;
+                t.init(params(e), o, d, tmax, lstack);
+            }
+        }
+        if (__ballot(entry >= 0) == 0ull) {
+            if (!q.left()) break;
+            continue;
+        }
+        if (entry >= 0) {
+            t.run(params(entry), spill, q.left() ? q.lanes * 5 / 8 : 0);
+            if (t.done) {
+                V3 o = v3(0.0f, 0.0f, 0.0f), d = o;
+                float tmax = 0.0f;
+                if (__builtin_expect(t.exact, 0)) load(entry, o, d, tmax);
+                store(entry, t.result(params(entry), o, d, tmax));
+                entry = -1;
+            }
+        }
+    }
+}
+
+// The traversal of a kernel in mode kMode.
+template <int kMode, bool kAny, int kStride, int kLds>
+using ModeTrav = Trav<kAny, kMode == kTraceSingle, kMode == kTraceMixed, kStride, kLds>;
+
+// Closest (kAny = false) or any hit in mode kMode.
+template <int kMode, bool kAny, int kStride, int kLds>
+__device__ __forceinline__ TraceHit trace_mode(const TraceParams& tp, V3 o, V3 d, float tmax, int* lstack) {
+    using T = ModeTrav<kMode, kAny, kStride, kLds>;
+    T t;
+    int spill[T::kSpill];
+    t.init(tp, o, d, tmax, lstack);
+    t.run(tp, spill, 0);
+    return t.result(tp, o, d, tmax);
 }
 
 }  // namespace mfh
