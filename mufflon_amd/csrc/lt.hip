@@ -3,7 +3,10 @@
 // lt_common.hpp:17-78) over the scene, camera and positional lights of a
 // path tracer.
 //
-// One thread per light path; path i of an iteration draws from generator i
+// A lane owns a light path and runs its iterations one after the other, every
+// iteration of a call in one launch (path regeneration, as in the path
+// tracer's megakernel; each iteration splats into an image of its own); path i
+// of an iteration draws from generator i
 // (seeded like the path tracer's) and emits a photon from the light tree
 // with index i of numPixels (emit, light_tree_sampling.hpp:81-187: the index
 // spreads the photons over the tree's flux intervals), then walks the
@@ -26,7 +29,7 @@ namespace {
 using namespace shade;
 using namespace path;
 
-constexpr int kLtThreads = 256;
+constexpr int kLtThreads = 64;
 
 // Sampler result of a positional light (Emitter, light_sampling.hpp:21-52).
 struct LtEmitter {
@@ -171,134 +174,196 @@ __device__ __forceinline__ bool project(const PtScene& S, V3 dir, int& px, int& 
 // Splat image of one iteration: Radiance (3), Lightness, Density per pixel.
 constexpr int kLtChannels = 5;
 
-template <int kMode>
-__global__ __launch_bounds__(kLtThreads) void k_lt_iterate(PtScene S, float* __restrict__ splat, int minPathLength,
-                                                          int maxPathLength, int density) {
-    __shared__ int sStack[kLdsDepth * kLtThreads];
-    const int num = S.width * S.height;
-    const int idx = blockIdx.x * kLtThreads + (int)threadIdx.x;
-    if (idx >= num) return;
-    int* const lstack = sStack + threadIdx.x;
-    u64 rng = S.rngs[idx];
+// A connection of a vertex to the camera, splatted when nothing is between.
+struct LtSplat {
+    V3 a, dir;
+    float tmax;
+    V3 radiance;
+    float lightness, density;
+    int pixel;
+};
+
+// Connection of the vertex at vpos to the camera (get_connection,
+// path_util.hpp:384-399): false when it falls outside the image or carries
+// nothing. light: the path's emitter at pathLen 0, vx its vertex after.
+__device__ __forceinline__ bool connect_camera(const PtScene& S, V3 vpos, bool atLight, const LtEmitter& light,
+                                               const Vertex& vx, V3 throughput, int density, LtSplat& c) {
     const V3 camPos = v3(S.camPos[0], S.camPos[1], S.camPos[2]);
-    V3 throughput = v3(1.0f, 1.0f, 1.0f);
-    const u64 xStart = pcg_next(rng);
-    const u64 treeSeed = pcg_next(rng);
-    const LtEmitter light =
-        emit(S, (u64)idx, (u64)num, treeSeed, sample_uniform((u32)xStart), sample_uniform((u32)(xStart >> 32)));
-    pcg_next(rng);  // create_camera's RndSet2, unused by the pinhole
-    Vertex vx;
-    int pathLen = 0;
-    do {
-        if (pathLen + 1 >= minPathLength && pathLen + 1 <= maxPathLength) {
-            // get_connection(camera, vertex) (path_util.hpp:384-399)
-            const V3 vpos = pathLen == 0 ? light.position : vx.position;
-            const V3 conn = vpos - camPos;
-            const float distSq = dot(conn, conn);
-            const float dist = fsqrt(distSq);
-            const float dden = dist + 1e-20f * (dist < 0.0f ? -1.0f : 1.0f);
-            const V3 dir = conn / dden;
-            int px, py;
-            float w;
-            if (project(S, dir, px, py, w)) {
-                V3 lval;
-                float lcos;
-                V3 geoN;
-                float geomFactor;
-                if (pathLen == 0) {
-                    if (light.area) {  // evaluate_area (lights.hpp:286-295)
-                        const float c = dot(light.normal, neg(dir));
-                        lval = c <= 0.0f ? v3(0, 0, 0) : light.intensity;
-                        lcos = c <= 0.0f ? 0.0f : c;
-                        geoN = light.normal;
-                        geomFactor = dot(dir, light.normal);
-                    } else {  // evaluate_point (lights.hpp:262-265)
-                        lval = light.intensity;
-                        lcos = 1.0f;
-                        geoN = v3(0, 0, 0);
-                        geomFactor = 0.0f;
-                    }
-                } else {
-                    lval = mat_evaluate_adjoint(vx.ts, vx.mat, vx.incident(), neg(dir), lcos);
-                    geoN = vx.ts.geoN;
-                    geomFactor = dot(dir, vx.ts.shadingN);
-                }
-                V3 bxdfProd = v3(w * lval.x, w * lval.y, w * lval.z);
-                const float cosProd = 1.0f * lcos;
-                if (density || ((bxdfProd.x > 0.0f || bxdfProd.y > 0.0f || bxdfProd.z > 0.0f) && cosProd > 0.0f)) {
-                    // any_intersection (intersection.cu:624-637); the camera has no normal
-                    const V3 a = add_epsilon(camPos, dir, v3(0, 0, 0));
-                    const V3 b = add_epsilon(vpos, neg(dir), geoN);
-                    const V3 d = b - a;
-                    const float tmax = len(d);
-                    const TraceHit sh =
-                        trace_mode<kMode, true, kLtThreads, kLdsDepth>(S.trace, a, d / tmax, tmax, lstack);
-                    if (sh.inst == -1) {
-                        bxdfProd = bxdfProd / distSq;
-                        const V3 rad = throughput * cosProd * bxdfProd;
-                        float* o = splat + (size_t)kLtChannels * ((size_t)px + (size_t)py * S.width);
-                        atomicAdd(o, rad.x);
-                        atomicAdd(o + 1, rad.y);
-                        atomicAdd(o + 2, rad.z);
-                        atomicAdd(o + 3, (throughput.x + throughput.y + throughput.z) / 3.0f * cosProd);
-                        if (density) atomicAdd(o + 4, w * 1.0f / distSq * fabsf(geomFactor));
-                    }
-                }
-            }
+    const V3 conn = vpos - camPos;
+    const float distSq = dot(conn, conn);
+    const float dist = fsqrt(distSq);
+    const float dden = dist + 1e-20f * (dist < 0.0f ? -1.0f : 1.0f);
+    const V3 dir = conn / dden;
+    int px, py;
+    float w;
+    if (!project(S, dir, px, py, w)) return false;
+    V3 lval;
+    float lcos;
+    V3 geoN;
+    float geomFactor;
+    if (atLight) {
+        if (light.area) {  // evaluate_area (lights.hpp:286-295)
+            const float k = dot(light.normal, neg(dir));
+            lval = k <= 0.0f ? v3(0, 0, 0) : light.intensity;
+            lcos = k <= 0.0f ? 0.0f : k;
+            geoN = light.normal;
+            geomFactor = dot(dir, light.normal);
+        } else {  // evaluate_point (lights.hpp:262-265)
+            lval = light.intensity;
+            lcos = 1.0f;
+            geoN = v3(0, 0, 0);
+            geomFactor = 0.0f;
         }
-        // walk (random_walk.hpp:38-112), adjoint
-        const u64 x0 = pcg_next(rng);
-        const u64 x1 = pcg_next(rng);
-        const float rndRoulette = sample_uniform((u32)pcg_next(rng));
-        V3 rayOrigin, dirOut, sThroughput, absorption, geoOut;
-        if (pathLen == 0) {
-            // the light's direction (sample_light_dir_point / _area,
-            // light_sampling.hpp:85-89, 201-211)
-            const float u0 = sample_uniform((u32)x0), u1 = sample_uniform((u32)(x0 >> 32));
-            if (light.area) {
-                const float cosT = fsqrt(u0);
-                const float sinT = fsqrt(1.0f - u0);
-                const float phi = u1 * 2 * kPi;
-                const SinCos sc = fsincos(phi);
-                const float lx = sinT * sc.s, ly = sinT * sc.c;
-                const V3 tx = normalize(perpendicular(light.normal));
-                const V3 ty = cross(light.normal, tx);
-                dirOut = smul(lx, tx) + smul(ly, ty) + smul(cosT, light.normal);
-                sThroughput = light.intensity * kPi;
-                geoOut = light.normal;
+    } else {
+        lval = mat_evaluate_adjoint(vx.ts, vx.mat, vx.incident(), neg(dir), lcos);
+        geoN = vx.ts.geoN;
+        geomFactor = dot(dir, vx.ts.shadingN);
+    }
+    V3 bxdfProd = v3(w * lval.x, w * lval.y, w * lval.z);
+    const float cosProd = 1.0f * lcos;
+    if (!(density || ((bxdfProd.x > 0.0f || bxdfProd.y > 0.0f || bxdfProd.z > 0.0f) && cosProd > 0.0f))) return false;
+    // any_intersection (intersection.cu:624-637); the camera has no normal
+    c.a = add_epsilon(camPos, dir, v3(0, 0, 0));
+    const V3 b = add_epsilon(vpos, neg(dir), geoN);
+    const V3 d = b - c.a;
+    c.tmax = len(d);
+    c.dir = d / c.tmax;
+    bxdfProd = bxdfProd / distSq;
+    c.radiance = throughput * cosProd * bxdfProd;
+    c.lightness = (throughput.x + throughput.y + throughput.z) / 3.0f * cosProd;
+    c.density = w * 1.0f / distSq * fabsf(geomFactor);
+    c.pixel = px + py * S.width;
+    return true;
+}
+
+// A turn of the loop is one path segment: the emission, or a closest hit and
+// its vertex; then the connection to the camera and the walk to the next
+// segment. The connection's shadow ray is traced after the walk, when the
+// vertex is no longer live. Against one path per lane and a launch per
+// iteration: Cornell box 256x256, 16 iterations 13.9 -> 13.0 ms, 64x87, one
+// iteration 1.13 -> 0.87 ms. The splats' atomics are not what bounds it (12.7
+// ms without them): it is the traversal's chain, as in the megakernel.
+template <int kMode>
+__global__ __launch_bounds__(kLtThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_lt_iterate(
+    PtScene S, PathWork W, float* __restrict__ splat, int minPathLength, int maxPathLength, int density) {
+    __shared__ int sStack[kLdsDepth * kLtThreads];
+    int* const lstack = sStack + threadIdx.x;
+    const int num = S.width * S.height;
+    SlotQueue slots(W);
+    bool busy = false;
+    int idx = 0, done = 0, pathLen = -1;  // -1: the light emits next
+    u64 rng = 0;
+    V3 throughput = v3(1.0f, 1.0f, 1.0f), rayOrigin = throughput, dir = throughput, absorption = throughput;
+    while (true) {
+        const int slot = slots.take(W, busy);
+        if (slot >= 0) {
+            busy = true;
+            idx = slot;
+            done = 0;
+            pathLen = -1;
+            rng = S.rngs[idx];
+        }
+        if (__ballot(busy) == 0ull && !slots.more) break;
+        if (busy) {
+            bool ended = false, shadow = false;
+            LtEmitter light;
+            Vertex vx;
+            LtSplat c;
+            if (pathLen < 0) {
+                throughput = v3(1.0f, 1.0f, 1.0f);
+                const u64 xStart = pcg_next(rng);
+                const u64 treeSeed = pcg_next(rng);
+                light = emit(S, (u64)idx, (u64)num, treeSeed, sample_uniform((u32)xStart),
+                             sample_uniform((u32)(xStart >> 32)));
+                pcg_next(rng);  // create_camera's RndSet2, unused by the pinhole
             } else {
-                const float cosT = u0 * 2.0f - 1.0f;
-                const float sinT = fsqrt((1.0f - cosT) * (1.0f + cosT));
-                const float phi = u1 * 2.0f * kPi;
-                const SinCos sc = fsincos(phi);
-                dirOut = v3(sinT * sc.s, sinT * sc.c, cosT);
-                sThroughput = light.intensity * 4 * kPi;
-                geoOut = v3(0, 0, 0);
+                const TraceHit hit =
+                    trace_mode<kMode, false, kLtThreads, kLdsDepth>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
+                throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
+                ended = hit.inst == -1;
+                if (!ended)
+                    make_vertex(S, rayOrigin, dir, 0.0f, hit.t, hit.inst, hit.prim, hit.w0, hit.w1, vx);
             }
-            rayOrigin = light.position;
-            absorption = light.absorption;
-        } else {
-            float pdfF;
-            if (!mat_sample(vx.ts, vx.mat, vx.incident(), sample_uniform((u32)x0), sample_uniform((u32)(x0 >> 32)),
-                            x1, sThroughput, dirOut, pdfF, true))
-                break;
-            absorption = vx.mat.medium(dot(dirOut, vx.ts.geoN)).absorption;
-            rayOrigin = vx.position;
-            geoOut = vx.ts.geoN;
+            if (!ended) {
+                ++pathLen;
+                ended = pathLen > 0 && pathLen >= maxPathLength;
+            }
+            if (!ended) {
+                const bool atLight = pathLen == 0;
+                if (pathLen + 1 >= minPathLength && pathLen + 1 <= maxPathLength)
+                    shadow = connect_camera(S, atLight ? light.position : vx.position, atLight, light, vx, throughput,
+                                            density, c);
+                // walk (random_walk.hpp:38-112), adjoint
+                const u64 x0 = pcg_next(rng);
+                const u64 x1 = pcg_next(rng);
+                const float rndRoulette = sample_uniform((u32)pcg_next(rng));
+                V3 origin, sThroughput, geoOut;
+                if (atLight) {
+                    // the light's direction (sample_light_dir_point / _area,
+                    // light_sampling.hpp:85-89, 201-211)
+                    const float u0 = sample_uniform((u32)x0), u1 = sample_uniform((u32)(x0 >> 32));
+                    if (light.area) {
+                        const float cosT = fsqrt(u0);
+                        const float sinT = fsqrt(1.0f - u0);
+                        const float phi = u1 * 2 * kPi;
+                        const SinCos sc = fsincos(phi);
+                        const float lx = sinT * sc.s, ly = sinT * sc.c;
+                        const V3 tx = normalize(perpendicular(light.normal));
+                        const V3 ty = cross(light.normal, tx);
+                        dir = smul(lx, tx) + smul(ly, ty) + smul(cosT, light.normal);
+                        sThroughput = light.intensity * kPi;
+                        geoOut = light.normal;
+                    } else {
+                        const float cosT = u0 * 2.0f - 1.0f;
+                        const float sinT = fsqrt((1.0f - cosT) * (1.0f + cosT));
+                        const float phi = u1 * 2.0f * kPi;
+                        const SinCos sc = fsincos(phi);
+                        dir = v3(sinT * sc.s, sinT * sc.c, cosT);
+                        sThroughput = light.intensity * 4 * kPi;
+                        geoOut = v3(0, 0, 0);
+                    }
+                    origin = light.position;
+                    absorption = light.absorption;
+                } else {
+                    float pdfF;
+                    V3 out;
+                    ended = !mat_sample(vx.ts, vx.mat, vx.incident(), sample_uniform((u32)x0),
+                                        sample_uniform((u32)(x0 >> 32)), x1, sThroughput, out, pdfF, true);
+                    if (!ended) {
+                        dir = out;
+                        absorption = vx.mat.medium(dot(dir, vx.ts.geoN)).absorption;
+                        origin = vx.position;
+                        geoOut = vx.ts.geoN;
+                    }
+                }
+                if (!ended) {
+                    throughput = throughput * sThroughput;
+                    const float cont = mn(mx(mx(throughput.x, throughput.y), throughput.z) + 0.1f, 1.0f);
+                    ended = rndRoulette >= cont;
+                    if (!ended) {
+                        throughput = throughput / cont;
+                        rayOrigin = add_epsilon(origin, dir, geoOut);
+                    }
+                }
+            }
+            if (shadow &&
+                trace_mode<kMode, true, kLtThreads, kLdsDepth>(S.trace, c.a, c.dir, c.tmax, lstack).inst == -1) {
+                float* o = splat + (size_t)kLtChannels * ((size_t)num * done + c.pixel);
+                atomicAdd(o, c.radiance.x);
+                atomicAdd(o + 1, c.radiance.y);
+                atomicAdd(o + 2, c.radiance.z);
+                atomicAdd(o + 3, c.lightness);
+                if (density) atomicAdd(o + 4, c.density);
+            }
+            if (ended) {
+                pathLen = -1;
+                if (++done == W.iterations) {
+                    S.rngs[idx] = rng;
+                    busy = false;
+                }
+            }
         }
-        throughput = throughput * sThroughput;
-        const float cont = mn(mx(mx(throughput.x, throughput.y), throughput.z) + 0.1f, 1.0f);
-        if (rndRoulette >= cont) break;
-        throughput = throughput / cont;
-        rayOrigin = add_epsilon(rayOrigin, dirOut, geoOut);
-        const TraceHit hit = trace_mode<kMode, false, kLtThreads, kLdsDepth>(S.trace, rayOrigin, dirOut,
-                                                                                 kMaxSceneSize, lstack);
-        throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
-        if (hit.inst == -1) break;
-        make_vertex(S, rayOrigin, dirOut, 0.0f, hit.t, hit.inst, hit.prim, hit.w0, hit.w1, vx);
-        ++pathLen;
-    } while (pathLen < maxPathLength);
-    S.rngs[idx] = rng;
+    }
 }
 
 __global__ void k_lt_clear(float* p, size_t n) {
@@ -306,40 +371,44 @@ __global__ void k_lt_clear(float* p, size_t n) {
     if (i < n) p[i] = 0.0f;
 }
 
-// Running mean (and variance) of the splat image (UpdateIter,
-// output_handler_variance.hpp:7-31).
+// Running mean (and variance) of the splat images of `iterations` iterations
+// from index `first` on (UpdateIter, output_handler_variance.hpp:7-31).
 __global__ void k_lt_accumulate(const float* __restrict__ splat, float* __restrict__ mean, float* __restrict__ var,
-                                size_t n, int iteration) {
+                                size_t n, int first, int iterations) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float denom = mx(1.0f, (float)iteration + 1);
-    const float iter = splat[i];
-    const float diff = iter - mean[i];
-    const float cum = mean[i] + diff / denom;
-    mean[i] = cum;
-    if (var) var[i] += (diff * (iter - cum) - var[i]) / mx(1.0f, (float)iteration);
+    float m = mean[i], v = var ? var[i] : 0.0f;
+    for (int k = 0; k < iterations; ++k) {
+        const int iteration = first + k;
+        const float iter = splat[n * k + i];
+        const float diff = iter - m;
+        m = m + diff / mx(1.0f, (float)iteration + 1);
+        v += (diff * (iter - m) - v) / mx(1.0f, (float)iteration);
+    }
+    mean[i] = m;
+    if (var) var[i] = v;
 }
 
 }  // namespace
 
-void launch_lighttracer(const PtScene& S, float* splat, float* mean, float* var, int minPathLength,
-                        int maxPathLength, bool density, hipStream_t stream) {
+void launch_lighttracer(const PtScene& S, int iterations, float* splat, float* mean, float* var, int minPathLength,
+                        int maxPathLength, bool density, LaunchQueue& queue, int numCUs, hipStream_t stream) {
     const size_t n = (size_t)kLtChannels * S.width * S.height;
-    const int clearBlocks = (int)((n + 255) / 256);
-    hipLaunchKernelGGL(k_lt_clear, dim3(clearBlocks), dim3(256), 0, stream, splat, n);
-    const int blocks = (S.width * S.height + kLtThreads - 1) / kLtThreads;
+    const size_t all = n * iterations;
+    hipLaunchKernelGGL(k_lt_clear, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, stream, splat, all);
     const int mode = trace_mode_of(S.trace);
-#define MFH_LT(M)                                                                                              \
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_lt_iterate<M>), dim3(blocks), dim3(kLtThreads), 0, stream, S, splat, \
-                       minPathLength, maxPathLength, density ? 1 : 0)
-    if (mode == kTraceSingle)
-        MFH_LT(kTraceSingle);
-    else if (mode == kTraceMixed)
-        MFH_LT(kTraceMixed);
-    else
-        MFH_LT(kTraceMulti);
-#undef MFH_LT
-    hipLaunchKernelGGL(k_lt_accumulate, dim3(clearBlocks), dim3(256), 0, stream, splat, mean, var, n, S.iteration);
+    auto* const fn = mode == kTraceSingle  ? k_lt_iterate<kTraceSingle>
+                     : mode == kTraceMixed ? k_lt_iterate<kTraceMixed>
+                                           : k_lt_iterate<kTraceMulti>;
+    PathWork W;
+    const int grid =
+        path_work(reinterpret_cast<const void*>(fn), S.width * S.height, iterations, queue, numCUs, W);
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(kLtThreads), 0, stream, S, W, splat, minPathLength, maxPathLength,
+                       density ? 1 : 0);
+    MFH_HIP(hipGetLastError());
+    queue.next ^= 1;
+    hipLaunchKernelGGL(k_lt_accumulate, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, splat, mean, var, n,
+                       S.iteration, iterations);
     MFH_HIP(hipGetLastError());
 }
 

@@ -29,11 +29,6 @@ using namespace path;
 
 constexpr int kPtTile = 8;  // a wave starts on an 8x8 pixel tile
 constexpr int kPtThreads = kPtTile * kPtTile;
-// Fewest lanes of a wave that take pixels (Cornell box 256x256, 64 / 32 / 16
-// lanes: 14.1 / 12.7 / 10.6 ms; 200x151 room, 64 / 32 / 16 / 8: 0.72 / 0.63 /
-// 0.57 / 0.55 ms; the terrain image, which fills the chip, 24.5 / 34.4 / 47.5).
-constexpr int kPtMinLanes = 8;
-
 // Path regeneration. Paths end after very different numbers of segments (2.5
 // of 8 on average in the Cornell box), and a wave that runs one path per lane
 // works until its longest has ended, a launch per iteration until the longest
@@ -58,19 +53,16 @@ constexpr int kPtMinLanes = 8;
 // kNeeOne: at most one next-event estimate a vertex (several are traced one
 // after the other, before the walk).
 template <int kMode, bool kNeeOne>
-__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_pt_iterate(PtScene S,
-                                                                                                  PtWork W) {
+__global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_pt_iterate(PtScene S, PathWork W,
+                                                                                                  int tilesX) {
     __shared__ int sStack[kLdsDepth * kPtThreads];
     int* const lstack = sStack + threadIdx.x;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *W.nextQueue = 0;
     auto any_hit = [&](const NeeCandidate& c) {
         return trace_mode<kMode, true, kPtThreads, kLdsDepth>(S.trace, c.a, c.dir, c.tmax, lstack).inst != -1;
     };
-    const int lane = (int)threadIdx.x;
-    const int first = (int)gridDim.x * W.lanes;  // slots below are assigned by block index
-    bool start = true, more = first < W.slots;   // more: the queue may hold further slots
-    bool busy = false;                           // the lane owns a pixel
-    int px = 0, py = 0, done = 0;                // its position, its finished iterations
+    SlotQueue slots(W);
+    bool busy = false;             // the lane owns a pixel
+    int px = 0, py = 0, done = 0;  // its position, its finished iterations
     int pathLen = 0;
     u64 rng = 0;
     Acc acc;
@@ -80,38 +72,19 @@ __global__ __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(3)))
     V3 throughput = v3(1.0f, 1.0f, 1.0f), rayOrigin = throughput, dir = throughput, absorption = throughput;
     V3 prevPos = throughput;
     while (true) {
-        const unsigned long long idle = __ballot(!busy && lane < W.lanes);
-        if (idle != 0ull) {
-            int slot = -1;
-            if (start) {
-                if (lane < W.lanes) slot = (int)blockIdx.x * W.lanes + lane;
-            } else if (more && 4 * __popcll(idle) >= W.lanes) {
-                const int want = __popcll(idle), leader = __ffsll((long long)idle) - 1;
-                int base = 0;
-                if (lane == leader) base = atomicAdd(W.queue, want);
-                base = __shfl(base, leader) + first;
-                more = base + want < W.slots;
-                if (!busy && lane < W.lanes)
-                    slot = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(idle >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)idle, 0u));
-            }
-            start = false;
-            if (slot >= 0 && slot < W.slots) {
-                const int tile = slot / kPtThreads, in = slot % kPtThreads;
-                px = (tile % W.tilesX) * kPtTile + in % kPtTile;
-                py = (tile / W.tilesX) * kPtTile + in / kPtTile;
-                if (px < S.width && py < S.height) {
-                    busy = true;
-                    done = 0;
-                    pathLen = 0;
-                    rng = S.rngs[(size_t)px + (size_t)py * S.width];
-                }
-            }
-            if (__ballot(busy) == 0ull) {
-                if (!more) break;
-                continue;  // every lane took a slot outside the image
+        const int slot = slots.take(W, busy);
+        if (slot >= 0) {
+            const int tile = slot / kPtThreads, in = slot % kPtThreads;
+            px = (tile % tilesX) * kPtTile + in % kPtTile;
+            py = (tile / tilesX) * kPtTile + in / kPtTile;
+            if (px < S.width && py < S.height) {
+                busy = true;
+                done = 0;
+                pathLen = 0;
+                rng = S.rngs[(size_t)px + (size_t)py * S.width];
             }
         }
+        if (__ballot(busy) == 0ull && !slots.more) break;
         if (busy) {
             if (pathLen == 0) {  // the camera's sample
                 acc.init(S.targetMask);
@@ -191,9 +164,31 @@ void launch_pt_init_rng(u64* rngs, int num, int seed, hipStream_t stream) {
     MFH_HIP(hipGetLastError());
 }
 
+// Fewest lanes of a wave that take pixels (Cornell box 256x256, 64 / 32 / 16
+// lanes: 14.1 / 12.7 / 10.6 ms; 200x151 room, 64 / 32 / 16 / 8: 0.72 / 0.63 /
+// 0.57 / 0.55 ms; the terrain image, which fills the chip, 24.5 / 34.4 / 47.5).
+constexpr int kMinLanes = 8;
+
+int path_work(const void* fn, int slots, int iterations, LaunchQueue& queue, int numCUs, PathWork& W) {
+    int blocksPerCU = 0;
+    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocksPerCU, fn, 64, 0));
+    // Lanes of a wave that take slots: all 64, or for launches too small to
+    // give every resident wave 64 slots, half as many until they do. More
+    // waves of fewer paths each hide one another's memory latency, and the
+    // segment of a wave waits for the longest of fewer rays.
+    const int resident = std::max(blocksPerCU, 1) * numCUs;
+    W.iterations = iterations;
+    W.slots = slots;
+    W.lanes = 64;
+    while (W.lanes > kMinLanes && slots / W.lanes < resident) W.lanes /= 2;
+    W.queue = queue.counters + queue.next;
+    W.nextQueue = queue.counters + (queue.next ^ 1);
+    return std::min((slots + W.lanes - 1) / W.lanes, resident);
+}
+
 namespace {
 
-using IterateFn = void (*)(PtScene, PtWork);
+using IterateFn = void (*)(PtScene, PathWork, int);
 
 template <int kMode>
 IterateFn iterate_kernel(bool neeOne) {
@@ -208,24 +203,11 @@ void launch_pt_iterate(const PtScene& S, int iterations, LaunchQueue& queue, int
     const IterateFn fn = mode == kTraceSingle  ? iterate_kernel<kTraceSingle>(neeOne)
                          : mode == kTraceMulti ? iterate_kernel<kTraceMulti>(neeOne)
                                                : iterate_kernel<kTraceMixed>(neeOne);
-    int blocksPerCU = 0;
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocksPerCU, fn, kPtThreads, 0));
-    PtWork W;
-    W.tilesX = (S.width + kPtTile - 1) / kPtTile;
-    const int tiles = W.tilesX * ((S.height + kPtTile - 1) / kPtTile);
-    W.slots = tiles * kPtThreads;
-    W.iterations = iterations;
-    W.queue = queue.counters + queue.next;
-    W.nextQueue = queue.counters + (queue.next ^ 1);
-    // Lanes of a wave that take pixels: all 64, or for images too small to
-    // give every wave slot of the chip 64 pixels, half as many until they do.
-    // More waves of fewer pixels each hide one another's memory latency, and
-    // the segment of a wave waits for the longest of fewer rays.
-    const int resident = std::max(blocksPerCU, 1) * numCUs;
-    W.lanes = kPtThreads;
-    while (W.lanes > kPtMinLanes && W.slots / W.lanes < resident) W.lanes /= 2;
-    const int grid = std::min(W.slots / W.lanes, resident);
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(kPtThreads), 0, stream, S, W);
+    const int tilesX = (S.width + kPtTile - 1) / kPtTile;
+    const int tiles = tilesX * ((S.height + kPtTile - 1) / kPtTile);
+    PathWork W;
+    const int grid = path_work(reinterpret_cast<const void*>(fn), tiles * kPtThreads, iterations, queue, numCUs, W);
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(kPtThreads), 0, stream, S, W, tilesX);
     MFH_HIP(hipGetLastError());
     queue.next ^= 1;
 }

@@ -15,6 +15,7 @@ struct AdjointState {
     int fixedDecisions;    // 0: derivative of the expected image; 1: of this realization (MFH_ADJOINT_*)
 };
 
-void launch_pt_adjoint(const PtScene& S, const AdjointState& A, int seed, hipStream_t stream);
+void launch_pt_adjoint(const PtScene& S, const AdjointState& A, int seed, LaunchQueue& queue, int numCUs,
+                       hipStream_t stream);
 
 }  // namespace mfh

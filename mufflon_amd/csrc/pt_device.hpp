@@ -124,26 +124,28 @@ struct PtScene {
 };
 
 void launch_pt_init_rng(uint64_t* rngs, int num, int seed, hipStream_t stream);
-// Work of one launch: `iterations` iterations of the pixels in 8x8 tile order
-// (`slots` = tiles * 64, `tilesX` tiles a row), taken by the first `lanes`
-// lanes of each wave. Blocks start on the slots of their index, later slots
-// come from *queue; *nextQueue is the queue of the next launch.
-struct PtWork {
-    int32_t iterations, slots, tilesX, lanes;
+// Work of a path-regenerating kernel: `slots` paths (or pixels) of
+// `iterations` iterations each, taken by the first `lanes` lanes of each wave.
+// Blocks of one wave start on the slots of their index, later slots come from
+// *queue; *nextQueue is the queue of the next launch, which the kernel clears.
+struct PathWork {
+    int32_t iterations, slots, lanes;
     int* queue;
     int* nextQueue;
 };
+// Fills W for a launch of kernel fn and returns its grid.
+int path_work(const void* fn, int slots, int iterations, LaunchQueue& queue, int numCUs, PathWork& W);
 // `iterations` iterations from index S.iteration on.
 void launch_pt_iterate(const PtScene& S, int iterations, LaunchQueue& queue, int numCUs, hipStream_t stream);
 // One iteration of the wireframe renderer into S.cum[MFH_TARGET_RADIANCE]
 // (and S.var[...] when recorded), S.iteration the iteration index.
 void launch_wireframe(const PtScene& S, const uint32_t* seeds, float lineWidth, int maxTraceDepth,
                       hipStream_t stream);
-// One iteration of the light tracer: clears the 5-channel splat image
-// (Radiance, Lightness, Density per pixel), traces width * height light
-// paths from S.rngs and folds the splats into mean (and var when non-null)
-// as iteration S.iteration.
-void launch_lighttracer(const PtScene& S, float* splat, float* mean, float* var, int minPathLength,
-                        int maxPathLength, bool density, hipStream_t stream);
+// `iterations` iterations of the light tracer from index S.iteration on: clears
+// their 5-channel splat images (Radiance, Lightness, Density per pixel; one
+// image after the other in `splat`), traces width * height light paths an
+// iteration from S.rngs and folds the splats into mean (and var when non-null).
+void launch_lighttracer(const PtScene& S, int iterations, float* splat, float* mean, float* var, int minPathLength,
+                        int maxPathLength, bool density, LaunchQueue& queue, int numCUs, hipStream_t stream);
 
 }  // namespace mfh

@@ -744,6 +744,7 @@ int mfh_pt_wireframe_get(mfh_context* ctx, int32_t ptId, int32_t variance, float
 
 namespace {
 constexpr int kLtChannels = 5;
+constexpr int64_t kLtSplatBytes = 64 << 20;  // of the splat images of one launch
 void lighttracer_reset(Context& c, PathTracer& t, bool recordVariance) {
     const size_t num = (size_t)t.camera.width * t.camera.height;
     t.ltIteration = -1;
@@ -756,7 +757,6 @@ void lighttracer_reset(Context& c, PathTracer& t, bool recordVariance) {
     } else {
         t.ltVar.release();
     }
-    t.ltSplat.reserve(4 * kLtChannels * num);
     // GpuLightTracer::post_reset (gpu_lt.cpp:31-36): generator i seeded with
     // i + seed * (pixels + 1), as the path tracer's
     t.ltRngs.reserve(8 * num);
@@ -786,11 +786,17 @@ int mfh_pt_lighttracer_iterate(mfh_context* ctx, int32_t ptId, int32_t iteration
             lighttracer_reset(c, t, t.ltVariance);  // first use, or the resolution grew
         PtScene S = device_scene(c, t);
         S.rngs = t.ltRngs.as<uint64_t>();
-        for (int32_t it = 0; it < iterations; ++it) {
-            S.iteration = ++t.ltIteration;
-            launch_lighttracer(S, t.ltSplat.as<float>(), t.ltMean.as<float>(),
+        // as many iterations a launch as splat images fit the bound
+        const int perLaunch = (int)std::max<int64_t>(1, kLtSplatBytes / (4 * kLtChannels * (int64_t)num));
+        t.ltSplat.reserve(4 * kLtChannels * num * (size_t)std::min(perLaunch, std::max(iterations, 1)));
+        for (int32_t it = 0; it < iterations;) {
+            const int n = std::min(iterations - it, perLaunch);
+            S.iteration = t.ltIteration + 1;
+            launch_lighttracer(S, n, t.ltSplat.as<float>(), t.ltMean.as<float>(),
                                t.ltVariance ? t.ltVar.as<float>() : nullptr, t.params.minPathLength,
-                               t.params.maxPathLength, density != 0, c.stream);
+                               t.params.maxPathLength, density != 0, t.queue, c.numCUs, c.stream);
+            t.ltIteration += n;
+            it += n;
         }
         MFH_HIP(hipStreamSynchronize(c.stream));
     });
@@ -856,7 +862,7 @@ int mfh_pt_adjoint(mfh_context* ctx, int32_t ptId, int32_t iterations, const flo
         A.texGrad = t.adjTexGradPtrs.as<float* const>();
         A.emissionGrad = t.adjEmGrad.as<float>();
         A.fixedDecisions = t.adjMode == MFH_ADJOINT_FIXED_DECISIONS ? 1 : 0;
-        launch_pt_adjoint(S, A, t.params.seed * (num + 1), c.stream);
+        launch_pt_adjoint(S, A, t.params.seed * (num + 1), t.queue, c.numCUs, c.stream);
         t.adjValid = true;
     });
 }

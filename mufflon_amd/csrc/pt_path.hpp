@@ -407,5 +407,38 @@ __device__ __forceinline__ void accumulate(const PtScene& S, size_t pixel, int i
     }
 }
 
+// Slots of a path-regenerating kernel (PathWork, blocks of one wave).
+struct SlotQueue {
+    int lane, first;
+    bool start, more;  // the block's own slots come next; the queue may hold further ones
+    __device__ __forceinline__ explicit SlotQueue(const PathWork& W) {
+        lane = (int)threadIdx.x;
+        first = (int)gridDim.x * W.lanes;
+        start = true;
+        more = first < W.slots;
+        if (blockIdx.x == 0 && lane == 0) *W.nextQueue = 0;
+    }
+    // New slots for the lanes that are not busy, once a quarter of the lanes
+    // is free; -1 where there is none.
+    __device__ __forceinline__ int take(const PathWork& W, bool busy) {
+        const u64 idle = __ballot(!busy && lane < W.lanes);
+        int slot = -1;
+        if (start) {
+            if (lane < W.lanes) slot = (int)blockIdx.x * W.lanes + lane;
+            start = false;
+        } else if (more && 4 * __popcll(idle) >= W.lanes) {
+            const int want = __popcll(idle), leader = __ffsll((long long)idle) - 1;
+            int base = 0;
+            if (lane == leader) base = atomicAdd(W.queue, want);
+            base = __shfl(base, leader) + first;
+            more = base + want < W.slots;
+            if ((idle >> lane) & 1ull)
+                slot = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(idle >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((unsigned)idle, 0u));
+        }
+        return slot < W.slots ? slot : -1;
+    }
+};
+
 }  // namespace path
 }  // namespace mfh
