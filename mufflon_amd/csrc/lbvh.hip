@@ -16,6 +16,8 @@
 //   scan        inclusive sum of the keep marks          (build_lbvh.cu:748-758)
 //   k_collapse  64-byte-node BVH with enlarged boxes     (build_lbvh.cu:503-566)
 //   k_wide      4-wide quantized nodes for the traversal kernels (LoDs)
+// Up to kSmallBuild primitives k_small_hierarchy and k_small_collapse do the
+// same in one workgroup.
 //
 // Determinism. The refit merges a node in a fixed operand order whatever
 // thread arrives second: box = min/max(right, left) and
@@ -335,10 +337,9 @@ __device__ __forceinline__ int refit_level(int lo, int hi) {
     return level;
 }
 
-__global__ __launch_bounds__(kThreads) void k_karras(const u64* __restrict__ keys, int n, i32* __restrict__ parents,
-                                                    i32* __restrict__ children, uint8_t* __restrict__ levels) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n - 1) return;
+// Internal node idx of the hierarchy over n sorted keys.
+__device__ __forceinline__ void karras_node(const u64* keys, int n, int idx, i32* __restrict__ parents,
+                                            i32* __restrict__ children, uint8_t* __restrict__ levels) {
     const u64 k1 = keys[idx];
     const int l1 = lcp(keys, n, idx, idx + 1, k1);
     const int l2 = lcp(keys, n, idx, idx - 1, k1);
@@ -368,6 +369,12 @@ __global__ __launch_bounds__(kThreads) void k_karras(const u64* __restrict__ key
     children[2 * idx + 1] = right;
     levels[idx] = (uint8_t)refit_level(min(idx, j), max(idx, j));
     if (idx == 0) parents[0] = kTreeHead;
+}
+
+__global__ __launch_bounds__(kThreads) void k_karras(const u64* __restrict__ keys, int n, i32* __restrict__ parents,
+                                                    i32* __restrict__ children, uint8_t* __restrict__ levels) {
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx < n - 1) karras_node(keys, n, idx, parents, children, levels);
 }
 
 __device__ __forceinline__ int parent_of(const i32* parents, int node) {
@@ -733,13 +740,7 @@ __global__ __launch_bounds__(kLevelThreads) void k_refit_level(int n, int level,
 // traversal hierarchy: a node is also kept there when it holds more than
 // refineAbove primitives, so no traversal leaf is longer than that. Both mark
 // sets are closed under descendants (a removed node's subtree is removed).
-template <class C>
-__global__ __launch_bounds__(kThreads) void k_mark(int nInt, const i32* __restrict__ parents,
-                                                  const uint8_t* __restrict__ flags, i32* __restrict__ marks,
-                                                  const float4* __restrict__ boxes, int refineAbove,
-                                                  i32* __restrict__ marks2) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= nInt) return;
+__device__ __forceinline__ int keep_mark(int x, const i32* __restrict__ parents, const uint8_t* __restrict__ flags) {
     int keep = 1;
     int y = x;
     for (int depth = 0; y != 0 && depth < kMaxDepth; ++depth) {
@@ -751,6 +752,17 @@ __global__ __launch_bounds__(kThreads) void k_mark(int nInt, const i32* __restri
         }
         y = parent_of(parents, y);
     }
+    return keep;
+}
+
+template <class C>
+__global__ __launch_bounds__(kThreads) void k_mark(int nInt, const i32* __restrict__ parents,
+                                                  const uint8_t* __restrict__ flags, i32* __restrict__ marks,
+                                                  const float4* __restrict__ boxes, int refineAbove,
+                                                  i32* __restrict__ marks2) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= nInt) return;
+    const int keep = keep_mark(x, parents, flags);
     marks[x] = keep;
     if (marks2) marks2[x] = (keep || C::sum(__float_as_int(boxes[2 * (size_t)x].w)) > refineAbove) ? 1 : 0;
 }
@@ -770,12 +782,11 @@ __device__ __forceinline__ void enlarged_box(float4 a, float4 b, V3& bl, V3& bh)
 // The reference's collapsed BVH: each kept node and leaf writes its record
 // (enlarged box, index in the collapsed numbering) into its parent.
 template <class C>
-__global__ __launch_bounds__(kThreads) void k_collapse(int n, const i32* __restrict__ parents,
-                                                      const float4* __restrict__ boxes,
-                                                      const i32* __restrict__ offsets, BvhChild* __restrict__ out) {
-    const int node = blockIdx.x * blockDim.x + threadIdx.x + 1;
+__device__ __forceinline__ void collapse_node(int node, int n, const i32* __restrict__ parents,
+                                              const float4* __restrict__ boxes, const i32* offsets,
+                                              BvhChild* __restrict__ out) {
     const int nInt = n - 1;
-    if (node >= 2 * n - 1 || is_collapsed(offsets, nInt, node)) return;
+    if (is_collapsed(offsets, nInt, node)) return;
     const int nAfter = offsets[nInt - 1];
     int parent = parents[node];
     int off = parent < 0 ? 0 : 1;
@@ -804,6 +815,14 @@ __global__ __launch_bounds__(kThreads) void k_collapse(int n, const i32* __restr
     out[outIdx + off] = r;
 }
 
+template <class C>
+__global__ __launch_bounds__(kThreads) void k_collapse(int n, const i32* __restrict__ parents,
+                                                      const float4* __restrict__ boxes,
+                                                      const i32* __restrict__ offsets, BvhChild* __restrict__ out) {
+    const int node = blockIdx.x * blockDim.x + threadIdx.x + 1;
+    if (node < 2 * n - 1) collapse_node<C>(node, n, parents, boxes, offsets, out);
+}
+
 // ---- traversal hierarchy
 // One 64-byte node per kept binary node: up to four descendants of it (the
 // larger-surface inner child is opened twice), their boxes quantized to 8 bits
@@ -825,7 +844,7 @@ struct WideChild {
 // Child c of binary node `parent`'s side (left or right) under the keep scan.
 template <class C>
 __device__ __forceinline__ WideChild wide_child(int c, bool left, int nInt, const float4* __restrict__ boxes,
-                                                const i32* __restrict__ offsets, i32& count) {
+                                                const i32* offsets, i32& count) {
     const float4 a = boxes[2 * (size_t)c], b = boxes[2 * (size_t)c + 1];
     WideChild w;
     enlarged_box(a, b, w.lo, w.hi);
@@ -844,13 +863,11 @@ __device__ __forceinline__ WideChild wide_child(int c, bool left, int nInt, cons
 }
 
 template <class C>
-__global__ __launch_bounds__(kThreads) void k_wide(int n, const i32* __restrict__ children,
-                                                  const float4* __restrict__ boxes,
-                                                  const i32* __restrict__ offsets, float4* __restrict__ wide,
-                                                  float4* __restrict__ leafBoxes) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void wide_node(int x, int n, const i32* __restrict__ children,
+                                          const float4* __restrict__ boxes, const i32* offsets,
+                                          float4* __restrict__ wide, float4* __restrict__ leafBoxes) {
     const int nInt = n - 1;
-    if (x >= nInt || is_collapsed(offsets, nInt, x)) return;
+    if (is_collapsed(offsets, nInt, x)) return;
     WideChild ch[4];
     int used = 2;
 #pragma unroll
@@ -934,14 +951,149 @@ __global__ __launch_bounds__(kThreads) void k_wide(int n, const i32* __restrict_
                        __uint_as_float(used > 3 ? ch[3].ref : ch[0].ref));
 }
 
-// Zero fill and count hand-off of the build (kernels, not memsets, so that a
+template <class C>
+__global__ __launch_bounds__(kThreads) void k_wide(int n, const i32* __restrict__ children,
+                                                  const float4* __restrict__ boxes,
+                                                  const i32* __restrict__ offsets, float4* __restrict__ wide,
+                                                  float4* __restrict__ leafBoxes) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x < n - 1) wide_node<C>(x, n, children, boxes, offsets, wide, leafBoxes);
+}
+
+// ---- builds of 2 to kSmallBuild primitives
+// One workgroup holds such a build, so its stages need no launch each: the
+// first kernel takes it from the primitives to the hierarchy (Morton codes,
+// sort, Karras), the tile refit is one workgroup already, the last kernel does
+// the marks, their scan and both collapses. With a launch per stage and digit
+// pass, 24 launches were the whole time of a build: 2000 triangles without
+// allocation 228 us, this way 128 us. The line lies at one refit tile: a second
+// tile needs the level kernels, and twice the pairs a second workgroup.
+constexpr int kSmallBuild = kRefitTile;
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallIpt = kSmallBuild / kSmallThreads;
+static_assert(kSmallBuild == 2 * kSmallThreads, "one pair of the sort per thread");
+
+// Bitonic sort of (code, id) pairs in LDS: the ids are distinct, so the order
+// is that of the stable radix sort by code.
+template <class P>
+__global__ __launch_bounds__(kSmallThreads) void k_small_hierarchy(P set, int n, Box6 bb, float4* __restrict__ stage,
+                                                                  u64* __restrict__ unsorted,
+                                                                  u64* __restrict__ keys, i32* __restrict__ ids,
+                                                                  i32* __restrict__ parents,
+                                                                  i32* __restrict__ children,
+                                                                  uint8_t* __restrict__ levels) {
+    __shared__ u64 sKey[kSmallBuild];
+    __shared__ i32 sId[kSmallBuild];
+    int padded = 2;
+    while (padded < n) padded *= 2;
+    for (int i = threadIdx.x; i < padded; i += kSmallThreads) {
+        u64 key = ~0ull;  // past the primitives: last, by the id
+        if (i < n) {
+            V3 c;
+            if constexpr (P::kStaged)
+                c = stage ? set.centroid_staged(i, stage) : set.centroid(i);
+            else
+                c = set.centroid(i);
+            if (!set.masked(i)) key = morton_of_point(c, bb);
+            if (unsorted) unsorted[i] = key;
+        }
+        sKey[i] = key;
+        sId[i] = i;
+    }
+    // A wave's pairs of the steps up to 64 lie in 128 slots of its own, so those
+    // steps need no barrier between them.
+    bool others = true;
+    for (int k = 2; k <= padded; k *= 2) {
+        for (int j = k / 2; j > 0; j /= 2) {
+            if (others || j > 64)
+                __syncthreads();
+            else
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            others = j > 64;
+            const int t = threadIdx.x;
+            if (t < padded / 2) {
+                const int a = 2 * t - (t & (j - 1)), b = a + j;
+                const u64 ka = sKey[a], kb = sKey[b];
+                const i32 ia = sId[a], ib = sId[b];
+                const bool after = ka > kb || (ka == kb && ia > ib);
+                if (after == ((a & k) == 0)) {
+                    sKey[a] = kb;
+                    sKey[b] = ka;
+                    sId[a] = ib;
+                    sId[b] = ia;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += kSmallThreads) {
+        keys[i] = sKey[i];
+        ids[i] = sId[i];
+        if (i < n - 1) karras_node(sKey, n, i, parents, children, levels);
+    }
+}
+
+// Inclusive sum over the block of one value per thread.
+__device__ __forceinline__ int small_scan(int v, int* sWave) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(v, o, 64);
+        if (lane >= o) v += t;
+    }
+    if (lane == 63) sWave[wave] = v;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) v += sWave[w];
+    __syncthreads();
+    return v;
+}
+
+template <class C>
+__global__ __launch_bounds__(kSmallThreads) void k_small_collapse(int n, const i32* __restrict__ parents,
+                                                                 const i32* __restrict__ children,
+                                                                 const uint8_t* __restrict__ flags,
+                                                                 const float4* __restrict__ boxes, int refineAbove,
+                                                                 i32* __restrict__ offsets,
+                                                                 BvhChild* __restrict__ out,
+                                                                 float4* __restrict__ wide,
+                                                                 float4* __restrict__ leafBoxes) {
+    __shared__ i32 sOff[kSmallBuild], sOff2[kSmallBuild];
+    __shared__ int sWave[kSmallThreads / 64];
+    const int nInt = n - 1;
+    int keep[kSmallIpt], keep2[kSmallIpt];
+    int sum = 0, sum2 = 0;
+#pragma unroll
+    for (int r = 0; r < kSmallIpt; ++r) {
+        const int x = kSmallIpt * (int)threadIdx.x + r;
+        keep[r] = x < nInt ? keep_mark(x, parents, flags) : 0;
+        keep2[r] = keep[r];
+        if (x < nInt && refineAbove > 0 && C::sum(__float_as_int(boxes[2 * (size_t)x].w)) > refineAbove) keep2[r] = 1;
+        sum += keep[r];
+        sum2 += keep2[r];
+    }
+    int at = small_scan(sum, sWave) - sum, at2 = small_scan(sum2, sWave) - sum2;
+#pragma unroll
+    for (int r = 0; r < kSmallIpt; ++r) {
+        const int x = kSmallIpt * (int)threadIdx.x + r;
+        at += keep[r];
+        at2 += keep2[r];
+        sOff[x] = at;
+        sOff2[x] = at2;
+        if (x < nInt) offsets[x] = at;
+    }
+    __syncthreads();
+    for (int node = 1 + threadIdx.x; node < 2 * n - 1; node += kSmallThreads)
+        collapse_node<C>(node, n, parents, boxes, sOff, out);
+    if (wide)
+        for (int x = threadIdx.x; x < nInt; x += kSmallThreads)
+            wide_node<C>(x, n, children, boxes, sOff2, wide, leafBoxes);
+}
+
+// Zero fill of the build (a kernel, not a memset, so that a
 // build can sit in a captured stream).
 __global__ void k_fill_u32(u32* p, int n, u32 v) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
-}
-__global__ void k_num_internal(const i32* offsets, int n, i32* out) {
-    if (threadIdx.x == 0) *out = n > 1 ? offsets[n - 2] : 0;
 }
 // World box of each instance (feeds the scene box of the instance level).
 __global__ __launch_bounds__(kThreads) void k_inst_boxes(InstPrims set, int n, float* out) {
@@ -991,12 +1143,10 @@ struct WideOut {
 
 // Shared orchestration (build_lbvh.cu:586-780). Returns the number of
 // internal nodes after the collapse; primIds and nodes receive the result.
-// With dNumInternal the count goes to that device int instead and nothing
-// waits for the stream (the return value is then -1).
 template <class P, class C>
 int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const float* bbox, DevBuf& nodes,
-                  DevBuf& primIds, float4* triVerts, StageSink* sink, i32* dNumInternal = nullptr,
-                  const WideOut* wideOut = nullptr, float4* stage = nullptr) {
+                  DevBuf& primIds, float4* triVerts, StageSink* sink, const WideOut* wideOut = nullptr,
+                  float4* stage = nullptr) {
     hipStream_t st = ctx.stream;
     MFH_REQUIRE(n < kMaxPrims, "an LBVH build holds fewer than 2^29 primitives");
     s.keysA.reserve(8 * (size_t)n);
@@ -1017,25 +1167,33 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
 
     u64* keys = s.keysA.as<u64>();
     i32* ids = s.idsA.as<i32>();
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_morton<P>), dim3(blocks_for(n)), dim3(kThreads), 0, st, set, n, bb, keys,
-                       ids, stage);
-    MFH_HIP(hipGetLastError());
-    if (sink) d2h(st, sink->unsortedKeys, keys, n);
-    radix_sort_pairs(keys, s.keysB.as<u64>(), ids, s.idsB.as<i32>(), n, 0, 64, s, st);
-    if (sink) {
-        d2h(st, sink->sortedKeys, keys, n);
-        d2h(st, sink->sortedIds, ids, n);
-    }
     i32* parents = s.parents.as<i32>();
     i32* children = s.children.as<i32>();
     float4* boxes = s.boxes.as<float4>();
     uint8_t* levels = s.levels.as<uint8_t>();
     u32* straddle = s.straddle.as<u32>();
     u32* straddleCount = straddle + n;
-    fill_u32(straddleCount, 1, 0u, st);
-    if (n > 1)
-        hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, keys, n, parents, children,
-                           levels);
+    const bool small = n > 1 && n <= kSmallBuild;
+    if (small) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_small_hierarchy<P>), dim3(1), dim3(kSmallThreads), 0, st, set, n, bb,
+                           stage, sink ? s.keysB.as<u64>() : nullptr, keys, ids, parents, children, levels);
+        MFH_HIP(hipGetLastError());
+        if (sink) d2h(st, sink->unsortedKeys, s.keysB.ptr, n);
+    } else {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_morton<P>), dim3(blocks_for(n)), dim3(kThreads), 0, st, set, n, bb,
+                           keys, ids, stage);
+        MFH_HIP(hipGetLastError());
+        if (sink) d2h(st, sink->unsortedKeys, keys, n);
+        radix_sort_pairs(keys, s.keysB.as<u64>(), ids, s.idsB.as<i32>(), n, 0, 64, s, st);
+        fill_u32(straddleCount, 1, 0u, st);
+        if (n > 1)
+            hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, keys, n, parents, children,
+                               levels);
+    }
+    if (sink) {
+        d2h(st, sink->sortedKeys, keys, n);
+        d2h(st, sink->sortedIds, ids, n);
+    }
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_refit_tiles<P, C>), dim3((n + kRefitTile - 1) / kRefitTile),
                        dim3(kRefitThreads), 0, st, set, n, ids, parents, children, levels, boxes,
                        s.flags.as<uint8_t>(), triVerts, stage, primIds.as<i32>(), straddle, straddleCount);
@@ -1052,43 +1210,42 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
         MFH_HIP(hipGetLastError());
     }
     if (n == 1) {
-        if (dNumInternal) {
-            hipLaunchKernelGGL(k_num_internal, dim3(1), dim3(64), 0, st, nullptr, 1, dNumInternal);
-            MFH_HIP(hipGetLastError());
-            return -1;
-        }
         MFH_HIP(hipStreamSynchronize(st));
         return 0;
     }
     i32* offsets = s.offsets.as<i32>();
     const bool refining = wideOut && wideOut->refineAbove > 0;
     i32* offsets2 = nullptr;
-    if (refining) {
-        s.offsets2.reserve(4 * (size_t)(n - 1));
-        offsets2 = s.offsets2.as<i32>();
-    }
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mark<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n - 1, parents,
-                       s.flags.as<uint8_t>(), offsets, boxes, refining ? wideOut->refineAbove : 0, offsets2);
-    if (refining)
-        scan_inclusive_i32_pair(offsets, offsets2, n - 1, s, st);
-    else
-        scan_inclusive_i32(offsets, offsets, n - 1, s, st);
     nodes.reserve(64 * (size_t)(n - 1));
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_collapse<C>), dim3(blocks_for(2 * n - 2)), dim3(kThreads), 0, st, n,
-                       parents, boxes, offsets, nodes.as<BvhChild>());
     if (wideOut) {
         wideOut->nodes->reserve(64 * (size_t)(n - 1));
         wideOut->leafBoxes->reserve(32 * (size_t)n);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wide<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n, children,
-                           boxes, refining ? offsets2 : offsets, wideOut->nodes->as<float4>(),
-                           wideOut->leafBoxes->as<float4>());
+    }
+    if (small) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_small_collapse<C>), dim3(1), dim3(kSmallThreads), 0, st, n, parents,
+                           children, s.flags.as<uint8_t>(), boxes, refining ? wideOut->refineAbove : 0, offsets,
+                           nodes.as<BvhChild>(), wideOut ? wideOut->nodes->as<float4>() : nullptr,
+                           wideOut ? wideOut->leafBoxes->as<float4>() : nullptr);
+    } else {
+        if (refining) {
+            s.offsets2.reserve(4 * (size_t)(n - 1));
+            offsets2 = s.offsets2.as<i32>();
+        }
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mark<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n - 1, parents,
+                           s.flags.as<uint8_t>(), offsets, boxes, refining ? wideOut->refineAbove : 0, offsets2);
+        if (refining)
+            scan_inclusive_i32_pair(offsets, offsets2, n - 1, s, st);
+        else
+            scan_inclusive_i32(offsets, offsets, n - 1, s, st);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_collapse<C>), dim3(blocks_for(2 * n - 2)), dim3(kThreads), 0, st, n,
+                           parents, boxes, offsets, nodes.as<BvhChild>());
+        if (wideOut) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wide<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n, children,
+                               boxes, refining ? offsets2 : offsets, wideOut->nodes->as<float4>(),
+                               wideOut->leafBoxes->as<float4>());
+        }
     }
     MFH_HIP(hipGetLastError());
-    if (dNumInternal) {
-        hipLaunchKernelGGL(k_num_internal, dim3(1), dim3(64), 0, st, offsets, n, dNumInternal);
-        MFH_HIP(hipGetLastError());
-        return -1;
-    }
     i32 nAfter = 0;
     MFH_HIP(hipMemcpyAsync(&nAfter, offsets + (n - 2), sizeof(nAfter), hipMemcpyDeviceToHost, st));
     MFH_HIP(hipStreamSynchronize(st));
@@ -1113,14 +1270,13 @@ void build_lod_bvh(Context& ctx, Lod& lod, const float* bbox, StageSink* sink) {
         MixedPrims set{lod.verts.as<float>(), lod.tris.as<u32>(),  lod.quads.as<u32>(), lod.spheres.as<float4>(),
                        lod.numQuads > 0 ? lod.quadV3.as<float4>() : nullptr, lod.numTris, lod.numQuads};
         lod.numInternal = build_generic<MixedPrims, LodCost>(ctx, ctx.scratch, set, n, lod.box, lod.nodes,
-                                                             lod.primIds, lod.triVerts.as<float4>(), sink, nullptr,
-                                                             &wide);
+                                                             lod.primIds, lod.triVerts.as<float4>(), sink, &wide);
     } else {
         TriPrims set{lod.verts.as<float>(), lod.tris.as<u32>()};
         ctx.scratch.stage.reserve(48 * (size_t)n);
         lod.numInternal = build_generic<TriPrims, LodCost>(ctx, ctx.scratch, set, n, lod.box, lod.nodes,
-                                                           lod.primIds, lod.triVerts.as<float4>(), sink, nullptr,
-                                                           &wide, ctx.scratch.stage.as<float4>());
+                                                           lod.primIds, lod.triVerts.as<float4>(), sink, &wide,
+                                                           ctx.scratch.stage.as<float4>());
     }
     lod.built = true;
 }
