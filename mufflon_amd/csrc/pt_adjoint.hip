@@ -57,7 +57,7 @@ namespace {
 using namespace shade;
 using namespace path;
 
-constexpr int kAdjThreads = 64;
+constexpr int kAdjThreads = 128;
 
 struct AdjVertex {
     int tex;        // albedo texture of the vertex's material, -1 when it has no albedo parameter
@@ -76,24 +76,20 @@ struct AdjVertex {
     float rn[2];    // sum over next-event estimates: weighted contribution * d ln / d(rx, ry)
 };
 
-// Emission gradients of the first kEmissionSlots materials are summed in LDS
-// per wave and go to memory once, at its end: a scene has few emitters, and
-// every next-event estimate adds to one of them (1.2M atomic additions on three
-// addresses took 11.6 of the 14.9 ms of the kernel on the Cornell box,
-// 256x256, 4 iterations).
-constexpr int kEmissionSlots = 64;
-__device__ __forceinline__ void add_emission_grad(const PtScene& S, const AdjointState& A, float* sEmission, int mat,
-                                                  V3 weighted) {
+// Every next-event estimate adds to an emitter's three sums, and a scene has few
+// emitters, so the additions to one address, which run one after another, bound
+// the kernel. With a sum every kEmissionStride floats the three do not also wait
+// for each other in one line: Cornell box, 256x256, 4 iterations, image and
+// gradients 22.6 -> 10.3 ms. (Sums in LDS per wave reach 7.5 ms; they round
+// less, and move the emission gradient by the 3e-4 that the rounding of a
+// million additions to one float makes.)
+__device__ __forceinline__ void add_emission_grad(const PtScene& S, const AdjointState& A, int mat, V3 weighted) {
     const PtMaterialRecord& m = S.materials[mat];
     const float w[3] = {weighted.x, weighted.y, weighted.z};
 #pragma unroll
     for (int c = 0; c < 3; ++c)
-        if (m.scale[c] != 0.0f && w[c] != 0.0f) {
-            if (mat < kEmissionSlots)
-                atomicAdd(sEmission + 3 * mat + c, w[c] / m.scale[c]);
-            else
-                atomicAdd(A.emissionGrad + 3 * mat + c, w[c] / m.scale[c]);
-        }
+        if (m.scale[c] != 0.0f && w[c] != 0.0f)
+            atomicAdd(A.emissionGrad + (size_t)(3 * mat + c) * kEmissionStride, w[c] / m.scale[c]);
 }
 
 // Texel weights of a texture lookup, as tex_sample forms them.
@@ -125,69 +121,88 @@ __device__ __forceinline__ int texel_weights(const DevTexture& t, float u, float
     return 4;
 }
 
-// Path regeneration, as in the megakernel: a turn of the loop is one segment of
-// the replay (closest hit, vertex, next-event estimates, walk); a lane whose
-// path has ended runs its backward pass and starts the pixel's next iteration
-// in the next turn. (Cornell box 256x256, 4 iterations: 14.9 -> 3.6 ms with
-// the emission sums above in LDS.)
 template <int kMode>
-__global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_pt_adjoint(PtScene S,
-                                                                                                  AdjointState A,
-                                                                                                  PathWork W) {
+__global__ __launch_bounds__(kAdjThreads) void k_pt_adjoint(PtScene S, AdjointState A) {
     __shared__ int sStack[kLdsDepth * kAdjThreads];
-    __shared__ float sEmission[3 * kEmissionSlots];
-    for (int k = threadIdx.x; k < 3 * kEmissionSlots; k += kAdjThreads) sEmission[k] = 0.0f;
-    __syncthreads();
+    const int pixel = blockIdx.x * kAdjThreads + threadIdx.x;
+    if (pixel >= S.width * S.height) return;
+    const int px = pixel % S.width, py = pixel / S.width;
     int* const lstack = sStack + threadIdx.x;
+    const float* dl = A.delta + 3 * (size_t)pixel;
     const float inv = 1.0f / (float)A.iterations;
-    SlotQueue slots(W);
-    bool busy = false;
-    int px = 0, py = 0, done = 0, pathLen = 0;
-    u64 rng = 0;
-    V3 delta = v3(0.0f, 0.0f, 0.0f), throughput = delta, rayOrigin = delta, dir = delta, absorption = delta;
-    V3 prevPos = delta;
-    float footA = 0.0f, pdfF = 1.0f;
+    const V3 delta = v3(dl[0] * inv, dl[1] * inv, dl[2] * inv);
+    if (!nonzero(delta)) return;
+    u64 rng = A.rngs[pixel];
     AdjVertex rec[kAdjMaxVertices + 1];
-    while (true) {
-        const int slot = slots.take(W, busy);
-        if (slot >= 0) {
-            px = slot % S.width;
-            py = slot / S.width;
-            const float* dl = A.delta + 3 * (size_t)slot;
-            delta = v3(dl[0] * inv, dl[1] * inv, dl[2] * inv);
-            busy = nonzero(delta);  // a pixel without an adjoint needs no replay
-            done = 0;
-            pathLen = 0;
-            rng = A.rngs[slot];
-        }
-        if (__ballot(busy) == 0ull && !slots.more) break;
-        if (!busy) continue;
-        // ---- forward replay (the megakernel's segment)
-        if (pathLen == 0) {
-            footA = 0.0f;
-            throughput = v3(1.0f, 1.0f, 1.0f);
-            pcg_next(rng);
-            rec[0].neeW = rec[0].emW = v3(0, 0, 0);
-            rec[0].tex = rec[0].rtex = -1;
-            rec[0].cont = 1.0f;
-            rec[0].misC = 0.0f;
-            const u64 x0 = pcg_next(rng);
-            pcg_next(rng);
-            pcg_next(rng);
-            camera_ray(S, px, py, x0, dir, pdfF);
-            rayOrigin = v3(S.camPos[0], S.camPos[1], S.camPos[2]);
-            absorption = v3(0.0f, 0.0f, 0.0f);
-            prevPos = rayOrigin;
-        }
+    for (int it = 0; it < A.iterations; ++it) {
+        // ---- forward replay (the megakernel's pt_sample)
+        float guideWeight = 1.0f, footA = 0.0f;
+        V3 throughput = v3(1.0f, 1.0f, 1.0f);
         Vertex vx;
-        const TraceHit hit =
-            trace_mode<kMode, false, kAdjThreads, kLdsDepth>(S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
-        throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
-        footA += 1.0f / fsqrt(pdfF);
-        const float guideWeight = 1.f / (1.f + footA * footA / 1.0f);
-        make_vertex(S, rayOrigin, dir, pdfF, hit.t, hit.inst, hit.prim, hit.w0, hit.w1, vx);
-        ++pathLen;
-        {
+        pcg_next(rng);
+        int pathLen = 0;
+        rec[0].neeW = rec[0].emW = v3(0, 0, 0);
+        rec[0].tex = rec[0].rtex = -1;
+        rec[0].cont = 1.0f;
+        rec[0].misC = 0.0f;
+        do {
+            if (pathLen > 0 && pathLen + 1 >= S.minPathLength && pathLen + 1 <= S.maxPathLength) {
+                const u64 neeSeed = pcg_next(rng);
+                for (int i = 0; i < S.neeCount; ++i) {
+                    const u64 x = pcg_next(rng);
+                    NeeCandidate c;
+                    if (nee_candidate(S, vx, throughput, guideWeight, i, neeSeed, x, c)) {
+                        const TraceHit sh = trace_mode<kMode, true, kAdjThreads, kLdsDepth>(
+                            S.trace, c.a, c.dir, c.tmax, lstack);
+                        if (sh.inst == -1) {
+                            AdjVertex& r = rec[pathLen];
+                            const V3 wgt = delta * c.radiance;
+                            r.neeW = r.neeW + wgt;
+                            if (c.lightMaterial >= 0) add_emission_grad(S, A, c.lightMaterial, wgt);
+                            float dv[2], dp[2];
+                            if (r.rtex >= 0 && dln_mat_evaluate(vx.ts, vx.mat, vx.incident(), c.lightDir, dv, dp)) {
+                                const float w = wgt.x + wgt.y + wgt.z;
+                                r.rn[0] += w * (dv[0] - c.misFactor * dp[0]);
+                                r.rn[1] += w * (dv[1] - c.misFactor * dp[1]);
+                            }
+                        }
+                    }
+                }
+            }
+            const u64 x0 = pcg_next(rng);
+            const u64 x1 = pcg_next(rng);
+            const float rndRoulette = sample_uniform((u32)pcg_next(rng));
+            V3 rayOrigin, dir, absorption, tPrime;
+            float pdfF, cont = 1.0f;
+            if (pathLen == 0) {
+                camera_ray(S, px, py, x0, dir, pdfF);
+                rayOrigin = v3(S.camPos[0], S.camPos[1], S.camPos[2]);
+                absorption = v3(0.0f, 0.0f, 0.0f);
+            } else {
+                const bool ok =
+                    walk_surface(vx, x0, x1, rndRoulette, throughput, rayOrigin, dir, pdfF, absorption, tPrime, cont);
+                AdjVertex& r = rec[pathLen];
+                r.cont = cont;
+                if (ok && r.rtex >= 0) {
+                    float dv[2], dp[2];
+                    dln_mat_evaluate(vx.ts, vx.mat, vx.incident(), dir, dv, dp);
+                    r.rw[0] = A.fixedDecisions ? dv[0] - dp[0] : dv[0];
+                    r.rw[1] = A.fixedDecisions ? dv[1] - dp[1] : dv[1];
+                    r.rp[0] = pdfF < 1e9f ? dp[0] : 0.0f;
+                    r.rp[1] = pdfF < 1e9f ? dp[1] : 0.0f;
+                }
+                r.astar = (tPrime.x < tPrime.y) ? ((tPrime.y < tPrime.z) ? 2 : 1) : ((tPrime.x < tPrime.z) ? 2 : 0);
+                r.tp = r.astar == 0 ? tPrime.x : (r.astar == 1 ? tPrime.y : tPrime.z);
+                if (!ok) break;
+            }
+            const TraceHit hit = trace_mode<kMode, false, kAdjThreads, kLdsDepth>(
+                S.trace, rayOrigin, dir, kMaxSceneSize, lstack);
+            throughput = throughput * transmission(Medium{1.0f, absorption}, hit.inst == -1 ? kMaxSceneSize : hit.t);
+            footA += 1.0f / fsqrt(pdfF);
+            guideWeight = 1.f / (1.f + footA * footA / 1.0f);
+            const V3 prevPos = pathLen == 0 ? rayOrigin : vx.position;
+            make_vertex(S, rayOrigin, dir, pdfF, hit.t, hit.inst, hit.prim, hit.w0, hit.w1, vx);
+            ++pathLen;
             AdjVertex& r = rec[pathLen];
             r.neeW = r.emW = v3(0, 0, 0);
             r.tex = r.rtex = -1;
@@ -201,7 +216,8 @@ __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(2))
             if (!vx.isVoid) {
                 matIdx = material_index(S, vx.inst, vx.prim);
                 if (vx.mat.type == kMatLambert || vx.mat.type == kMatTorrance) r.tex = S.materials[matIdx].albedoTexture;
-                if (mat_has_roughness(vx.mat.type)) r.rtex = S.materials[matIdx].roughnessTexture;
+                if (mat_has_roughness(vx.mat.type))
+                    r.rtex = S.materials[matIdx].roughnessTexture;
             }
             if (pathLen >= S.minPathLength) {
                 V3 em;
@@ -209,53 +225,10 @@ __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(2))
                 const V3 cc = emission_contribution(S, vx, pathLen, throughput, em, prevPos, mis);
                 r.emW = delta * cc;
                 r.misC = 1.0f - mis;
-                if (matIdx >= 0 && vx.mat.type == kMatEmissive) add_emission_grad(S, A, sEmission, matIdx, r.emW);
+                if (matIdx >= 0 && vx.mat.type == kMatEmissive) add_emission_grad(S, A, matIdx, r.emW);
             }
-        }
-        bool ended = vx.isVoid || pathLen >= S.maxPathLength || pathLen >= kAdjMaxVertices;
-        if (!ended) {
-            AdjVertex& r = rec[pathLen];
-            if (pathLen + 1 >= S.minPathLength && pathLen + 1 <= S.maxPathLength) {
-                const u64 neeSeed = pcg_next(rng);
-                for (int i = 0; i < S.neeCount; ++i) {
-                    const u64 x = pcg_next(rng);
-                    NeeCandidate c;
-                    if (nee_candidate(S, vx, throughput, guideWeight, i, neeSeed, x, c) &&
-                        trace_mode<kMode, true, kAdjThreads, kLdsDepth>(S.trace, c.a, c.dir, c.tmax, lstack).inst == -1) {
-                        const V3 wgt = delta * c.radiance;
-                        r.neeW = r.neeW + wgt;
-                        if (c.lightMaterial >= 0) add_emission_grad(S, A, sEmission, c.lightMaterial, wgt);
-                        float dv[2], dp[2];
-                        if (r.rtex >= 0 && dln_mat_evaluate(vx.ts, vx.mat, vx.incident(), c.lightDir, dv, dp)) {
-                            const float w = wgt.x + wgt.y + wgt.z;
-                            r.rn[0] += w * (dv[0] - c.misFactor * dp[0]);
-                            r.rn[1] += w * (dv[1] - c.misFactor * dp[1]);
-                        }
-                    }
-                }
-            }
-            const u64 x0 = pcg_next(rng);
-            const u64 x1 = pcg_next(rng);
-            const float rndRoulette = sample_uniform((u32)pcg_next(rng));
-            V3 tPrime;
-            float cont = 1.0f;
-            const bool ok =
-                walk_surface(vx, x0, x1, rndRoulette, throughput, rayOrigin, dir, pdfF, absorption, tPrime, cont);
-            r.cont = cont;
-            if (ok && r.rtex >= 0) {
-                float dv[2], dp[2];
-                dln_mat_evaluate(vx.ts, vx.mat, vx.incident(), dir, dv, dp);
-                r.rw[0] = A.fixedDecisions ? dv[0] - dp[0] : dv[0];
-                r.rw[1] = A.fixedDecisions ? dv[1] - dp[1] : dv[1];
-                r.rp[0] = pdfF < 1e9f ? dp[0] : 0.0f;
-                r.rp[1] = pdfF < 1e9f ? dp[1] : 0.0f;
-            }
-            r.astar = (tPrime.x < tPrime.y) ? ((tPrime.y < tPrime.z) ? 2 : 1) : ((tPrime.x < tPrime.z) ? 2 : 0);
-            r.tp = r.astar == 0 ? tPrime.x : (r.astar == 1 ? tPrime.y : tPrime.z);
-            prevPos = vx.position;
-            ended = !ok;
-        }
-        if (!ended) continue;
+            if (vx.isVoid) break;
+        } while (pathLen < S.maxPathLength && pathLen < kAdjMaxVertices);
         // ---- backward: G[v] = sum of the weighted contributions after the walk from v
         const int last = pathLen;
         rec[last].G = v3(0, 0, 0);
@@ -310,12 +283,7 @@ __global__ __launch_bounds__(kAdjThreads) __attribute__((amdgpu_waves_per_eu(2))
                     for (int q = 0; q < nt; ++q) atomicAdd(grad + 4 * (size_t)idx[q] + c, w[q] * g);
             }
         }
-        pathLen = 0;
-        if (++done == A.iterations) busy = false;
     }
-    __syncthreads();
-    for (int k = threadIdx.x; k < 3 * kEmissionSlots; k += kAdjThreads)
-        if (sEmission[k] != 0.0f) atomicAdd(A.emissionGrad + k, sEmission[k]);
 }
 
 __global__ void k_adjoint_rng(u64* rngs, int num, int seed) {
@@ -331,19 +299,18 @@ __global__ void k_adjoint_rng(u64* rngs, int num, int seed) {
 
 }  // namespace
 
-void launch_pt_adjoint(const PtScene& S, const AdjointState& A, int seed, LaunchQueue& queue, int numCUs,
-                       hipStream_t stream) {
+void launch_pt_adjoint(const PtScene& S, const AdjointState& A, int seed, hipStream_t stream) {
     const int num = S.width * S.height;
     hipLaunchKernelGGL(k_adjoint_rng, dim3((num + 255) / 256), dim3(256), 0, stream, A.rngs, num, seed);
+    const dim3 grid((num + kAdjThreads - 1) / kAdjThreads);
     const int mode = trace_mode_of(S.trace);
-    auto* const fn = mode == kTraceSingle  ? k_pt_adjoint<kTraceSingle>
-                     : mode == kTraceMulti ? k_pt_adjoint<kTraceMulti>
-                                           : k_pt_adjoint<kTraceMixed>;
-    PathWork W;
-    const int grid = path_work(reinterpret_cast<const void*>(fn), num, A.iterations, queue, numCUs, W);
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(kAdjThreads), 0, stream, S, A, W);
+    if (mode == kTraceSingle)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pt_adjoint<kTraceSingle>), grid, dim3(kAdjThreads), 0, stream, S, A);
+    else if (mode == kTraceMulti)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pt_adjoint<kTraceMulti>), grid, dim3(kAdjThreads), 0, stream, S, A);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pt_adjoint<kTraceMixed>), grid, dim3(kAdjThreads), 0, stream, S, A);
     MFH_HIP(hipGetLastError());
-    queue.next ^= 1;
 }
 
 }  // namespace mfh
