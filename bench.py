@@ -53,7 +53,6 @@ def parse():
                     help="only a short run of one path-tracer workload (for rocprofv3)")
     ap.add_argument("--trace-block", type=int, default=256, help="wavefront trace block (with --pt-profile)")
     ap.add_argument("--stack-depth", type=int, default=16, help="wavefront LDS stack depth (with --pt-profile)")
-    ap.add_argument("--refill", type=int, default=0, help="wavefront lane refill budget (with --pt-profile)")
     ap.add_argument("--sort-bounces", type=int, default=0, help="wavefront sorted bounces (with --pt-profile)")
     ap.add_argument("--tail-after", type=int, default=0, help="wavefront tail bounce (with --pt-profile)")
     ap.add_argument("--terrain-ray-costs", action="store_true",
@@ -62,8 +61,6 @@ def parse():
     ap.add_argument("--leaf-limit", type=int, default=None,
                     help="longest traversal leaf of the LoD builds (0: traverse the reference BVH; default: the "
                          "library's)")
-    ap.add_argument("--leaf-batch", type=int, default=1, choices=[1, 8],
-                    help="triangles of a BVH leaf loaded ahead of their tests (with --pt-profile)")
     ap.add_argument("--profile-only", action="store_true",
                     help="steps only (no stats pass, no CPU baseline): for rocprofv3 runs")
     ap.add_argument("--pt-iterations", type=int, default=64,
@@ -204,8 +201,7 @@ def cornell_tracer(ctx):
 def pt_cornell(args, cpu_baseline_too):
     """Megakernel path tracer on the procedural Cornell box: 256x256, 128x256
     sphere, depth 8, NEE 1, seed 1; Mpaths/s = pixels * iterations / time.
-    Also the megakernel with leaf batch 8, the autotuned wavefront form and
-    the light tracer over the same scene."""
+    Also the autotuned wavefront form and the light tracer over the same scene."""
     from mufflon_amd import scenes as S
     from mufflon_amd.hip import HipContext
     ctx = HipContext(0)
@@ -224,15 +220,6 @@ def pt_cornell(args, cpu_baseline_too):
            "iterations": n, "ms_per_iteration": round(ms / n, 4),
            "mpaths_s": round(pixels * n / (ms / 1e3) / 1e6, 3)}
     from mufflon_amd import hip
-    # the megakernel with 8 triangles of a BVH leaf loaded ahead of their tests
-    ctx.pt_set_tuning(pt, leaf_batch=8)
-    ctx.pt_reset(pt)
-    ctx.timer_begin()
-    ctx.pt_iterate(pt, n)
-    m8 = ctx.timer_end()
-    same = np.array_equal(ctx.pt_target(pt), mega)
-    out["megakernel_leaf_batch_8"] = {"ms_per_iteration": round(m8 / n, 4),
-                                      "mpaths_s": round(pixels * n / (m8 / 1e3) / 1e6, 3)}
     ctx.pt_set_mode(pt, hip.PT_WAVEFRONT, True)
     tuned, _ = ctx.pt_autotune(pt, 2)
     ctx.pt_reset(pt)
@@ -243,7 +230,7 @@ def pt_cornell(args, cpu_baseline_too):
     wms = ctx.timer_end()
     out["wavefront"] = {"ms_per_iteration": round(wms / n, 4), "mpaths_s": round(pixels * n / (wms / 1e3) / 1e6, 3),
                         "tuning": tuned, "graph": True,
-                        "identical_to_megakernel": bool(same and np.array_equal(ctx.pt_target(pt), mega))}
+                        "identical_to_megakernel": bool(np.array_equal(ctx.pt_target(pt), mega))}
     out["rmse"] = converged_rmse(mega)
     from oracle import oracle as O
     sys.path.insert(0, os.path.join(ROOT, "tests"))
@@ -319,30 +306,23 @@ def pt_terrain(args):
         return ms, ctx.pt_target(pt)
 
     mk_ms, mk_img = run(hip.PT_MEGAKERNEL, False)
-    # the megakernel again with 8 triangles of a BVH leaf loaded ahead of their tests
-    ctx.pt_set_tuning(pt, leaf_batch=8)
-    mk8_ms, mk8_img = run(hip.PT_MEGAKERNEL, False)
     ctx.pt_set_mode(pt, hip.PT_WAVEFRONT, True)
     tuned, _ = ctx.pt_autotune(pt, 1)
     wf_ms, wf_img = run(hip.PT_WAVEFRONT, True)
     box, _, _, _ = ctx.scene_get(scid, len(sc["inst_lod"]))
     lt = ctx.pt_light_tree(pt)
     ctx.close()
-    best = min(mk_ms, mk8_ms)
     out = {"workload": "terrain 2236^2 fBm heightfield (9,990,450 tris) + 4096 rock instances (2000 tris), "
                        "1024 point lights, 2048x1024 env map, 1920x1080, depth 16, NEE 1, seed 1",
            "scene_generation_s": round(gen_s, 2),
            "lbvh_10m_build_ms": round(float(np.mean(builds)), 3), "lbvh_10m_build_ms_min": round(min(builds), 3),
            "iterations": its,
            "megakernel": {"ms_per_iteration": round(mk_ms, 3), "mpaths_s": round(pixels / mk_ms / 1e3, 3)},
-           "megakernel_leaf_batch_8": {"ms_per_iteration": round(mk8_ms, 3),
-                                       "mpaths_s": round(pixels / mk8_ms / 1e3, 3)},
            "wavefront": {"ms_per_iteration": round(wf_ms, 3), "mpaths_s": round(pixels / wf_ms / 1e3, 3),
                          "tuning": tuned, "graph": True},
            "wavefront_over_megakernel": round(mk_ms / wf_ms, 3),
-           "wavefront_over_best_megakernel": round(best / wf_ms, 3),
-           "identical_images": bool(np.array_equal(mk_img, wf_img) and np.array_equal(mk_img, mk8_img)),
-           "equal_rmse": "the three forms give identical images, so their RMSE against any reference is equal"}
+           "identical_images": bool(np.array_equal(mk_img, wf_img)),
+           "equal_rmse": "the two forms give identical images, so their RMSE against any reference is equal"}
     # algorithmic bytes from the oracle's work counts of every path of one
     # iteration, and the oracle itself as the CPU baseline
     from oracle import oracle as O
@@ -352,8 +332,7 @@ def pt_terrain(args):
     ps = P.oracle_pt_scene_general(O, sc, lt, box, parallel=True)
     setup_s = time.perf_counter() - t0
     stats = O.pt_path_stats(ps, 1, 0, 16, 1, 0, 0, sc["camera"]["width"], sc["camera"]["height"])
-    fast = "megakernel" if mk_ms <= mk8_ms else "megakernel_leaf_batch_8"
-    out["roofline"] = path_roofline(stats, 32, best, "k_pt_iterate (%s)" % fast)
+    out["roofline"] = path_roofline(stats, 32, mk_ms, "k_pt_iterate")
     out["roofline"]["wavefront_achieved"] = round(path_bytes(stats, 32) / (wf_ms / 1e3) / 1e9, 1)
     if not args.no_cpu_baseline:
         w, h = sc["camera"]["width"], sc["camera"]["height"]
@@ -578,7 +557,7 @@ def pt_profile(args):
     else:
         its = 8
         pt, _, _ = cornell_tracer(ctx)
-    ctx.pt_set_tuning(pt, args.trace_block, args.stack_depth, 256, args.sort_bounces, args.refill, args.leaf_batch,
+    ctx.pt_set_tuning(pt, args.trace_block, args.stack_depth, 256, args.sort_bounces, 0, 1,
                       args.tail_after)
     for mode in (hip.PT_MEGAKERNEL, hip.PT_WAVEFRONT):
         ctx.pt_set_mode(pt, mode, False)

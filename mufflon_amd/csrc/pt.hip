@@ -38,7 +38,8 @@ constexpr int kPtThreads = kPtTile * kPtTile;
 // from the queue once the call's iterations are done. Against one path per
 // lane and one launch per iteration: Cornell box 256x256, 16 iterations 22.3
 // -> 10.6 ms; terrain of 2.1M triangles and 2048 instances, 1280x720, 4
-// iterations 31.5 -> 24.5 ms; one iteration of a 200x151 room 0.82 -> 0.55 ms.
+// iterations 31.5 -> 24.5 ms; one iteration of a 200x151 room 0.82 -> 0.55 ms
+// (over binary nodes; 8.4, 20.3 and 0.43 ms over the wide ones).
 // What bounds it now is the traversal's chain of dependent loads (80 % of a
 // wave's time; about 1500 cycles a node or triangle step in the Cornell box).
 //
