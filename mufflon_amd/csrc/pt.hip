@@ -167,7 +167,8 @@ void launch_pt_init_rng(u64* rngs, int num, int seed, hipStream_t stream) {
 
 // Fewest lanes of a wave that take pixels (Cornell box 256x256, 64 / 32 / 16
 // lanes: 14.1 / 12.7 / 10.6 ms; 200x151 room, 64 / 32 / 16 / 8: 0.72 / 0.63 /
-// 0.57 / 0.55 ms; the terrain image, which fills the chip, 24.5 / 34.4 / 47.5).
+// 0.57 / 0.55 ms; the terrain image, which fills the chip, 24.5 / 34.4 / 47.5;
+// all over binary nodes).
 constexpr int kMinLanes = 8;
 
 int path_work(const void* fn, int slots, int iterations, LaunchQueue& queue, int numCUs, PathWork& W) {
