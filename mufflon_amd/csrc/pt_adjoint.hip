@@ -76,20 +76,21 @@ struct AdjVertex {
     float rn[2];    // sum over next-event estimates: weighted contribution * d ln / d(rx, ry)
 };
 
-// Every next-event estimate adds to an emitter's three sums, and a scene has few
-// emitters, so the additions to one address, which run one after another, bound
-// the kernel. With a sum every kEmissionStride floats the three do not also wait
-// for each other in one line: Cornell box, 256x256, 4 iterations, image and
-// gradients 22.6 -> 10.3 ms. (Sums in LDS per wave reach 7.5 ms; they round
-// less, and move the emission gradient by the 3e-4 that the rounding of a
-// million additions to one float makes.)
+// Every next-event estimate adds to an emitter's three sums, and a scene has
+// few emitters, so the additions to one address run one after another and bound
+// the kernel (Cornell box, 256x256, 4 iterations, image and gradients: 22.7 ms
+// over binary nodes, 18.9 over the wide ones, and 10.4 with the three sums 256
+// bytes apart). They also fix the result's rounding: a float sum of a million
+// terms of both signs lies 6e-4 to 8e-4 off the 64-bit sum of the terms, and
+// what it rounds depends on the order of arrival. Orders differ by 1e-5 between
+// runs, by up to 8e-5 with where the buffer lies in memory, and by 5e-5 to 9e-5
+// with the sums apart, which is why they stay side by side.
 __device__ __forceinline__ void add_emission_grad(const PtScene& S, const AdjointState& A, int mat, V3 weighted) {
     const PtMaterialRecord& m = S.materials[mat];
     const float w[3] = {weighted.x, weighted.y, weighted.z};
 #pragma unroll
     for (int c = 0; c < 3; ++c)
-        if (m.scale[c] != 0.0f && w[c] != 0.0f)
-            atomicAdd(A.emissionGrad + (size_t)(3 * mat + c) * kEmissionStride, w[c] / m.scale[c]);
+        if (m.scale[c] != 0.0f && w[c] != 0.0f) atomicAdd(A.emissionGrad + 3 * mat + c, w[c] / m.scale[c]);
 }
 
 // Texel weights of a texture lookup, as tex_sample forms them.

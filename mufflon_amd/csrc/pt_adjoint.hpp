@@ -5,14 +5,13 @@
 namespace mfh {
 
 constexpr int kAdjMaxVertices = 32;  // longest path the replay records
-constexpr int kEmissionStride = 64;  // 256 bytes
 
 struct AdjointState {
     const float* delta;    // dLoss/dRadiance, 3 floats per pixel
     int iterations;        // iterations of the primal image being differentiated
     uint64_t* rngs;        // replay RNG states (seeded as a reset seeds them)
     float* const* texGrad; // per texture id: gradient buffer (4 floats per texel) or null
-    float* emissionGrad;   // 3 sums per material, kEmissionStride floats apart: d loss / d emission scale
+    float* emissionGrad;   // 3 floats per material: d loss / d emission scale
     int fixedDecisions;    // 0: derivative of the expected image; 1: of this realization (MFH_ADJOINT_*)
 };
 

@@ -835,9 +835,8 @@ int mfh_pt_adjoint(mfh_context* ctx, int32_t ptId, int32_t iterations, const flo
         t.adjRngs.reserve(8 * (size_t)num);
         upload(c, t.adjDelta, radianceAdjoint, 12 * (size_t)num);
         const size_t nm = t.materials.size();
-        const size_t emBytes = sizeof(float) * 3 * kEmissionStride * nm;
-        t.adjEmGrad.reserve(emBytes);
-        MFH_HIP(hipMemsetAsync(t.adjEmGrad.ptr, 0, emBytes, c.stream));
+        t.adjEmGrad.reserve(12 * nm);
+        MFH_HIP(hipMemsetAsync(t.adjEmGrad.ptr, 0, 12 * nm, c.stream));
         // gradient buffers for every texture used as an albedo or a roughness
         t.adjTexGrad.resize(c.textures.size());
         std::vector<float*> ptrs(std::max<size_t>(c.textures.size(), 1), nullptr);
@@ -903,9 +902,7 @@ int mfh_pt_get_emission_gradient(mfh_context* ctx, int32_t ptId, int32_t materia
         MFH_REQUIRE(t.adjValid, "no adjoint has been run");
         MFH_REQUIRE(materialIndex >= 0 && materialIndex < (int32_t)t.materials.size(), "material index out of range");
         MFH_HIP(hipStreamSynchronize(c.stream));
-        MFH_HIP(hipMemcpy2D(out, sizeof(float),
-                            t.adjEmGrad.as<float>() + 3 * kEmissionStride * (size_t)materialIndex,
-                            sizeof(float) * kEmissionStride, sizeof(float), 3, hipMemcpyDeviceToHost));
+        MFH_HIP(hipMemcpy(out, t.adjEmGrad.as<float>() + 3 * (size_t)materialIndex, 12, hipMemcpyDeviceToHost));
     });
 }
 

@@ -62,6 +62,36 @@ def test_adjoint_matches_oracle_fp64(hip_ctx, oracle, sphere, shadowing, mode):
     np.testing.assert_allclose(e_gpu, e_orc[0], rtol=1e-3)
 
 
+def test_emission_gradient_of_a_large_image(hip_ctx):
+    """256x256, 4 paths per pixel: the emission gradient, one float sum of some
+    350,000 terms a channel, against the same terms summed strip by strip (64
+    strips of rows, each a sum of some 5,500 terms) in 64 bits. Every addition
+    loses at most half an ulp of the sum so far; were all the losses of one sign
+    they would reach 350000 * 2^-25 = 1e-2 of the result. Measured: 6e-4 to
+    8e-4. Two runs add in different orders: 1e-5, up to 1e-4 measured."""
+    c = S.cornell_textured(128, 256, 256, 64, 64)
+    its = 4
+    pt, ids = _setup(hip_ctx, c, 8)
+    hip_ctx.pt_iterate(pt, its)
+    img = hip_ctx.pt_target(pt)
+    delta = (2.0 * (img - np.random.default_rng(1).uniform(0.0, 1.0, img.shape))).astype(np.float32)
+    runs = []
+    for _ in range(2):
+        hip_ctx.pt_adjoint(pt, its, delta)
+        runs.append(hip_ctx.pt_emission_gradient(pt, 0).astype(np.float64))
+    strips = np.zeros(3)
+    for k in range(64):
+        part = np.zeros_like(delta)
+        part[k::64] = delta[k::64]
+        hip_ctx.pt_adjoint(pt, its, part)
+        strips += hip_ctx.pt_emission_gradient(pt, 0)
+    off = np.linalg.norm(runs[0] - strips) / np.linalg.norm(strips)
+    twice = np.linalg.norm(runs[0] - runs[1]) / np.linalg.norm(strips)
+    print("emission gradient %s, off the 64-bit sum by %.2g, twice by %.2g" % (runs[0], off, twice), flush=True)
+    assert off < 2e-3
+    assert twice < 2e-4
+
+
 def test_adjoint_finite_differences_config3(hip_ctx):
     """Fixed-decision form: 256x256, 4 spp, L2 loss to a target rendered from
     a texture of seed 11; 64 random albedo texels with a non-negligible
