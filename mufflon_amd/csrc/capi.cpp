@@ -62,10 +62,11 @@ void refresh_scene(Context& c, Scene& s) {
         lods[i].wide = l->numPrims() > 1 ? l->wideNodes.as<float4>() : nullptr;
         lods[i].leafBoxes = l->leafBoxes.as<float4>();
     }
-    s.mixed = false;
+    s.mixed = s.flat = false;
     for (int32_t li : s.instLod) {
         MFH_REQUIRE(c.lods[li]->built, "instance refers to a LoD whose BVH is not built");
         if (c.lods[li]->mixed()) s.mixed = true;
+        if (c.lods[li]->flat) s.flat = true;
     }
     upload(c, s.dLods, lods.data(), sizeof(DevLod) * lods.size());
     build_scene_bvh(c, s, nullptr);

@@ -759,8 +759,9 @@ template <class C>
 __global__ __launch_bounds__(kThreads) void k_mark(int nInt, const i32* __restrict__ parents,
                                                   const uint8_t* __restrict__ flags, i32* __restrict__ marks,
                                                   const float4* __restrict__ boxes, int refineAbove,
-                                                  i32* __restrict__ marks2) {
+                                                  i32* __restrict__ marks2, i32* __restrict__ flat) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
+    if (x == 0 && flat) *flat = 0;
     if (x >= nInt) return;
     const int keep = keep_mark(x, parents, flags);
     marks[x] = keep;
@@ -865,7 +866,8 @@ __device__ __forceinline__ WideChild wide_child(int c, bool left, int nInt, cons
 template <class C>
 __device__ __forceinline__ void wide_node(int x, int n, const i32* __restrict__ children,
                                           const float4* __restrict__ boxes, const i32* offsets,
-                                          float4* __restrict__ wide, float4* __restrict__ leafBoxes) {
+                                          float4* __restrict__ wide, float4* __restrict__ leafBoxes, float flatBelow,
+                                          i32* flat) {
     const int nInt = n - 1;
     if (is_collapsed(offsets, nInt, x)) return;
     WideChild ch[4];
@@ -878,6 +880,8 @@ __device__ __forceinline__ void wide_node(int x, int n, const i32* __restrict__ 
             const size_t at = 2 * (size_t)(ch[k].ref & ~kWideLeaf);
             leafBoxes[at] = make_float4(ch[k].lo.x, ch[k].lo.y, ch[k].lo.z, ch[k].hi.x);
             leafBoxes[at + 1] = make_float4(ch[k].hi.y, ch[k].hi.z, __int_as_float(count), 0.0f);
+            const V3 e = ch[k].hi - ch[k].lo;
+            if (!(e.x > flatBelow && e.y > flatBelow && e.z > flatBelow)) *flat = 1;
         }
     }
 #pragma unroll
@@ -955,9 +959,9 @@ template <class C>
 __global__ __launch_bounds__(kThreads) void k_wide(int n, const i32* __restrict__ children,
                                                   const float4* __restrict__ boxes,
                                                   const i32* __restrict__ offsets, float4* __restrict__ wide,
-                                                  float4* __restrict__ leafBoxes) {
+                                                  float4* __restrict__ leafBoxes, float flatBelow, i32* flat) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x < n - 1) wide_node<C>(x, n, children, boxes, offsets, wide, leafBoxes);
+    if (x < n - 1) wide_node<C>(x, n, children, boxes, offsets, wide, leafBoxes, flatBelow, flat);
 }
 
 // ---- builds of 2 to kSmallBuild primitives
@@ -1056,9 +1060,12 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_collapse(int n, const i
                                                                  i32* __restrict__ offsets,
                                                                  BvhChild* __restrict__ out,
                                                                  float4* __restrict__ wide,
-                                                                 float4* __restrict__ leafBoxes) {
+                                                                 float4* __restrict__ leafBoxes, float flatBelow,
+                                                                 i32* __restrict__ flat) {
     __shared__ i32 sOff[kSmallBuild], sOff2[kSmallBuild];
     __shared__ int sWave[kSmallThreads / 64];
+    __shared__ i32 sFlat;
+    if (threadIdx.x == 0) sFlat = 0;
     const int nInt = n - 1;
     int keep[kSmallIpt], keep2[kSmallIpt];
     int sum = 0, sum2 = 0;
@@ -1086,7 +1093,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_collapse(int n, const i
         collapse_node<C>(node, n, parents, boxes, sOff, out);
     if (wide)
         for (int x = threadIdx.x; x < nInt; x += kSmallThreads)
-            wide_node<C>(x, n, children, boxes, sOff2, wide, leafBoxes);
+            wide_node<C>(x, n, children, boxes, sOff2, wide, leafBoxes, flatBelow, &sFlat);
+    __syncthreads();
+    if (flat && threadIdx.x == 0) *flat = sFlat;
 }
 
 // Zero fill of the build (a kernel, not a memset, so that a
@@ -1139,13 +1148,15 @@ struct WideOut {
     int refineAbove;
     DevBuf* nodes;
     DevBuf* leafBoxes;
+    float flatBelow;  // a leaf box with no more extent than this along an axis is flat
+    bool flat;        // out: there is one
 };
 
 // Shared orchestration (build_lbvh.cu:586-780). Returns the number of
 // internal nodes after the collapse; primIds and nodes receive the result.
 template <class P, class C>
 int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const float* bbox, DevBuf& nodes,
-                  DevBuf& primIds, float4* triVerts, StageSink* sink, const WideOut* wideOut = nullptr,
+                  DevBuf& primIds, float4* triVerts, StageSink* sink, WideOut* wideOut = nullptr,
                   float4* stage = nullptr) {
     hipStream_t st = ctx.stream;
     MFH_REQUIRE(n < kMaxPrims, "an LBVH build holds fewer than 2^29 primitives");
@@ -1160,7 +1171,7 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
     s.boxes.reserve(32 * (size_t)(2 * n - 1));
     s.counters.reserve(4 * (size_t)std::max(n - 1, 1));
     s.flags.reserve((size_t)std::max(n - 1, 1));
-    s.offsets.reserve(4 * (size_t)std::max(n - 1, 1));
+    s.offsets.reserve(4 * (size_t)std::max(n - 1, 1) + (wideOut ? 4 : 0));  // LoDs: and whether there are flat leaves
     primIds.reserve(4 * (size_t)n);
     Box6 bb;
     std::memcpy(bb.v, bbox, sizeof(bb.v));
@@ -1221,18 +1232,20 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
         wideOut->nodes->reserve(64 * (size_t)(n - 1));
         wideOut->leafBoxes->reserve(32 * (size_t)n);
     }
+    i32* const flat = wideOut ? offsets + (n - 1) : nullptr;
+    const float flatBelow = wideOut ? wideOut->flatBelow : 0.0f;
     if (small) {
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_small_collapse<C>), dim3(1), dim3(kSmallThreads), 0, st, n, parents,
                            children, s.flags.as<uint8_t>(), boxes, refining ? wideOut->refineAbove : 0, offsets,
                            nodes.as<BvhChild>(), wideOut ? wideOut->nodes->as<float4>() : nullptr,
-                           wideOut ? wideOut->leafBoxes->as<float4>() : nullptr);
+                           wideOut ? wideOut->leafBoxes->as<float4>() : nullptr, flatBelow, flat);
     } else {
         if (refining) {
             s.offsets2.reserve(4 * (size_t)(n - 1));
             offsets2 = s.offsets2.as<i32>();
         }
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_mark<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n - 1, parents,
-                           s.flags.as<uint8_t>(), offsets, boxes, refining ? wideOut->refineAbove : 0, offsets2);
+                           s.flags.as<uint8_t>(), offsets, boxes, refining ? wideOut->refineAbove : 0, offsets2, flat);
         if (refining)
             scan_inclusive_i32_pair(offsets, offsets2, n - 1, s, st);
         else
@@ -1242,19 +1255,20 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
         if (wideOut) {
             hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wide<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n, children,
                                boxes, refining ? offsets2 : offsets, wideOut->nodes->as<float4>(),
-                               wideOut->leafBoxes->as<float4>());
+                               wideOut->leafBoxes->as<float4>(), flatBelow, flat);
         }
     }
     MFH_HIP(hipGetLastError());
-    i32 nAfter = 0;
-    MFH_HIP(hipMemcpyAsync(&nAfter, offsets + (n - 2), sizeof(nAfter), hipMemcpyDeviceToHost, st));
+    i32 counts[2] = {0, 0};  // internal nodes, flat leaves
+    MFH_HIP(hipMemcpyAsync(counts, offsets + (n - 2), wideOut ? 8 : 4, hipMemcpyDeviceToHost, st));
     MFH_HIP(hipStreamSynchronize(st));
+    if (wideOut) wideOut->flat = counts[1] != 0;
     if (sink) {
         d2h(st, sink->parents, parents, 2 * (size_t)n - 1);
         d2h(st, sink->boxes, boxes, 8 * (size_t)(2 * n - 1));
         d2h(st, sink->offsets, offsets, (size_t)n - 1);
     }
-    return nAfter;
+    return counts[0];
 }
 
 }  // namespace
@@ -1264,7 +1278,11 @@ void build_lod_bvh(Context& ctx, Lod& lod, const float* bbox, StageSink* sink) {
     MFH_REQUIRE(n >= 1, "LoD has no primitives");
     if (bbox) std::memcpy(lod.box, bbox, sizeof(lod.box));
     lod.triVerts.reserve(48 * (size_t)n);
-    const WideOut wide{ctx.traversalLeafLimit, &lod.wideNodes, &lod.leafBoxes};
+    // Flat: no more extent than two ulps of the largest coordinate, so that where a
+    // ray enters the box is lost in rounding (Trav's kTies). A line at 64 ulps would
+    // take 33 of the 2.1M triangles of a heightfield for flat, and with them the
+    // whole scene through the slower kernels.
+    WideOut wide{ctx.traversalLeafLimit, &lod.wideNodes, &lod.leafBoxes, lod.coordMax * 0x1p-22f, false};
     if (lod.mixed()) {
         if (lod.numQuads > 0) lod.quadV3.reserve(16 * (size_t)n);
         MixedPrims set{lod.verts.as<float>(), lod.tris.as<u32>(),  lod.quads.as<u32>(), lod.spheres.as<float4>(),
@@ -1278,6 +1296,7 @@ void build_lod_bvh(Context& ctx, Lod& lod, const float* bbox, StageSink* sink) {
                                                            lod.primIds, lod.triVerts.as<float4>(), sink, &wide,
                                                            ctx.scratch.stage.as<float4>());
     }
+    lod.flat = wide.flat;
     lod.built = true;
 }
 

@@ -397,9 +397,11 @@ void launch_lighttracer(const PtScene& S, int iterations, float* splat, float* m
     const size_t all = n * iterations;
     hipLaunchKernelGGL(k_lt_clear, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, stream, splat, all);
     const int mode = trace_mode_of(S.trace);
-    auto* const fn = mode == kTraceSingle  ? k_lt_iterate<kTraceSingle>
-                     : mode == kTraceMixed ? k_lt_iterate<kTraceMixed>
-                                           : k_lt_iterate<kTraceMulti>;
+    auto* const fn = mode == kTraceSingle       ? k_lt_iterate<kTraceSingle>
+                     : mode == kTraceMulti      ? k_lt_iterate<kTraceMulti>
+                     : mode == kTraceSingleTies ? k_lt_iterate<kTraceSingleTies>
+                     : mode == kTraceMultiTies  ? k_lt_iterate<kTraceMultiTies>
+                                                : k_lt_iterate<kTraceMixed>;
     PathWork W;
     const int grid =
         path_work(reinterpret_cast<const void*>(fn), S.width * S.height, iterations, queue, numCUs, W);

@@ -144,6 +144,7 @@ struct Lod {
     // leaves' first primitive that leaf's box and primitive count (32 bytes)
     DevBuf wideNodes;
     DevBuf leafBoxes;
+    bool flat = false;        // a leaf's box has (next to) no extent along an axis
     int32_t numPrims() const { return numTris + numQuads + numSpheres; }
     bool mixed() const { return numQuads > 0 || numSpheres > 0; }
 };
@@ -158,6 +159,7 @@ struct Scene {
     int32_t tlasNumInternal = 0;
     DevBuf tlasNodes, tlasPrimIds;
     bool mixed = false;  // an instance's LoD holds quads or spheres
+    bool flat = false;   // an instance's LoD has flat leaves
 };
 
 struct PathTracer;
@@ -256,6 +258,7 @@ struct TraceParams {
     int32_t tlasNumInternal;
     float tlasCoordMax;  // largest |coordinate| of the scene box (bounds the instance-level node boxes)
     int32_t mixed;       // an instance's LoD holds quads or spheres (kernels with kMixed)
+    int32_t flat;        // an instance's LoD has flat leaves (kernels with kTies)
 };
 TraceParams trace_params(const Scene& sc);
 void launch_trace_closest(const TraceParams& p, const float* rays, int n, float4* hits, float2* bary,

@@ -202,9 +202,11 @@ IterateFn iterate_kernel(bool neeOne) {
 void launch_pt_iterate(const PtScene& S, int iterations, LaunchQueue& queue, int numCUs, hipStream_t stream) {
     const int mode = trace_mode_of(S.trace);
     const bool neeOne = S.neeCount <= 1;
-    const IterateFn fn = mode == kTraceSingle  ? iterate_kernel<kTraceSingle>(neeOne)
-                         : mode == kTraceMulti ? iterate_kernel<kTraceMulti>(neeOne)
-                                               : iterate_kernel<kTraceMixed>(neeOne);
+    const IterateFn fn = mode == kTraceSingle       ? iterate_kernel<kTraceSingle>(neeOne)
+                         : mode == kTraceMulti      ? iterate_kernel<kTraceMulti>(neeOne)
+                         : mode == kTraceSingleTies ? iterate_kernel<kTraceSingleTies>(neeOne)
+                         : mode == kTraceMultiTies  ? iterate_kernel<kTraceMultiTies>(neeOne)
+                                                    : iterate_kernel<kTraceMixed>(neeOne);
     const int tilesX = (S.width + kPtTile - 1) / kPtTile;
     const int tiles = tilesX * ((S.height + kPtTile - 1) / kPtTile);
     PathWork W;

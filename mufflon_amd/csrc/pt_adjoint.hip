@@ -305,12 +305,12 @@ void launch_pt_adjoint(const PtScene& S, const AdjointState& A, int seed, hipStr
     hipLaunchKernelGGL(k_adjoint_rng, dim3((num + 255) / 256), dim3(256), 0, stream, A.rngs, num, seed);
     const dim3 grid((num + kAdjThreads - 1) / kAdjThreads);
     const int mode = trace_mode_of(S.trace);
-    if (mode == kTraceSingle)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pt_adjoint<kTraceSingle>), grid, dim3(kAdjThreads), 0, stream, S, A);
-    else if (mode == kTraceMulti)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pt_adjoint<kTraceMulti>), grid, dim3(kAdjThreads), 0, stream, S, A);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pt_adjoint<kTraceMixed>), grid, dim3(kAdjThreads), 0, stream, S, A);
+    auto* const fn = mode == kTraceSingle       ? k_pt_adjoint<kTraceSingle>
+                     : mode == kTraceMulti      ? k_pt_adjoint<kTraceMulti>
+                     : mode == kTraceSingleTies ? k_pt_adjoint<kTraceSingleTies>
+                     : mode == kTraceMultiTies  ? k_pt_adjoint<kTraceMultiTies>
+                                                : k_pt_adjoint<kTraceMixed>;
+    hipLaunchKernelGGL(fn, grid, dim3(kAdjThreads), 0, stream, S, A);
     MFH_HIP(hipGetLastError());
 }
 

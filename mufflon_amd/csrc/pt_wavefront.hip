@@ -146,11 +146,11 @@ __global__ void k_wf_begin(WfState W) {
 }
 
 // Camera rays and their closest hits, one thread per pixel: 16x16 tiles for
-// one scene, one path per thread in path order for a batch (kMode 2).
+// one scene, one path per thread in path order for a batch (kTraceBatch).
 template <int kMode>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMode == 1 ? 5 : 4))) void k_wf_primary(PtScene S0, WfState W) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(mode_single(kMode) ? 5 : 4))) void k_wf_primary(PtScene S0, WfState W) {
     __shared__ int sStack[kLdsDepth * 256];
-    constexpr bool kBatch = kMode == 2;
+    constexpr bool kBatch = kMode == kTraceBatch;
     int px, py, p, local, s = 0;
     if constexpr (kBatch) {
         p = blockIdx.x * 256 + threadIdx.x;
@@ -191,10 +191,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMode == 1 
 
 // Closest hit of queue `buf` (length at counters[count]).
 template <int kMode, int kBlock, int kLds>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMode == 1 ? 5 : 4))) void k_wf_extend(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(mode_single(kMode) ? 5 : 4))) void k_wf_extend(
     PtScene S0, WfState W, int buf, int count, int work, const int* perm) {
     __shared__ int sStack[kLds * kBlock];
-    constexpr bool kBatch = kMode == 2;
+    constexpr bool kBatch = kMode == kTraceBatch;
     using T = ModeTrav<kMode, false, kBlock, kLds>;
     const int n = W.counters[count];
     const int waves = (int)(gridDim.x * blockDim.x) / 64;
@@ -228,10 +228,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMode ==
 // candidate's ray when every slot holds at most one (neeStride 1); otherwise
 // the candidates of a slot are traced in turn.
 template <int kMode, int kBlock, int kLds>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMode == 1 ? 5 : 4))) void k_wf_shadow(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(mode_single(kMode) ? 5 : 4))) void k_wf_shadow(
     PtScene S0, WfState W, int count, int work, const int* perm) {
     __shared__ int sStack[kLds * kBlock];
-    constexpr bool kBatch = kMode == 2;
+    constexpr bool kBatch = kMode == kTraceBatch;
     using T = ModeTrav<kMode, true, kBlock, kLds>;
     const int n = W.counters[count];
     const int waves = (int)(gridDim.x * blockDim.x) / 64;
@@ -405,7 +405,7 @@ template <int kMode>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_wf_tail(PtScene S0, WfState W, int k,
                                                                                        int buf, int count, int work) {
     __shared__ int sStack[kLdsDepth * 256];
-    constexpr bool kBatch = kMode == 2;
+    constexpr bool kBatch = kMode == kTraceBatch;
     const int n = W.counters[count];
     int* const lstack = sStack + threadIdx.x;
     for (QueueWalk wk(n, W.chunk); wk.base < n; wk.next(W.counters + work)) {
@@ -547,13 +547,13 @@ struct TraceKernels {
     }
     static void shadow(const PtScene& S, const WfState& W, int grid, int count, int work, const int* perm,
                        hipStream_t st) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_shadow<kMode, kBlock, kLds>), dim3(grid), dim3(kBlock), 0, st, S, W,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wf_shadow<any_mode(kMode), kBlock, kLds>), dim3(grid), dim3(kBlock), 0, st, S, W,
                            count, work, perm);
     }
     static int occupancy() {
         int a = 0, b = 0;
         MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_wf_extend<kMode, kBlock, kLds>, kBlock, 0));
-        MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_shadow<kMode, kBlock, kLds>, kBlock, 0));
+        MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_shadow<any_mode(kMode), kBlock, kLds>, kBlock, 0));
         return std::max(1, std::min(a, b));
     }
 };
@@ -575,15 +575,14 @@ constexpr TraceVariant variant() {
 }
 
 // Tuning space of the trace stages: block size x LDS stack depth, for
-// multi-instance scenes (0), single-instance scenes (1), batches (2) and
-// scenes with quads or spheres (3).
+// each traversal mode.
 template <int kMode>
 constexpr std::array<TraceVariant, kWfNumTraceVariants> variants() {
     return {variant<kMode, 64, 8>(),   variant<kMode, 64, 16>(), variant<kMode, 128, 8>(), variant<kMode, 128, 16>(),
             variant<kMode, 256, 8>(), variant<kMode, 256, 16>(), variant<kMode, 256, 24>()};
 }
-const std::array<TraceVariant, kWfNumTraceVariants> kVariants[4] = {variants<0>(), variants<1>(), variants<2>(),
-                                                                     variants<3>()};
+const std::array<TraceVariant, kWfNumTraceVariants> kVariants[kTraceModes] = {
+    variants<0>(), variants<1>(), variants<2>(), variants<3>(), variants<4>(), variants<5>()};
 
 }  // namespace
 
@@ -606,20 +605,25 @@ int wf_shade_grid(int numCUs) {
     return std::max(1, std::min(a, b)) * numCUs;
 }
 
+namespace {
+using TailFn = void (*)(PtScene, WfState, int, int, int, int);
+const TailFn kTail[kTraceModes] = {k_wf_tail<0>, k_wf_tail<1>, k_wf_tail<2>, k_wf_tail<3>, k_wf_tail<4>, k_wf_tail<5>};
+}  // namespace
+
 int wf_tail_grid(int numCUs) {
-    int a = 0, b = 0, c = 0, d = 0;
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, k_wf_tail<0>, 256, 0));
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_wf_tail<1>, 256, 0));
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, k_wf_tail<2>, 256, 0));
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&d, k_wf_tail<3>, 256, 0));
-    return std::max(1, std::min(std::min(a, d), std::min(b, c))) * numCUs;
+    int blocks = 0;
+    for (int mode = 0; mode < kTraceModes; ++mode) {
+        int b = 0;
+        MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, kTail[mode], 256, 0));
+        blocks = mode == 0 ? b : std::min(blocks, b);
+    }
+    return std::max(1, blocks) * numCUs;
 }
 
 namespace {
 void launch_tail(int mode, const PtScene& S, const WfState& W, int grid, int k, int buf, int count, int work,
                  hipStream_t st) {
-    auto* const fn = mode == 0 ? k_wf_tail<0> : (mode == 1 ? k_wf_tail<1> : (mode == 2 ? k_wf_tail<2> : k_wf_tail<3>));
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, st, S, W, k, buf, count, work);
+    hipLaunchKernelGGL(kTail[mode], dim3(grid), dim3(256), 0, st, S, W, k, buf, count, work);
     MFH_HIP(hipGetLastError());
 }
 }  // namespace
@@ -639,7 +643,11 @@ void launch_pt_wavefront(const PtScene& S, const WfState& W, const WfTuning& tun
     hipLaunchKernelGGL(k_wf_begin, dim3((W.numCounters + 255) / 256), dim3(256), 0, stream, W);
     const dim3 pgrid((S.width + 15) / 16, (S.height + 15) / 16);
     auto* const primary =
-        mode == kTraceSingle ? k_wf_primary<1> : (mode == kTraceMulti ? k_wf_primary<0> : k_wf_primary<3>);
+        mode == kTraceSingle       ? k_wf_primary<kTraceSingle>
+        : mode == kTraceMulti      ? k_wf_primary<kTraceMulti>
+        : mode == kTraceSingleTies ? k_wf_primary<kTraceSingleTies>
+        : mode == kTraceMultiTies  ? k_wf_primary<kTraceMultiTies>
+                                   : k_wf_primary<kTraceMixed>;
     hipLaunchKernelGGL(primary, pgrid, dim3(256), 0, stream, S, W);
     // pt_sample's loop is a do-while: the first hit is shaded even at maximum path length 0
     const int L = S.maxPathLength > 1 ? S.maxPathLength : 1;

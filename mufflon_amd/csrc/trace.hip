@@ -10,16 +10,16 @@ constexpr int kThreads = 64;
 
 // Persistent waves over the rays (trace_queue). kAny: stop at the first
 // accepted hit. kSingle: the scene has one instance (no instance level).
-// kMixed: the scene's LoDs hold quads or spheres. Waves per SIMD: what the
+// kMixed: the scene's LoDs hold quads or spheres. kTies: see Trav. Waves per SIMD: what the
 // persistent traversal needs itself (89 and 127 VGPRs; one wave more a SIMD
 // spills in the loop: 1M-triangle trace 1.75 instead of 1.65 ms, instanced
 // 1.64 instead of 0.92 ms). The called reference traversal would take 150.
-template <bool kAny, bool kSingle, bool kMixed>
+template <bool kAny, bool kSingle, bool kMixed, bool kTies>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kSingle ? 5 : 4))) void k_trace(
     TraceParams p, const float4* __restrict__ rays, int n, float4* __restrict__ hits, float2* __restrict__ bary,
     int* __restrict__ occluded, int lanes, int chunk, int* queue, int* nextQueue) {
     __shared__ int sStack[kLdsDepth * kThreads];
-    using T = Trav<kAny, kSingle, kMixed, kThreads, kLdsDepth>;
+    using T = Trav<kAny, kSingle, kMixed, kTies, kThreads, kLdsDepth>;
     if (blockIdx.x == 0 && threadIdx.x == 0) *nextQueue = 0;
     WaveQueue q(n, lanes, chunk, (int)blockIdx.x, (int)gridDim.x, queue);
     trace_queue<T>(
@@ -57,10 +57,14 @@ __global__ __launch_bounds__(kThreads) void k_trace_counts(TraceParams p, const 
 
 using TraceFn = void (*)(TraceParams, const float4*, int, float4*, float2*, int*, int, int, int*, int*);
 
+template <bool kAny, bool kSingle>
+TraceFn trace_kernel(const TraceParams& p) {
+    if (p.mixed) return k_trace<kAny, kSingle, true, !kAny>;
+    return !kAny && p.flat ? k_trace<kAny, kSingle, false, !kAny> : k_trace<kAny, kSingle, false, false>;
+}
 template <bool kAny>
 TraceFn trace_kernel(const TraceParams& p) {
-    if (p.numInstances == 1) return p.mixed ? k_trace<kAny, true, true> : k_trace<kAny, true, false>;
-    return p.mixed ? k_trace<kAny, false, true> : k_trace<kAny, false, false>;
+    return p.numInstances == 1 ? trace_kernel<kAny, true>(p) : trace_kernel<kAny, false>(p);
 }
 
 void launch_trace(TraceFn fn, const TraceParams& p, const float* rays, int n, float4* hits, float2* bary, int* occ,
@@ -92,6 +96,7 @@ TraceParams trace_params(const Scene& sc) {
     p.tlasCoordMax = 0.0f;
     for (int k = 0; k < 6; ++k) p.tlasCoordMax = std::max(p.tlasCoordMax, std::fabs(sc.box[k]));
     p.mixed = sc.mixed ? 1 : 0;
+    p.flat = sc.flat ? 1 : 0;
     return p;
 }
 

@@ -15,9 +15,11 @@
 // slab test of the reference CPU path (intersection.cu:57-75); the quantized
 // boxes above contain that box and are tested with an error margin, so they
 // only cull. (A node step replaces two binary ones, with half their dependent
-// loads; 44 -> 23.5 steps a ray on a 1M-triangle mesh, 8.3 triangle tests.) Closest hit is the lexicographic minimum of (t, instance,
-// primitive), which does not depend on the order inside an object; the order
-// of the objects, whose entry and exit round the hit distance
+// loads; 44 -> 23.5 steps a ray on a 1M-triangle mesh, 8.3 triangle tests.)
+// Closest hit is the lexicographic minimum of (t, instance, primitive), which
+// depends on the order inside an object only where surfaces coincide
+// (Trav::test_leaf hands such rays to the reference's order); the order of the
+// objects, whose entry and exit round the hit distance
 // (intersection.cu:321-361), is the reference's.
 #pragma once
 #include "mfh_device.hpp"
@@ -559,7 +561,7 @@ __device__ __forceinline__ ObjectData object_data(const DevLod& lod) {
 // descending until it reaches a second one or half of the active lanes hold
 // one; then the held leaves are tested, so node steps and leaf tests run with
 // more lanes active.
-template <bool kAny, bool kSingle, bool kMixed, int kStride, int kLds>
+template <bool kAny, bool kSingle, bool kMixed, bool kTies, int kStride, int kLds>
 struct Trav {
     static constexpr int kSpill = kWideCap - kLds;
     WideStack<kStride, kLds> st;
@@ -574,6 +576,7 @@ struct Trav {
     int node, count, offset;  // instance level: node (count 2) or the rest of a leaf
     u32 cur, held;     // node or leaf to do next, the postponed leaf
     bool inObj, done, exact;  // exact: the ray is reference_ray's
+    bool flat;                // kTies: the best hit lies before the entry of its leaf's box
 
     __device__ __forceinline__ void enter(const ObjectEntry& e, const DevLod& lod, int instance) {
         inst = instance;
@@ -590,6 +593,7 @@ struct Trav {
         inObj = true;
         cur = 0u;
         held = kWideNone;
+        if (kTies) flat = false;
     }
     // An object of a single primitive: tested at once. The hit distance takes
     // the way through the object's space and back as for any entered object.
@@ -618,6 +622,7 @@ struct Trav {
         hInst = hPrim = -1;
         hw0 = hw1 = 0.0f;
         scale = 1.0f;
+        if (kTies) flat = false;
         inObj = done = exact = false;
         cur = held = kWideNone;
         node = count = offset = 0;
@@ -694,6 +699,18 @@ struct Trav {
     }
     // The primitives of the held leaf: its box, then its records, the next one
     // loaded while one is tested.
+    //
+    // Where surfaces coincide in flat boxes the closest hit depends on the order
+    // of the leaves: such a box has no extent along its normal, so the rounded
+    // distance at which a ray enters it may exceed that of the hit inside
+    // (entry > t), and whether a second leaf is still entered once a hit is known
+    // then depends on which came first. So with kTies a leaf that is entered past
+    // the hit by no more than the rounding (make_wide_ray's margin) is tested too,
+    // and the ray is the reference traversal's (exact) when it holds a closer hit,
+    // or when a hit lies that close behind a best one with entry > t. (1 ray in
+    // 1300 in a room whose boxes stand on the floor, none in 10M rays of the
+    // Cornell box. kTies takes 1.05 times the time on the 1M-triangle mesh and in
+    // the Cornell box, so scenes without flat leaves go without.)
     __device__ __forceinline__ void test_leaf(const ObjectData& od) {
         const u32 first = held & ~kWideLeaf;
         held = kWideNone;
@@ -704,7 +721,15 @@ struct Trav {
         const float lo[3] = {b0.x, b0.y, b0.z}, hi[3] = {b0.w, b1.x, b1.y};
         const FastRay r{w.o, dir, w.inv, w.o * w.inv};
         float entry;
-        if (!slab_fast(lo, hi, r, hitT, entry)) return;
+        bool late = false;
+        if constexpr (kTies) {
+            float margin = 0.0f;
+            if (hInst == inst) margin = __builtin_fmaxf(__builtin_fmaxf(w.eps.x, w.eps.y), w.eps.z);
+            if (!slab_fast(lo, hi, r, hitT + margin, entry)) return;
+            late = entry > hitT;
+        } else {
+            if (!slab_fast(lo, hi, r, hitT, entry)) return;
+        }
         const int n = __float_as_int(b1.z);
         for (int k = 0;;) {
             float4 na = a, nb = b, nc = c;
@@ -716,15 +741,25 @@ struct Trav {
             }
             float t, w0, w1;
             const int prim = __float_as_int(a.w);
-            if (prim_hit<kMixed>(r, a, b, c, (int)first + k, [&] { return od.quadV3; }, t, w0, w1) &&
-                better(t, inst, prim, hitT, hInst, hPrim)) {
-                hitT = t;
-                hInst = inst;
-                hPrim = prim;
-                hw0 = w0;
-                hw1 = w1;
-                if (kAny) {
-                    done = true;
+            if (prim_hit<kMixed>(r, a, b, c, (int)first + k, [&] { return od.quadV3; }, t, w0, w1)) {
+                if (better(t, inst, prim, hitT, hInst, hPrim)) {
+                    if (kTies && late) {
+                        exact = done = true;
+                        return;
+                    }
+                    hitT = t;
+                    hInst = inst;
+                    hPrim = prim;
+                    hw0 = w0;
+                    hw1 = w1;
+                    if (kTies) flat = t < entry;
+                    if (kAny) {
+                        done = true;
+                        return;
+                    }
+                } else if (kTies && flat && hInst == inst &&
+                           t - hitT <= __builtin_fmaxf(__builtin_fmaxf(w.eps.x, w.eps.y), w.eps.z)) {
+                    exact = done = true;
                     return;
                 }
             }
@@ -808,13 +843,24 @@ struct Trav {
 // for one scene, or chosen per ray (a batch of scenes mixes single- and
 // multi-instance scenes; a scene with quads or spheres takes the general
 // form).
-constexpr int kTraceMulti = 0;   // instance level, triangle LoDs
-constexpr int kTraceSingle = 1;  // one instance, triangle LoDs
-constexpr int kTraceBatch = 2;   // per ray, triangle LoDs
-constexpr int kTraceMixed = 3;   // per ray, LoDs with quads and spheres
+constexpr int kTraceMulti = 0;       // instance level, triangle LoDs without flat leaves
+constexpr int kTraceSingle = 1;      // one instance, a triangle LoD without flat leaves
+constexpr int kTraceBatch = 2;       // per ray, triangle LoDs
+constexpr int kTraceMixed = 3;       // per ray, LoDs with quads and spheres
+constexpr int kTraceMultiTies = 4;   // instance level, triangle LoDs (Trav's kTies)
+constexpr int kTraceSingleTies = 5;  // one instance, a triangle LoD
+constexpr int kTraceModes = 6;
+constexpr bool mode_single(int mode) { return mode == kTraceSingle || mode == kTraceSingleTies; }
+constexpr bool mode_ties(int mode) { return mode != kTraceMulti && mode != kTraceSingle; }
+// The mode of any hits, which do not depend on the order of the leaves.
+constexpr int any_mode(int mode) {
+    return mode == kTraceMultiTies ? kTraceMulti : (mode == kTraceSingleTies ? kTraceSingle : mode);
+}
 // The mode of a kernel tracing one scene.
 inline int trace_mode_of(const TraceParams& p) {
-    return p.mixed ? kTraceMixed : (p.numInstances == 1 ? kTraceSingle : kTraceMulti);
+    if (p.mixed) return kTraceMixed;
+    if (p.numInstances == 1) return p.flat ? kTraceSingleTies : kTraceSingle;
+    return p.flat ? kTraceMultiTies : kTraceMulti;
 }
 // Lanes of each wave that take entries of a queue of n: all 64, or where that
 // would leave more than three quarters of the `waves` resident waves without
@@ -920,7 +966,7 @@ __device__ __forceinline__ void trace_queue(WaveQueue& q, int* lstack, Params pa
 
 // The traversal of a kernel in mode kMode.
 template <int kMode, bool kAny, int kStride, int kLds>
-using ModeTrav = Trav<kAny, kMode == kTraceSingle, kMode == kTraceMixed, kStride, kLds>;
+using ModeTrav = Trav<kAny, mode_single(kMode), kMode == kTraceMixed, !kAny && mode_ties(kMode), kStride, kLds>;
 
 // Closest (kAny = false) or any hit in mode kMode.
 template <int kMode, bool kAny, int kStride, int kLds>

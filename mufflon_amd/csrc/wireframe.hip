@@ -149,15 +149,12 @@ void launch_wireframe(const PtScene& S, const uint32_t* seeds, float lineWidth, 
                       hipStream_t stream) {
     const dim3 grid((S.width + kWfTile - 1) / kWfTile, (S.height + kWfTile - 1) / kWfTile);
     const int mode = trace_mode_of(S.trace);
-    if (mode == kTraceSingle)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wireframe<kTraceSingle>), grid, dim3(kWfThreads), 0, stream, S, seeds,
-                           lineWidth, maxTraceDepth);
-    else if (mode == kTraceMulti)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wireframe<kTraceMulti>), grid, dim3(kWfThreads), 0, stream, S, seeds,
-                           lineWidth, maxTraceDepth);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wireframe<kTraceMixed>), grid, dim3(kWfThreads), 0, stream, S, seeds,
-                           lineWidth, maxTraceDepth);
+    auto* const fn = mode == kTraceSingle       ? k_wireframe<kTraceSingle>
+                     : mode == kTraceMulti      ? k_wireframe<kTraceMulti>
+                     : mode == kTraceSingleTies ? k_wireframe<kTraceSingleTies>
+                     : mode == kTraceMultiTies  ? k_wireframe<kTraceMultiTies>
+                                                : k_wireframe<kTraceMixed>;
+    hipLaunchKernelGGL(fn, grid, dim3(kWfThreads), 0, stream, S, seeds, lineWidth, maxTraceDepth);
     MFH_HIP(hipGetLastError());
 }
 

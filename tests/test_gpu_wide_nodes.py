@@ -79,6 +79,45 @@ def test_wide_traversal_matches_oracle(hip_ctx, oracle, name, limit):
         assert np.array_equal(hip_ctx.trace_any(sc, rays), oracle.trace_any(oscene, rays))
 
 
+@pytest.mark.parametrize("shift", [0.0, 0.3, 7.7])
+@pytest.mark.parametrize("instances", [1, 2])
+def test_coinciding_surfaces(hip_ctx, oracle, instances, shift):
+    """Two sheets of different cells in one plane, and a fine one a few ulps
+    beside them: at every ray two or three surfaces lie equally far to the last
+    bits, their boxes are flat, and which of them is reported depends on the
+    order of the leaves. Bit for bit the oracle's."""
+    v, t = [], []
+    for n, y in ((40, shift), (7, shift), (23, shift + 2e-7 * max(shift, 1.0))):
+        gv, gt = _grid(n)
+        t.append(gt + sum(len(x) for x in v))
+        v.append(gv * np.float32([1.0, 0.0, 1.0]) + np.float32([0.013 * n, y, 0.007 * n]))
+    v, t = np.concatenate(v).astype(np.float32), np.concatenate(t).astype(np.uint32)
+    lod = hip_ctx.lod_create(v, t)
+    hip_ctx.lbvh_build(lod)
+    w = np.concatenate([S.IDENTITY34.reshape(1, 12), U.random_transforms(1, 5)])[:instances]
+    il = np.zeros(instances, np.int32)
+    sc = hip_ctx.scene_create(np.full(instances, lod, np.int32), w)
+    oscene, _ = U.oracle_scene(oracle, [(v, t)], il, w)
+    rng = np.random.default_rng(2)
+    lo, hi = v.min(0), v.max(0)
+    n = 100_000
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, 0:3] = lo + (hi - lo) * rng.random((n, 3)) + [0, 0.5, 0]
+    rays[: n // 2, 1] += rng.random(n // 2) * 3
+    d = rng.normal(size=(n, 3)) * [1, 0.3, 1] - [0, 1, 0]
+    rays[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays[:, 3] = S.MAX_SCENE_SIZE
+    print("coinciding surfaces, %d instances, shift %g" % (instances, shift), flush=True)
+    gt, gi, gp, gb, st = hip_ctx.trace_closest(sc, rays)
+    ot, oi, op, ob = oracle.trace_closest(oscene, rays)
+    assert (oi >= 0).sum() > n // 5 and (st == 0).all()
+    assert np.array_equal(gi, oi) and np.array_equal(gp, op)
+    assert np.array_equal(gt.view(np.uint32), ot.view(np.uint32))
+    hit = oi >= 0
+    assert np.array_equal(gb[hit].view(np.uint32), ob[hit].view(np.uint32))
+    assert np.array_equal(hip_ctx.trace_any(sc, rays), oracle.trace_any(oscene, rays))
+
+
 @pytest.mark.parametrize("instances", [1, 40])
 def test_persistent_queue_sizes(hip_ctx, oracle, instances):
     """Rays are handed to the lanes of persistent waves: fewer rays than a
