@@ -199,39 +199,45 @@ struct TraceHit {
     unsigned nodeVisits, primTests;
 };
 
-// Closest or any hit over the reference's BVHs in its order (nearer child
-// first with ties to the left, the farther child pushed, leaves pushed as
-// (count, index)) with its compare-select slab test. The visit counts come
-// from it (kCount: internal nodes visited, an object-box test at instance
-// entry among them, and primitives tested), and it takes the rays that the
-// wide traversals hand over: rays whose slab values may be NaN (slab_finite)
-// and rays that fill the wide stack. Both are rare, so it is a call: its
-// registers and its stack burden no kernel's main path.
-template <bool kAny, bool kCount, bool kMixed>
-__device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstances, const float* worldToInst,
-                                                             const int32_t* instLod, const DevLod* lods,
-                                                             const void* tlasNodes, const int32_t* tlasPrimIds,
-                                                             int tlasNumInternal, V3 wo, V3 wd, float tmax) {
-    TraceParams p;
-    p.numInstances = numInstances;
-    p.worldToInst = worldToInst;
-    p.instLod = instLod;
-    p.lods = lods;
-    p.tlasNodes = tlasNodes;
-    p.tlasPrimIds = tlasPrimIds;
-    p.tlasNumInternal = tlasNumInternal;
-    const bool single = p.numInstances == 1;
-    int stack[kStackCap];
-    int sp = 0;
-    bool overflow = false;
-    auto push = [&](int v) {
+// Stack of the binary traversal: the lowest entries in this lane's LDS column,
+// the deeper ones in the private array `spill` of the caller (an array in here
+// would keep the scalars beside it in private memory).
+template <int kStride, int kLds>
+struct BinaryStack {
+    static constexpr int kSpill = kStackCap - kLds;
+    int* lds;
+    int sp;
+    bool overflow;
+    __device__ __forceinline__ void push(int* spill, int v) {
+        if (sp < kLds)
+            lds_at(lds, sp * kStride) = v;
+        else if (sp < kStackCap)
+            spill[sp - kLds] = v;
         if (sp < kStackCap)
-            stack[sp++] = v;
+            ++sp;
         else
             overflow = true;
-    };
-    auto pop = [&]() { return stack[--sp]; };
+    }
+    __device__ __forceinline__ int pop(const int* spill) {
+        --sp;
+        return sp < kLds ? lds_at((const int*)lds, sp * kStride) : spill[sp - kLds];
+    }
+};
 
+// Closest or any hit over the reference's BVHs in its order (nearer child
+// first with ties to the left, the farther child pushed, leaves pushed as
+// (count, index)). kInstances: 1 one instance (no instance level), 0 instance
+// level, 2 one of them at run time. kCount: the visit counts (internal nodes
+// visited, an object-box test at instance entry among them, and primitives
+// tested). kBatch primitives of a leaf are loaded before the first is tested,
+// so that a long leaf costs one memory latency per batch; the tests and hit
+// updates run in leaf order.
+template <bool kAny, bool kCount, int kInstances, bool kMixed, int kBatch, class Stack>
+__device__ __forceinline__ TraceHit binary_ray(const TraceParams& p, V3 wo, V3 wd, float tmax, Stack st) {
+    int spill[Stack::kSpill];
+    st.sp = 0;
+    st.overflow = false;
+    const bool single = kInstances == 2 ? p.numInstances == 1 : kInstances == 1;
     FastRay cur = make_fast_ray(wo, wd);
     float hitT = tmax;
     int hInst = -1, hPrim = -1;
@@ -248,6 +254,8 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
     int curInst = -1;
     int nodeAddr = 0, primCount = 2, primOffset = 0;
     bool done = false;
+    // no NaN can reach this lane's slab tests at the current level
+    bool finite = slab_finite(cur, p.tlasCoordMax);
 
     if (single) {
         DevLod lod;
@@ -257,6 +265,7 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
             primCount = 0;
         } else {
             cur = e.ray;
+            finite = slab_finite(cur, lod.coordMax);
             scale = e.scale;
             hitT = e.tmax;
             bvh = (const BvhChild*)lod.nodes;
@@ -279,14 +288,15 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
             const int lIdx = __float_as_int(q1.z), lCnt = __float_as_int(q1.w);
             const int rIdx = __float_as_int(q3.z), rCnt = __float_as_int(q3.w);
             float c0, c1;
-            const bool t0 = slab(lLo, lHi, cur, hitT, c0), t1 = slab(rLo, rHi, cur, hitT, c1);
+            bool t0, t1;
+            slab_pair(__all(finite), lLo, lHi, rLo, rHi, cur, hitT, t0, t1, c0, c1);
             if (!t0) c0 = 1e38f;
             if (!t1) c1 = 1e38f;
             if (t0 && t1) {
                 const bool farLeft = c1 < c0;
                 const int far = farLeft ? lIdx : rIdx;
-                if (far >= numInternal) push(farLeft ? lCnt : rCnt);
-                push(far);
+                if (far >= numInternal) st.push(spill, farLeft ? lCnt : rCnt);
+                st.push(spill, far);
             }
             const bool nearLeft = c0 <= c1;
             nodeAddr = nearLeft ? lIdx : rIdx;
@@ -294,10 +304,45 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
             primOffset = 0;
             if (!t0 && !t1) primCount = 0;
         }
-        if (overflow) break;
+        if (st.overflow) break;
         // the primitives of a leaf, one after the other
         bool descend = false;
         while (nodeAddr >= numInternal && primCount > 0) {
+            if (kBatch > 1 && (single || inObj)) {
+                const int first = nodeAddr - numInternal + primOffset;
+                const int nb = primCount < kBatch ? primCount : kBatch;
+                float4 ta[kBatch], tb[kBatch], tc[kBatch];
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) {
+                    if (j < nb) {
+                        const size_t id = (size_t)(first + j);
+                        ta[j] = gload(tris + 3 * id);
+                        tb[j] = gload(tris + 3 * id + 1);
+                        tc[j] = gload(tris + 3 * id + 2);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) {
+                    if (j >= nb || done) continue;
+                    float t, w0, w1;
+                    const int prim = __float_as_int(ta[j].w);
+                    if (kCount) ++primTests;
+                    if (prim_hit<kMixed>(cur, ta[j], tb[j], tc[j], first + j,
+                                 [&] { return p.lods[p.instLod[single ? 0 : curInst]].quadV3; }, t, w0, w1) &&
+                        better(t, curInst, prim, hitT, hInst, hPrim)) {
+                        hitT = t;
+                        hInst = curInst;
+                        hPrim = prim;
+                        hw0 = w0;
+                        hw1 = w1;
+                        if (kAny) done = true;
+                    }
+                }
+                primOffset += nb;
+                primCount -= nb;
+                if (done) break;
+                continue;
+            }
             const int leafId = nodeAddr - numInternal + primOffset;
             ++primOffset;
             --primCount;
@@ -329,11 +374,12 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
                     continue;
                 }
                 if (primCount > 0) {
-                    push(primCount);
-                    push(nodeAddr + primOffset);
+                    st.push(spill, primCount);
+                    st.push(spill, nodeAddr + primOffset);
                 }
-                push(kSentinel);
+                st.push(spill, kSentinel);
                 cur = e.ray;
+                finite = slab_finite(cur, lod.coordMax);
                 scale = e.scale;
                 hitT = e.tmax;
                 bvh = (const BvhChild*)lod.nodes;
@@ -353,7 +399,7 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
             float t, w0, w1;
             const int prim = __float_as_int(a.w);
             if (kCount) ++primTests;
-            if (prim_hit<kMixed>(cur, a, b, c, leafId, [&] { return p.lods[p.instLod[curInst]].quadV3; },
+            if (prim_hit<kMixed>(cur, a, b, c, leafId, [&] { return p.lods[p.instLod[single ? 0 : curInst]].quadV3; },
                                  t, w0, w1) &&
                 better(t, curInst, prim, hitT, hInst, hPrim)) {
                 hitT = t;
@@ -367,22 +413,23 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
                 }
             }
         }
-        if (done || overflow) break;
+        if (done || st.overflow) break;
         if (descend) continue;
         // pop the next subtree (or return from an object to the instance level)
-        if (sp == 0) break;
-        nodeAddr = pop();
+        if (st.sp == 0) break;
+        nodeAddr = st.pop(spill);
         if (!single && nodeAddr == kSentinel) {
-            if (sp == 0) break;
+            if (st.sp == 0) break;
             cur = make_fast_ray(wo, wd);
+            finite = slab_finite(cur, p.tlasCoordMax);
             hitT /= scale;
             scale = 1.0f;
             bvh = (const BvhChild*)p.tlasNodes;
             numInternal = p.tlasNumInternal;
             inObj = false;
-            nodeAddr = pop();
+            nodeAddr = st.pop(spill);
         }
-        primCount = (nodeAddr >= numInternal) ? pop() : 2;
+        primCount = (nodeAddr >= numInternal) ? st.pop(spill) : 2;
         primOffset = 0;
     }
     if (!kAny && inObj) hitT /= scale;  // object_to_world_space
@@ -392,18 +439,39 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
     h.prim = hPrim;
     h.w0 = hw0;
     h.w1 = hw1;
-    h.overflow = overflow;
+    h.overflow = st.overflow;
     h.nodeVisits = nodeVisits;
     h.primTests = primTests;
     return h;
 }
 
+// The same as a call, for the rays that the wide traversals hand over: rays
+// whose slab values may be NaN (slab_finite) and rays that fill the wide stack.
+// Its registers and its stack burden no kernel's main path.
+template <bool kAny, bool kMixed>
+__device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstances, const float* worldToInst,
+                                                             const int32_t* instLod, const DevLod* lods,
+                                                             const void* tlasNodes, const int32_t* tlasPrimIds,
+                                                             int tlasNumInternal, float tlasCoordMax, V3 wo, V3 wd,
+                                                             float tmax) {
+    TraceParams p;
+    p.numInstances = numInstances;
+    p.worldToInst = worldToInst;
+    p.instLod = instLod;
+    p.lods = lods;
+    p.tlasNodes = tlasNodes;
+    p.tlasPrimIds = tlasPrimIds;
+    p.tlasNumInternal = tlasNumInternal;
+    p.tlasCoordMax = tlasCoordMax;
+    return binary_ray<kAny, false, 2, kMixed, 1>(p, wo, wd, tmax, BinaryStack<1, 0>{nullptr, 0, false});
+}
+
 // The call takes the scene's pointers one by one: a reference would make the
 // kernels keep their argument block in private memory.
-template <bool kAny, bool kCount, bool kMixed>
+template <bool kAny, bool kMixed>
 __device__ __forceinline__ TraceHit reference_ray(const TraceParams& p, V3 wo, V3 wd, float tmax) {
-    return reference_call<kAny, kCount, kMixed>(p.numInstances, p.worldToInst, p.instLod, p.lods, p.tlasNodes,
-                                                p.tlasPrimIds, p.tlasNumInternal, wo, wd, tmax);
+    return reference_call<kAny, kMixed>(p.numInstances, p.worldToInst, p.instLod, p.lods, p.tlasNodes, p.tlasPrimIds,
+                                        p.tlasNumInternal, p.tlasCoordMax, wo, wd, tmax);
 }
 
 // A ray in an object's space for the wide nodes: the margin (in distance along
@@ -826,7 +894,7 @@ struct Trav {
     }
     // The hit of a ray that is done (o, d, maxT: as given to init).
     __device__ __forceinline__ TraceHit result(const TraceParams& p, V3 o, V3 d, float maxT) const {
-        if (__builtin_expect(exact, 0)) return reference_ray<kAny, false, kMixed>(p, o, d, maxT);
+        if (__builtin_expect(exact, 0)) return reference_ray<kAny, kMixed>(p, o, d, maxT);
         TraceHit h;
         h.t = hitT;
         h.inst = hInst;
