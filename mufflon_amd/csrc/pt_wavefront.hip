@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(mode_sin
     const int lanes = queue_lanes(n, waves);
     WaveQueue wq(n, lanes, queue_chunk(n, W.chunk), (int)(blockIdx.x * blockDim.x + threadIdx.x) / 64, waves,
                  W.counters + work);
-    trace_queue<T>(
+    trace_queue<T, mode_instances(kMode)>(
         wq, sStack + threadIdx.x,
         [&](int) -> const TraceParams& { return scene_ref<kBatch>(S0, W, s).trace; },
         [&](int qs, V3& o, V3& d, float& tmax) {
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(mode_sin
     WaveQueue wq(n, lanes, queue_chunk(n, W.chunk), (int)(blockIdx.x * blockDim.x + threadIdx.x) / 64, waves,
                  W.counters + work);
     if (W.neeStride == 1) {
-        trace_queue<T>(
+        trace_queue<T, mode_instances(kMode)>(
             wq, lstack, [&](int) -> const TraceParams& { return scene_ref<kBatch>(S0, W, si).trace; },
             [&](int ss, V3& o, V3& d, float& tmax) {
                 const int sl = perm ? perm[ss] : ss;

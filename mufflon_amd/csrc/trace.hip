@@ -23,7 +23,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kSingl
     using T = Trav<kAny, kSingle, kMixed, kTies, kThreads, kLdsDepth>;
     if (blockIdx.x == 0 && threadIdx.x == 0) *nextQueue = 0;
     WaveQueue q(n, lanes, chunk, (int)blockIdx.x, (int)gridDim.x, queue);
-    trace_queue<T>(
+    trace_queue<T, kSingle ? 1 : 0>(
         q, sStack + threadIdx.x, [&](int) -> const TraceParams& { return p; },
         [&](int i, V3& o, V3& d, float& tmax) {
             const float4 r0 = rays[2 * (size_t)i], r1 = rays[2 * (size_t)i + 1];
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kCountThreads) void k_trace_counts(TraceParams p, c
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4 r0 = rays[2 * (size_t)i], r1 = rays[2 * (size_t)i + 1];
-    const TraceHit h = binary_ray<false, true, kSingle ? 1 : 0, kMixed, 1>(
+    const TraceHit h = binary_ray<false, true, kSingle ? 1 : 0, kMixed>(
         p, v3(r0.x, r0.y, r0.z), v3(r1.x, r1.y, r1.z), r0.w,
         BinaryStack<kCountThreads, kLdsDepth>{sStack + threadIdx.x, 0, false});
     hits[i] = make_float4(h.t, __int_as_float(h.inst), __int_as_float(h.prim), h.overflow ? 1.0f : 0.0f);

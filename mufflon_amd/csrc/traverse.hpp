@@ -224,15 +224,42 @@ struct BinaryStack {
     }
 };
 
+// The leaves of the reference's BVH are cut into parts of at most the traversal
+// leaf limit for the wide nodes; a leaf longer than this is walked part by part
+// where nothing is counted. (A heightfield's longest leaves hold some 1400
+// triangles, a sphere's poles 570.)
+constexpr int kLongLeaf = 16;
+
+// True when the ray can hit nothing inside the box before tmax: the slab test
+// with a margin for its rounding (make_wide_ray), and on an axis along which the
+// ray does not move whether it runs beside the box. NaN makes it false.
+__device__ __forceinline__ bool surely_missed(V3 lo, V3 hi, const FastRay& r, float coordMax, float tmax) {
+    float enter = 0.0f, leave = tmax;
+    bool beside = false;
+    auto axis = [&](float l, float h, float o, float inv) {
+        const float m = (fabsf(o) + coordMax) * 0x1p-21f;
+        beside |= (o < l - m && inv <= 0.0f) || (o > h + m && inv >= 0.0f);
+        if (fabsf(inv) <= 18446744073709551616.0f) {
+            const float e = m * fabsf(inv), a = (l - o) * inv, b = (h - o) * inv;
+            enter = __builtin_fmaxf(enter, __builtin_fminf(a, b) - e);
+            leave = __builtin_fminf(leave, __builtin_fmaxf(a, b) + e);
+        } else {
+            beside |= o < l - m || o > h + m;
+        }
+    };
+    axis(lo.x, hi.x, r.o.x, r.inv.x);
+    axis(lo.y, hi.y, r.o.y, r.inv.y);
+    axis(lo.z, hi.z, r.o.z, r.inv.z);
+    return beside || enter > leave;
+}
+
 // Closest or any hit over the reference's BVHs in its order (nearer child
 // first with ties to the left, the farther child pushed, leaves pushed as
 // (count, index)). kInstances: 1 one instance (no instance level), 0 instance
 // level, 2 one of them at run time. kCount: the visit counts (internal nodes
 // visited, an object-box test at instance entry among them, and primitives
-// tested). kBatch primitives of a leaf are loaded before the first is tested,
-// so that a long leaf costs one memory latency per batch; the tests and hit
-// updates run in leaf order.
-template <bool kAny, bool kCount, int kInstances, bool kMixed, int kBatch, class Stack>
+// tested).
+template <bool kAny, bool kCount, int kInstances, bool kMixed, class Stack>
 __device__ __forceinline__ TraceHit binary_ray(const TraceParams& p, V3 wo, V3 wd, float tmax, Stack st) {
     int spill[Stack::kSpill];
     st.sp = 0;
@@ -256,6 +283,9 @@ __device__ __forceinline__ TraceHit binary_ray(const TraceParams& p, V3 wo, V3 w
     bool done = false;
     // no NaN can reach this lane's slab tests at the current level
     bool finite = slab_finite(cur, p.tlasCoordMax);
+    const float4* leafBoxes = nullptr;
+    float coordMax = 0.0f;
+    int part = 0;  // primitives left of the entered part of a long leaf
 
     if (single) {
         DevLod lod;
@@ -270,6 +300,8 @@ __device__ __forceinline__ TraceHit binary_ray(const TraceParams& p, V3 wo, V3 w
             hitT = e.tmax;
             bvh = (const BvhChild*)lod.nodes;
             tris = lod.triVerts;
+            leafBoxes = lod.leafBoxes;
+            coordMax = lod.coordMax;
             numInternal = lod.numInternal;
             inObj = true;
             curInst = 0;
@@ -308,40 +340,19 @@ __device__ __forceinline__ TraceHit binary_ray(const TraceParams& p, V3 wo, V3 w
         // the primitives of a leaf, one after the other
         bool descend = false;
         while (nodeAddr >= numInternal && primCount > 0) {
-            if (kBatch > 1 && (single || inObj)) {
-                const int first = nodeAddr - numInternal + primOffset;
-                const int nb = primCount < kBatch ? primCount : kBatch;
-                float4 ta[kBatch], tb[kBatch], tc[kBatch];
-#pragma unroll
-                for (int j = 0; j < kBatch; ++j) {
-                    if (j < nb) {
-                        const size_t id = (size_t)(first + j);
-                        ta[j] = gload(tris + 3 * id);
-                        tb[j] = gload(tris + 3 * id + 1);
-                        tc[j] = gload(tris + 3 * id + 2);
+            if (!kCount && (single || inObj)) {
+                if (part == 0 && primCount > kLongLeaf) {
+                    const float4* bx = leafBoxes + 2 * (size_t)(nodeAddr - numInternal + primOffset);
+                    const float4 b0 = gload(bx), b1 = gload(bx + 1);
+                    part = __float_as_int(b1.z);
+                    if (surely_missed(v3(b0.x, b0.y, b0.z), v3(b0.w, b1.x, b1.y), cur, coordMax, hitT)) {
+                        primOffset += part;
+                        primCount -= part;
+                        part = 0;
+                        continue;
                     }
                 }
-#pragma unroll
-                for (int j = 0; j < kBatch; ++j) {
-                    if (j >= nb || done) continue;
-                    float t, w0, w1;
-                    const int prim = __float_as_int(ta[j].w);
-                    if (kCount) ++primTests;
-                    if (prim_hit<kMixed>(cur, ta[j], tb[j], tc[j], first + j,
-                                 [&] { return p.lods[p.instLod[single ? 0 : curInst]].quadV3; }, t, w0, w1) &&
-                        better(t, curInst, prim, hitT, hInst, hPrim)) {
-                        hitT = t;
-                        hInst = curInst;
-                        hPrim = prim;
-                        hw0 = w0;
-                        hw1 = w1;
-                        if (kAny) done = true;
-                    }
-                }
-                primOffset += nb;
-                primCount -= nb;
-                if (done) break;
-                continue;
+                if (part > 0) --part;
             }
             const int leafId = nodeAddr - numInternal + primOffset;
             ++primOffset;
@@ -384,6 +395,8 @@ __device__ __forceinline__ TraceHit binary_ray(const TraceParams& p, V3 wo, V3 w
                 hitT = e.tmax;
                 bvh = (const BvhChild*)lod.nodes;
                 tris = lod.triVerts;
+                leafBoxes = lod.leafBoxes;
+                coordMax = lod.coordMax;
                 numInternal = lod.numInternal;
                 objPrims = lod.numPrims;
                 inObj = true;
@@ -446,9 +459,11 @@ __device__ __forceinline__ TraceHit binary_ray(const TraceParams& p, V3 wo, V3 w
 }
 
 // The same as a call, for the rays that the wide traversals hand over: rays
-// whose slab values may be NaN (slab_finite) and rays that fill the wide stack.
-// Its registers and its stack burden no kernel's main path.
-template <bool kAny, bool kMixed>
+// whose slab values may be NaN (slab_finite), rays that fill the wide stack and
+// rays among coinciding surfaces. Its registers and its stack burden no kernel's
+// main path. The call takes the scene's pointers one by one: a reference would
+// make the kernels keep their argument block in private memory.
+template <bool kAny, bool kMixed, int kInstances>
 __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstances, const float* worldToInst,
                                                              const int32_t* instLod, const DevLod* lods,
                                                              const void* tlasNodes, const int32_t* tlasPrimIds,
@@ -463,15 +478,12 @@ __device__ __attribute__((noinline, cold)) TraceHit reference_call(int numInstan
     p.tlasPrimIds = tlasPrimIds;
     p.tlasNumInternal = tlasNumInternal;
     p.tlasCoordMax = tlasCoordMax;
-    return binary_ray<kAny, false, 2, kMixed, 1>(p, wo, wd, tmax, BinaryStack<1, 0>{nullptr, 0, false});
+    return binary_ray<kAny, false, kInstances, kMixed>(p, wo, wd, tmax, BinaryStack<1, 0>{nullptr, 0, false});
 }
-
-// The call takes the scene's pointers one by one: a reference would make the
-// kernels keep their argument block in private memory.
-template <bool kAny, bool kMixed>
+template <bool kAny, bool kMixed, int kInstances>
 __device__ __forceinline__ TraceHit reference_ray(const TraceParams& p, V3 wo, V3 wd, float tmax) {
-    return reference_call<kAny, kMixed>(p.numInstances, p.worldToInst, p.instLod, p.lods, p.tlasNodes, p.tlasPrimIds,
-                                        p.tlasNumInternal, p.tlasCoordMax, wo, wd, tmax);
+    return reference_call<kAny, kMixed, kInstances>(p.numInstances, p.worldToInst, p.instLod, p.lods, p.tlasNodes,
+                                                    p.tlasPrimIds, p.tlasNumInternal, p.tlasCoordMax, wo, wd, tmax);
 }
 
 // A ray in an object's space for the wide nodes: the margin (in distance along
@@ -632,6 +644,8 @@ __device__ __forceinline__ ObjectData object_data(const DevLod& lod) {
 template <bool kAny, bool kSingle, bool kMixed, bool kTies, int kStride, int kLds>
 struct Trav {
     static constexpr int kSpill = kWideCap - kLds;
+    static constexpr bool kAnyHit = kAny, kMixedLods = kMixed;
+    using Binary = BinaryStack<kStride, kLds>;
     WideStack<kStride, kLds> st;
     V3 wo, wd;         // the ray in world space (kSingle: unused)
     V3 dir;            // in the entered object's space, with w
@@ -894,7 +908,12 @@ struct Trav {
     }
     // The hit of a ray that is done (o, d, maxT: as given to init).
     __device__ __forceinline__ TraceHit result(const TraceParams& p, V3 o, V3 d, float maxT) const {
-        if (__builtin_expect(exact, 0)) return reference_ray<kAny, kMixed>(p, o, d, maxT);
+        if (__builtin_expect(exact, 0))
+            return reference_ray<kAny, kMixed, kSingle ? 1 : 2>(p, o, d, maxT);
+        return hit();
+    }
+    // The same of a ray that is not exact.
+    __device__ __forceinline__ TraceHit hit() const {
         TraceHit h;
         h.t = hitT;
         h.inst = hInst;
@@ -920,6 +939,10 @@ constexpr int kTraceSingleTies = 5;  // one instance, a triangle LoD
 constexpr int kTraceModes = 6;
 constexpr bool mode_single(int mode) { return mode == kTraceSingle || mode == kTraceSingleTies; }
 constexpr bool mode_ties(int mode) { return mode != kTraceMulti && mode != kTraceSingle; }
+// binary_ray's kInstances for a mode.
+constexpr int mode_instances(int mode) {
+    return mode_single(mode) ? 1 : (mode == kTraceMulti || mode == kTraceMultiTies ? 0 : 2);
+}
 // The mode of any hits, which do not depend on the order of the leaves.
 constexpr int any_mode(int mode) {
     return mode == kTraceMultiTies ? kTraceMulti : (mode == kTraceSingleTies ? kTraceSingle : mode);
@@ -998,15 +1021,24 @@ struct WaveQueue {
 // after very different numbers of steps, so a lane whose ray has ended takes
 // the next one as soon as fewer than 5/8 of the lanes are under way; a wave
 // that runs one ray per lane spends most of its steps on its few longest.
-template <class T, class Params, class Load, class Store>
+//
+// A lane whose ray is the reference traversal's (Trav::exact) holds it until a
+// quarter of the lanes do, or the queue ends; the wave then finishes what is
+// under way and traces the held rays together, where no other traversal's
+// state is alive. (Rays with a zero component, 1M of them through a 1M-triangle
+// mesh: 0.61 ms, as a call each time 1.01; along a heightfield of 4.5M
+// triangles 35 ms, 51.) kInstances: as binary_ray's.
+template <class T, int kInstances, class Params, class Load, class Store>
 __device__ __forceinline__ void trace_queue(WaveQueue& q, int* lstack, Params params, Load load, Store store) {
     T t;
     int spill[T::kSpill];
     t.done = true;
+    t.exact = false;
     int entry = -1;
     while (true) {
+        const bool open = 4 * __popcll(__ballot(entry >= 0 && t.exact)) < q.lanes;  // takes further rays
         const u64 idle = q.takers(entry < 0);
-        if (idle != 0ull && q.left()) {
+        if (idle != 0ull && open && q.left()) {
             const int e = q.take(idle);
             V3 o, d;
             float tmax;
@@ -1015,17 +1047,26 @@ __device__ __forceinline__ void trace_queue(WaveQueue& q, int* lstack, Params pa
                 t.init(params(e), o, d, tmax, lstack);
             }
         }
-        if (__ballot(entry >= 0) == 0ull) {
-            if (!q.left()) break;
+        if (__ballot(entry >= 0 && !t.exact) == 0ull) {
+            if (__ballot(entry >= 0) == 0ull) {
+                if (!q.left()) break;
+                continue;
+            }
+            if (open && q.left()) continue;
+            if (entry >= 0) {
+                V3 o, d;
+                float tmax;
+                load(entry, o, d, tmax);
+                store(entry, binary_ray<T::kAnyHit, false, kInstances, T::kMixedLods>(params(entry), o, d, tmax,
+                                                                                     typename T::Binary{lstack, 0, false}));
+                entry = -1;
+            }
             continue;
         }
-        if (entry >= 0) {
-            t.run(params(entry), spill, q.left() ? q.lanes * 5 / 8 : 0);
-            if (t.done) {
-                V3 o = v3(0.0f, 0.0f, 0.0f), d = o;
-                float tmax = 0.0f;
-                if (__builtin_expect(t.exact, 0)) load(entry, o, d, tmax);
-                store(entry, t.result(params(entry), o, d, tmax));
+        if (entry >= 0 && !t.exact) {
+            t.run(params(entry), spill, open && q.left() ? q.lanes * 5 / 8 : 0);
+            if (t.done && !t.exact) {
+                store(entry, t.hit());
                 entry = -1;
             }
         }
