@@ -96,8 +96,9 @@ int mfh_create(int32_t deviceIndex, mfh_context** outCtx) {
             noalloc_scratch_init(deviceIndex);
             MFH_HIP(hipDeviceGetAttribute(&ctx->c.numCUs, hipDeviceAttributeMultiprocessorCount, deviceIndex));
             ctx->c.numCUs = std::max(ctx->c.numCUs, 1);
-            ctx->c.queueCounters.reserve(8);
-            MFH_HIP(hipMemsetAsync(ctx->c.queueCounters.ptr, 0, 8, ctx->c.stream));
+            ctx->c.traceQueue.split = kTraceQueueSplit;
+            ctx->c.queueCounters.reserve(ctx->c.traceQueue.bytes());
+            MFH_HIP(hipMemsetAsync(ctx->c.queueCounters.ptr, 0, ctx->c.traceQueue.bytes(), ctx->c.stream));
             ctx->c.traceQueue.counters = ctx->c.queueCounters.as<int>();
         } catch (...) {
             ctx->c.queueCounters.release();

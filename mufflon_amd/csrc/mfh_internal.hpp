@@ -173,12 +173,20 @@ struct Texture {
     DevBuf dev;
 };
 
-// Work queue of persistent kernels: two device counters that start at 0. A
-// launch takes work through one and clears the other for the launch after it
-// (all launches of a queue go to one stream).
+// Work queue of persistent kernels: two sets of `split` device counters,
+// kQueueStride ints apart, that start at 0. A launch takes work through one set
+// and clears the other for the launch after it (all launches of a queue go to one
+// stream).
+constexpr int kQueueStride = 32;  // 128 bytes, a cache line each
+constexpr int kTraceQueueSplit = 16;
 struct LaunchQueue {
     int* counters = nullptr;
+    int split = 1;
     int next = 0;
+    size_t bytes() const { return 2 * sizeof(int) * kQueueStride * (size_t)split; }
+    int* set(int k) const { return counters + (size_t)k * kQueueStride * split; }
+    int* taken() const { return set(next); }
+    int* cleared() const { return set(next ^ 1); }
 };
 
 struct Context {

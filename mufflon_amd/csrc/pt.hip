@@ -183,8 +183,8 @@ int path_work(const void* fn, int slots, int iterations, LaunchQueue& queue, int
     W.slots = slots;
     W.lanes = 64;
     while (W.lanes > kMinLanes && slots / W.lanes < resident) W.lanes /= 2;
-    W.queue = queue.counters + queue.next;
-    W.nextQueue = queue.counters + (queue.next ^ 1);
+    W.queue = queue.taken();
+    W.nextQueue = queue.cleared();
     return std::min((slots + W.lanes - 1) / W.lanes, resident);
 }
 

@@ -594,8 +594,8 @@ int mfh_pt_create(mfh_context* ctx, int32_t sceneId, const mfh_material* materia
             const size_t num = (size_t)camera->width * camera->height;
             t->dRngs.reserve(8 * num);
             t->dNan.reserve(4);
-            t->dQueue.reserve(8);
-            MFH_HIP(hipMemsetAsync(t->dQueue.ptr, 0, 8, c.stream));
+            t->dQueue.reserve(t->queue.bytes());
+            MFH_HIP(hipMemsetAsync(t->dQueue.ptr, 0, t->queue.bytes(), c.stream));
             t->queue.counters = t->dQueue.as<int>();
             reset(c, *t);
             MFH_HIP(hipStreamSynchronize(c.stream));

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(mode_sin
     int s = 0;  // this lane's scene (batches)
     const int lanes = queue_lanes(n, waves);
     WaveQueue wq(n, lanes, queue_chunk(n, W.chunk), (int)(blockIdx.x * blockDim.x + threadIdx.x) / 64, waves,
-                 W.counters + work);
+                 W.counters + work, 1);
     trace_queue<T, mode_instances(kMode)>(
         wq, sStack + threadIdx.x,
         [&](int) -> const TraceParams& { return scene_ref<kBatch>(S0, W, s).trace; },
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(mode_sin
     };
     const int lanes = queue_lanes(n, waves);
     WaveQueue wq(n, lanes, queue_chunk(n, W.chunk), (int)(blockIdx.x * blockDim.x + threadIdx.x) / 64, waves,
-                 W.counters + work);
+                 W.counters + work, 1);
     if (W.neeStride == 1) {
         trace_queue<T, mode_instances(kMode)>(
             wq, lstack, [&](int) -> const TraceParams& { return scene_ref<kBatch>(S0, W, si).trace; },

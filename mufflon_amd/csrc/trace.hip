@@ -18,11 +18,11 @@ constexpr int kCountThreads = 256;
 template <bool kAny, bool kSingle, bool kMixed, bool kTies>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kSingle ? 5 : 4))) void k_trace(
     TraceParams p, const float4* __restrict__ rays, int n, float4* __restrict__ hits, float2* __restrict__ bary,
-    int* __restrict__ occluded, int lanes, int chunk, int* queue, int* nextQueue) {
+    int* __restrict__ occluded, int lanes, int chunk, int split, int* queue, int* nextQueue) {
     __shared__ int sStack[kLdsDepth * kThreads];
     using T = Trav<kAny, kSingle, kMixed, kTies, kThreads, kLdsDepth>;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *nextQueue = 0;
-    WaveQueue q(n, lanes, chunk, (int)blockIdx.x, (int)gridDim.x, queue);
+    if (blockIdx.x == 0 && (int)threadIdx.x < kTraceQueueSplit) nextQueue[kQueueStride * (int)threadIdx.x] = 0;
+    WaveQueue q(n, lanes, chunk, (int)blockIdx.x, (int)gridDim.x, queue, split);
     trace_queue<T, kSingle ? 1 : 0>(
         q, sStack + threadIdx.x, [&](int) -> const TraceParams& { return p; },
         [&](int i, V3& o, V3& d, float& tmax) {
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(kCountThreads) void k_trace_counts(TraceParams p, c
     stats[i] = make_uint2(h.nodeVisits, h.primTests);
 }
 
-using TraceFn = void (*)(TraceParams, const float4*, int, float4*, float2*, int*, int, int, int*, int*);
+using TraceFn = void (*)(TraceParams, const float4*, int, float4*, float2*, int*, int, int, int, int*, int*);
 
 template <bool kAny, bool kSingle>
 TraceFn trace_kernel(const TraceParams& p) {
@@ -83,7 +83,7 @@ void launch_trace(TraceFn fn, const TraceParams& p, const float* rays, int n, fl
     // about four chunks a wave, at most 256 rays, so that the waves end together
     const int chunk = std::max(64, std::min(256, n / (4 * resident) / 64 * 64));
     hipLaunchKernelGGL(fn, dim3(waves), dim3(kThreads), 0, stream, p, reinterpret_cast<const float4*>(rays), n, hits,
-                       bary, occ, lanes, chunk, queue.counters + queue.next, queue.counters + (queue.next ^ 1));
+                       bary, occ, lanes, chunk, std::min(queue.split, waves), queue.taken(), queue.cleared());
     MFH_HIP(hipGetLastError());
     queue.next ^= 1;
 }
