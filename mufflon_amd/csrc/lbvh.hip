@@ -15,7 +15,7 @@
 //   k_mark      collapse decision per internal node      (build_lbvh.cu:417-463)
 //   scan        inclusive sum of the keep marks          (build_lbvh.cu:748-758)
 //   k_collapse  64-byte-node BVH with enlarged boxes     (build_lbvh.cu:503-566)
-//   k_wide      4-wide quantized nodes for the traversal kernels (LoDs)
+//               and, for LoDs, the 4-wide quantized nodes of the traversal kernels
 // Up to kSmallBuild primitives k_small_hierarchy and k_small_collapse do the
 // same in one workgroup.
 //
@@ -290,8 +290,12 @@ struct InstCost {
 // ------------------------------------------------------------- kernels
 template <class P>
 __global__ __launch_bounds__(kThreads) void k_morton(P set, int n, Box6 bb, u64* __restrict__ keys,
-                                                    i32* __restrict__ ids, float4* __restrict__ stage) {
+                                                    i32* __restrict__ ids, float4* __restrict__ stage,
+                                                    u32* __restrict__ zero, SortZeros sortZeros) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    // cleared here for the kernels after it: a launch each costs 4 us
+    if (i == 0) *zero = 0u;
+    for (int k = i; k < sortZeros.count; k += (int)(gridDim.x * blockDim.x)) sortZeros.words[k] = 0u;
     if (i >= n) return;
     V3 c;
     if constexpr (P::kStaged)
@@ -780,48 +784,48 @@ __device__ __forceinline__ void enlarged_box(float4 a, float4 b, V3& bl, V3& bh)
     bh = (hi - c) * 1.0001f + c;
 }
 
-// The reference's collapsed BVH: each kept node and leaf writes its record
-// (enlarged box, index in the collapsed numbering) into its parent.
+// A child of a binary node: its enlarged box and primitive count, and the sorted
+// position of its first primitive, if it is a leaf of a collapsed tree.
+struct NodeChild {
+    V3 lo, hi;
+    i32 count;
+    int node;
+};
 template <class C>
-__device__ __forceinline__ void collapse_node(int node, int n, const i32* __restrict__ parents,
-                                              const float4* __restrict__ boxes, const i32* offsets,
-                                              BvhChild* __restrict__ out) {
-    const int nInt = n - 1;
-    if (is_collapsed(offsets, nInt, node)) return;
-    const int nAfter = offsets[nInt - 1];
-    int parent = parents[node];
-    int off = parent < 0 ? 0 : 1;
-    if (parent < 0) parent = ~parent;
-    int fin = node;
-    if (fin >= nInt) {
-        for (int depth = 0; depth < kMaxDepth && is_collapsed(offsets, nInt, parent); ++depth) {
-            if (off == 1) return;  // only the left-most leaf writes the collapsed subtree
-            fin = parent;
-            parent = parents[parent];
-            off = parent < 0 ? 0 : 1;
-            if (parent < 0) parent = ~parent;
-        }
-    }
-    const float4 a = boxes[2 * (size_t)fin], b = boxes[2 * (size_t)fin + 1];
-    const i32 primCount = C::sum(__float_as_int(a.w));
-    const int outIdx = (offsets[parent] - 1) * 2;
-    const int outNode = (node >= nInt) ? node - nInt + nAfter : offsets[node] - 1;
-    V3 bl, bh;
-    enlarged_box(a, b, bl, bh);
-    BvhChild r;
-    r.lo[0] = bl.x; r.lo[1] = bl.y; r.lo[2] = bl.z;
-    r.hi[0] = bh.x; r.hi[1] = bh.y; r.hi[2] = bh.z;
-    r.index = outNode;
-    r.primCount = primCount;
-    out[outIdx + off] = r;
+__device__ __forceinline__ NodeChild node_child(int c, const float4* __restrict__ boxes) {
+    const float4 a = boxes[2 * (size_t)c], b = boxes[2 * (size_t)c + 1];
+    NodeChild w;
+    enlarged_box(a, b, w.lo, w.hi);
+    w.count = C::sum(__float_as_int(a.w));
+    w.node = c;
+    return w;
+}
+// First primitive of a leaf: a removed left child's index is the last of its
+// primitives, a right child's the first.
+__device__ __forceinline__ int first_primitive(const NodeChild& c, bool left, int nInt) {
+    return c.node >= nInt ? c.node - nInt : (left ? c.node - c.count + 1 : c.node);
 }
 
-template <class C>
-__global__ __launch_bounds__(kThreads) void k_collapse(int n, const i32* __restrict__ parents,
-                                                      const float4* __restrict__ boxes,
-                                                      const i32* __restrict__ offsets, BvhChild* __restrict__ out) {
-    const int node = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (node < 2 * n - 1) collapse_node<C>(node, n, parents, boxes, offsets, out);
+// The reference's collapsed BVH: a kept node's record is those of its two
+// children (enlarged box, primitive count, index in the collapsed numbering: kept
+// nodes first, then the leaves by their first primitive).
+__device__ __forceinline__ void collapse_node(int x, int nInt, const NodeChild& left, const NodeChild& right,
+                                              const i32* offsets, BvhChild* __restrict__ out) {
+    if (is_collapsed(offsets, nInt, x)) return;
+    const int nAfter = offsets[nInt - 1];
+    BvhChild* o = out + 2 * (size_t)(offsets[x] - 1);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const NodeChild& c = k == 0 ? left : right;
+        const bool inner = c.node < nInt && !is_collapsed(offsets, nInt, c.node);
+        const int index = inner ? offsets[c.node] - 1 : first_primitive(c, k == 0, nInt) + nAfter;
+        BvhChild r;
+        r.lo[0] = c.lo.x; r.lo[1] = c.lo.y; r.lo[2] = c.lo.z;
+        r.hi[0] = c.hi.x; r.hi[1] = c.hi.y; r.hi[2] = c.hi.z;
+        r.index = index;
+        r.primCount = c.count;
+        o[k] = r;
+    }
 }
 
 // ---- traversal hierarchy
@@ -842,44 +846,38 @@ struct WideChild {
     u32 ref;
 };
 
-// Child c of binary node `parent`'s side (left or right) under the keep scan.
-template <class C>
-__device__ __forceinline__ WideChild wide_child(int c, bool left, int nInt, const float4* __restrict__ boxes,
-                                                const i32* offsets, i32& count) {
-    const float4 a = boxes[2 * (size_t)c], b = boxes[2 * (size_t)c + 1];
+// A child on its parent's left or right side under the keep scan.
+__device__ __forceinline__ WideChild wide_child(const NodeChild& c, bool left, int nInt, const i32* offsets) {
     WideChild w;
-    enlarged_box(a, b, w.lo, w.hi);
-    w.node = c;
-    count = C::sum(__float_as_int(a.w));
-    if (c < nInt && !is_collapsed(offsets, nInt, c)) {
+    w.lo = c.lo;
+    w.hi = c.hi;
+    w.node = c.node;
+    if (c.node < nInt && !is_collapsed(offsets, nInt, c.node)) {
         w.area = surface(w.lo, w.hi);
-        w.ref = (u32)(offsets[c] - 1);
+        w.ref = (u32)(offsets[c.node] - 1);
     } else {
-        // a removed left child's index is the last of its leaves, a right child's the first
-        const int first = c >= nInt ? c - nInt : (left ? c - count + 1 : c);
         w.area = -1.0f;
-        w.ref = kWideLeaf | (u32)first;
+        w.ref = kWideLeaf | (u32)first_primitive(c, left, nInt);
     }
     return w;
 }
 
 template <class C>
-__device__ __forceinline__ void wide_node(int x, int n, const i32* __restrict__ children,
-                                          const float4* __restrict__ boxes, const i32* offsets,
-                                          float4* __restrict__ wide, float4* __restrict__ leafBoxes, float flatBelow,
-                                          i32* flat) {
-    const int nInt = n - 1;
+__device__ __forceinline__ void wide_node(int x, int nInt, const NodeChild& left, const NodeChild& right,
+                                          const i32* __restrict__ children, const float4* __restrict__ boxes,
+                                          const i32* offsets, float4* __restrict__ wide,
+                                          float4* __restrict__ leafBoxes, float flatBelow, i32* flat) {
     if (is_collapsed(offsets, nInt, x)) return;
     WideChild ch[4];
     int used = 2;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        i32 count;
-        ch[k] = wide_child<C>(children[2 * x + k], k == 0, nInt, boxes, offsets, count);
+        ch[k] = wide_child(k == 0 ? left : right, k == 0, nInt, offsets);
         if (ch[k].area < 0.0f) {  // the leaf's own record, from its binary parent
             const size_t at = 2 * (size_t)(ch[k].ref & ~kWideLeaf);
             leafBoxes[at] = make_float4(ch[k].lo.x, ch[k].lo.y, ch[k].lo.z, ch[k].hi.x);
-            leafBoxes[at + 1] = make_float4(ch[k].hi.y, ch[k].hi.z, __int_as_float(count), 0.0f);
+            leafBoxes[at + 1] = make_float4(ch[k].hi.y, ch[k].hi.z,
+                                            __int_as_float(k == 0 ? left.count : right.count), 0.0f);
             const V3 e = ch[k].hi - ch[k].lo;
             if (!(e.x > flatBelow && e.y > flatBelow && e.z > flatBelow)) *flat = 1;
         }
@@ -899,9 +897,9 @@ __device__ __forceinline__ void wide_node(int x, int n, const i32* __restrict__ 
 #pragma unroll
         for (int k = 1; k < open; ++k)
             if (k == best) node = ch[k].node;
-        i32 count;
-        const WideChild l = wide_child<C>(children[2 * node], true, nInt, boxes, offsets, count);
-        const WideChild r = wide_child<C>(children[2 * node + 1], false, nInt, boxes, offsets, count);
+        const int2 below = reinterpret_cast<const int2*>(children)[node];
+        const WideChild l = wide_child(node_child<C>(below.x, boxes), true, nInt, offsets);
+        const WideChild r = wide_child(node_child<C>(below.y, boxes), false, nInt, offsets);
 #pragma unroll
         for (int k = 0; k < open; ++k)
             if (k == best) ch[k] = l;
@@ -931,13 +929,15 @@ __device__ __forceinline__ void wide_node(int x, int n, const i32* __restrict__ 
         const float slack = __builtin_fmaxf(fabsf(mnv), fabsf(mxv)) * 0x1p-21f + 1e-36f;
         org[axis] = mnv - 2.0f * slack;
         scale[axis] = __builtin_fmaxf((mxv + 2.0f * slack - org[axis]) / 254.0f, 1e-38f);
+        // (one division an axis: 24 more were a fifth of the kernel's instructions)
+        const float inv = 1.0f / scale[axis];
         u32 l = 0, h = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             u32 ql = 255u, qh = 0u;
             if (k < used) {
-                ql = (u32)clampf(floorf((lo[k] - slack - org[axis]) / scale[axis]), 0.0f, 255.0f);
-                qh = (u32)clampf(ceilf((hi[k] + slack - org[axis]) / scale[axis]), 0.0f, 255.0f);
+                ql = (u32)clampf(floorf((lo[k] - slack - org[axis]) * inv), 0.0f, 255.0f);
+                qh = (u32)clampf(ceilf((hi[k] + slack - org[axis]) * inv), 0.0f, 255.0f);
             }
             l |= ql << (8 * k);
             h |= qh << (8 * k);
@@ -955,13 +955,33 @@ __device__ __forceinline__ void wide_node(int x, int n, const i32* __restrict__ 
                        __uint_as_float(used > 3 ? ch[3].ref : ch[0].ref));
 }
 
+// Both collapsed forms of binary node x, which share the loads of its children.
 template <class C>
-__global__ __launch_bounds__(kThreads) void k_wide(int n, const i32* __restrict__ children,
-                                                  const float4* __restrict__ boxes,
-                                                  const i32* __restrict__ offsets, float4* __restrict__ wide,
-                                                  float4* __restrict__ leafBoxes, float flatBelow, i32* flat) {
+__device__ __forceinline__ void collapse_both(int x, int nInt, const i32* __restrict__ children,
+                                              const float4* __restrict__ boxes, const i32* offsets,
+                                              BvhChild* __restrict__ out, const i32* offsets2,
+                                              float4* __restrict__ wide, float4* __restrict__ leafBoxes,
+                                              float flatBelow, i32* flat) {
+    const bool keep = !is_collapsed(offsets, nInt, x);
+    if (!keep && (!wide || is_collapsed(offsets2, nInt, x))) return;
+    const int2 ch = reinterpret_cast<const int2*>(children)[x];
+    const NodeChild left = node_child<C>(ch.x, boxes), right = node_child<C>(ch.y, boxes);
+    collapse_node(x, nInt, left, right, offsets, out);
+    if (wide) wide_node<C>(x, nInt, left, right, children, boxes, offsets2, wide, leafBoxes, flatBelow, flat);
+}
+
+// One thread a binary node. (600,000 triangles: 43 us; as two kernels with a
+// thread for each collapsed child and one for each wide node 25 + 40.)
+template <class C, bool kWide>
+__global__ __launch_bounds__(kThreads) void k_collapse(int n, const i32* __restrict__ children,
+                                                      const float4* __restrict__ boxes,
+                                                      const i32* __restrict__ offsets, BvhChild* __restrict__ out,
+                                                      const i32* __restrict__ offsets2, float4* __restrict__ wide,
+                                                      float4* __restrict__ leafBoxes, float flatBelow, i32* flat) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x < n - 1) wide_node<C>(x, n, children, boxes, offsets, wide, leafBoxes, flatBelow, flat);
+    if (x < n - 1)
+        collapse_both<C>(x, n - 1, children, boxes, offsets, out, offsets2, kWide ? wide : nullptr, leafBoxes,
+                         flatBelow, flat);
 }
 
 // ---- builds of 2 to kSmallBuild primitives
@@ -1089,11 +1109,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_collapse(int n, const i
         if (x < nInt) offsets[x] = at;
     }
     __syncthreads();
-    for (int node = 1 + threadIdx.x; node < 2 * n - 1; node += kSmallThreads)
-        collapse_node<C>(node, n, parents, boxes, sOff, out);
-    if (wide)
-        for (int x = threadIdx.x; x < nInt; x += kSmallThreads)
-            wide_node<C>(x, n, children, boxes, sOff2, wide, leafBoxes, flatBelow, &sFlat);
+    for (int x = threadIdx.x; x < nInt; x += kSmallThreads)
+        collapse_both<C>(x, nInt, children, boxes, sOff, out, sOff2, wide, leafBoxes, flatBelow, &sFlat);
     __syncthreads();
     if (flat && threadIdx.x == 0) *flat = sFlat;
 }
@@ -1138,7 +1155,7 @@ void fill_u32(void* p, int n, u32 v, hipStream_t st) {
     MFH_HIP(hipGetLastError());
 }
 
-// The traversal hierarchy of a build (k_wide): over the reference's collapsed
+// The traversal hierarchy of a build (wide_node): over the reference's collapsed
 // BVH with every collapsed subtree of more than refineAbove primitives kept
 // split (0: none), and the same sorted primitive records. Closest and any hit
 // do not depend on the hierarchy they are found through (the closest hit is
@@ -1192,11 +1209,10 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
         if (sink) d2h(st, sink->unsortedKeys, s.keysB.ptr, n);
     } else {
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_morton<P>), dim3(blocks_for(n)), dim3(kThreads), 0, st, set, n, bb,
-                           keys, ids, stage);
+                           keys, ids, stage, straddleCount, radix_sort_zeros(n, 0, 64, s));
         MFH_HIP(hipGetLastError());
         if (sink) d2h(st, sink->unsortedKeys, keys, n);
-        radix_sort_pairs(keys, s.keysB.as<u64>(), ids, s.idsB.as<i32>(), n, 0, 64, s, st);
-        fill_u32(straddleCount, 1, 0u, st);
+        radix_sort_pairs(keys, s.keysB.as<u64>(), ids, s.idsB.as<i32>(), n, 0, 64, s, st, true);
         if (n > 1)
             hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, keys, n, parents, children,
                                levels);
@@ -1250,13 +1266,14 @@ int build_generic(Context& ctx, BuildScratch& s, const P& set, int n, const floa
             scan_inclusive_i32_pair(offsets, offsets2, n - 1, s, st);
         else
             scan_inclusive_i32(offsets, offsets, n - 1, s, st);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_collapse<C>), dim3(blocks_for(2 * n - 2)), dim3(kThreads), 0, st, n,
-                           parents, boxes, offsets, nodes.as<BvhChild>());
-        if (wideOut) {
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wide<C>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n, children,
-                               boxes, refining ? offsets2 : offsets, wideOut->nodes->as<float4>(),
-                               wideOut->leafBoxes->as<float4>(), flatBelow, flat);
-        }
+        if (wideOut)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_collapse<C, true>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st, n,
+                               children, boxes, offsets, nodes.as<BvhChild>(), refining ? offsets2 : offsets,
+                               wideOut->nodes->as<float4>(), wideOut->leafBoxes->as<float4>(), flatBelow, flat);
+        else
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_collapse<C, false>), dim3(blocks_for(n - 1)), dim3(kThreads), 0, st,
+                               n, children, boxes, offsets, nodes.as<BvhChild>(), nullptr, nullptr, nullptr, 0.0f,
+                               nullptr);
     }
     MFH_HIP(hipGetLastError());
     i32 counts[2] = {0, 0};  // internal nodes, flat leaves

@@ -242,8 +242,15 @@ int build_lod_bvh_noalloc(Context& ctx, const float* dVerts, int numVerts, const
                           const float* bbox, void* dNodes, int32_t* dPrimIds);
 
 // Stable LSD radix sort of (u64 key, i32 value) pairs; result ends in keysA/idsA.
+// zeroed: a kernel before it has cleared the words of radix_sort_zeros.
 void radix_sort_pairs(uint64_t* keysA, uint64_t* keysB, int32_t* idsA, int32_t* idsB, int n, int beginBit,
-                      int endBit, BuildScratch& s, hipStream_t stream);
+                      int endBit, BuildScratch& s, hipStream_t stream, bool zeroed = false);
+// The words that such a sort needs cleared (null: none).
+struct SortZeros {
+    uint32_t* words;
+    int count;
+};
+SortZeros radix_sort_zeros(int n, int beginBit, int endBit, BuildScratch& s);
 // Scratch bytes a radix sort of n pairs over [beginBit, endBit) reserves:
 // digit counts (+ group sums) in BuildScratch::hist, scan partials in
 // BuildScratch::partials (callers that must not allocate size them up front).

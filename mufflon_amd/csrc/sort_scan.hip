@@ -323,21 +323,29 @@ size_t radix_sort_partials_bytes(int n) {
     return sizeof(int) * ((scanned + kScanChunk - 1) / kScanChunk + 1);
 }
 
+SortZeros radix_sort_zeros(int n, int beginBit, int endBit, BuildScratch& s) {
+    const int numTiles = (n + kRsTile - 1) / kRsTile;
+    if (n <= 1 || numTiles > kFusedTiles) return {nullptr, 0};
+    const int groups = (numTiles + kGroupTiles - 1) / kGroupTiles;
+    const int passes8 = (endBit - beginBit + 7) / 8;
+    // digit counts, then one set of group sums per pass
+    s.hist.reserve(radix_sort_hist_bytes(n, beginBit, endBit));
+    return {s.hist.as<u32>() + 256 * (size_t)numTiles, 256 * groups * passes8};
+}
+
 void radix_sort_pairs(uint64_t* keysA, uint64_t* keysB, int32_t* idsA, int32_t* idsB, int n, int beginBit,
-                      int endBit, BuildScratch& s, hipStream_t stream) {
+                      int endBit, BuildScratch& s, hipStream_t stream, bool zeroed) {
     if (n <= 1) return;
     const int numTiles = (n + kRsTile - 1) / kRsTile;
     const bool fused = numTiles <= kFusedTiles;
     const int groups = (numTiles + kGroupTiles - 1) / kGroupTiles;
-    const int passes8 = (endBit - beginBit + 7) / 8;
-    // digit counts, then (fused) one set of group sums per pass
     s.hist.reserve(radix_sort_hist_bytes(n, beginBit, endBit));
     u32* counts = s.hist.as<u32>();
-    u32* groupSums = fused ? counts + 256 * (size_t)numTiles : nullptr;
-    if (fused) {
-        const int words = 256 * groups * passes8;
-        hipLaunchKernelGGL(k_zero_u32, dim3((words + kScanThreads - 1) / kScanThreads), dim3(kScanThreads), 0,
-                           stream, groupSums, words);
+    const SortZeros zeros = radix_sort_zeros(n, beginBit, endBit, s);
+    u32* groupSums = zeros.words;
+    if (fused && !zeroed) {
+        hipLaunchKernelGGL(k_zero_u32, dim3((zeros.count + kScanThreads - 1) / kScanThreads), dim3(kScanThreads), 0,
+                           stream, groupSums, zeros.count);
     }
     u64* kin = keysA;
     u64* kout = keysB;

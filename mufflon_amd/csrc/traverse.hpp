@@ -4,7 +4,7 @@
 //
 // One ray per lane, through two levels: the instances over Mufflon's 64-byte
 // collapsed LBVH nodes in the reference's order, the primitives of an object
-// over its 4-wide traversal hierarchy (k_wide in lbvh.hip). The primitives of
+// over its 4-wide traversal hierarchy (wide_node in lbvh.hip). The primitives of
 // a leaf are contiguous 48-byte records in BVH order ({v0, primId}, {v1, kind},
 // {v2} for triangles and quads, {center, primId}, {radius, .., kind} for
 // spheres). The stack keeps its lowest kLdsDepth entries in LDS (one column
