@@ -183,6 +183,10 @@ struct LaunchQueue {
     int* counters = nullptr;
     int split = 1;
     int next = 0;
+    // Resident blocks a CU of the kernels launched so far (asking the runtime takes
+    // the host 10 us, in which the device waits for the launch).
+    std::vector<std::pair<const void*, int>> occupancy;
+    int blocks_per_cu(const void* fn, int threads);
     size_t bytes() const { return 2 * sizeof(int) * kQueueStride * (size_t)split; }
     int* set(int k) const { return counters + (size_t)k * kQueueStride * split; }
     int* taken() const { return set(next); }

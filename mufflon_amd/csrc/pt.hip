@@ -172,13 +172,11 @@ void launch_pt_init_rng(u64* rngs, int num, int seed, hipStream_t stream) {
 constexpr int kMinLanes = 8;
 
 int path_work(const void* fn, int slots, int iterations, LaunchQueue& queue, int numCUs, PathWork& W) {
-    int blocksPerCU = 0;
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocksPerCU, fn, 64, 0));
     // Lanes of a wave that take slots: all 64, or for launches too small to
     // give every resident wave 64 slots, half as many until they do. More
     // waves of fewer paths each hide one another's memory latency, and the
     // segment of a wave waits for the longest of fewer rays.
-    const int resident = std::max(blocksPerCU, 1) * numCUs;
+    const int resident = queue.blocks_per_cu(fn, 64) * numCUs;
     W.iterations = iterations;
     W.slots = slots;
     W.lanes = 64;

@@ -75,9 +75,7 @@ TraceFn trace_kernel(const TraceParams& p) {
 
 void launch_trace(TraceFn fn, const TraceParams& p, const float* rays, int n, float4* hits, float2* bary, int* occ,
                   LaunchQueue& queue, int numCUs, hipStream_t stream) {
-    int blocksPerCU = 0;
-    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocksPerCU, fn, kThreads, 0));
-    const int resident = std::max(blocksPerCU, 1) * numCUs;
+    const int resident = queue.blocks_per_cu(reinterpret_cast<const void*>(fn), kThreads) * numCUs;
     const int lanes = queue_lanes(n, resident);
     const int waves = std::min(resident, (n + lanes - 1) / lanes);
     // about four chunks a wave, at most 256 rays, so that the waves end together
@@ -89,6 +87,15 @@ void launch_trace(TraceFn fn, const TraceParams& p, const float* rays, int n, fl
 }
 
 }  // namespace
+
+int LaunchQueue::blocks_per_cu(const void* fn, int threads) {
+    for (const auto& [known, blocks] : occupancy)
+        if (known == fn) return blocks;
+    int blocks = 0;
+    MFH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, threads, 0));
+    occupancy.emplace_back(fn, std::max(blocks, 1));
+    return occupancy.back().second;
+}
 
 TraceParams trace_params(const Scene& sc) {
     TraceParams p;
