@@ -37,6 +37,19 @@ def test_launch_shapes_agree(hip_ctx, width, height):
     assert np.isfinite(one[0]).all() and (width * height < 64 or one[0].max() > 0)
 
 
+def test_calls_of_more_than_one_launch(hip_ctx):
+    """A call of more than 2^26 paths is split into launches: five iterations of a
+    4096x4096 image run as four and one, with the bits of one launch each."""
+    c = S.cornell_box(4, 8, 4096, 4096)
+    print("pt regeneration 4096x4096 x 5", flush=True)
+    pt = P.gpu_pt(hip_ctx, c, seed=5, max_path_length=1, nee_count=0)
+    one = _image(hip_ctx, pt, [5])
+    each = _image(hip_ctx, pt, [1] * 5)
+    assert np.array_equal(one[0].view(np.uint32), each[0].view(np.uint32))
+    assert np.array_equal(one[1], each[1])
+    assert one[0].max() > 0
+
+
 @pytest.mark.parametrize("depth,nee", [(0, 1), (1, 1), (4, 0), (4, 3)])
 def test_depths_and_estimates(hip_ctx, oracle, depth, nee):
     c = S.cornell_box(8, 16, 37, 21)

@@ -34,13 +34,13 @@ def terrain(hip_ctx, oracle):
     return pt, windows
 
 
-@pytest.mark.parametrize("form,leaf,sort,tail", [("megakernel", 1, 0, 0), ("megakernel", 8, 0, 0),
-                                                 ("wavefront", 1, 0, 0), ("wavefront", 8, 0, 0),
-                                                 ("wavefront", 8, 2, 0), ("wavefront", 1, 1, 3)])
-def test_terrain_windows_match_oracle(hip_ctx, terrain, form, leaf, sort, tail):
+@pytest.mark.parametrize("form,chunk,sort,tail", [("megakernel", 256, 0, 0), ("wavefront", 256, 0, 0),
+                                                  ("wavefront", 64, 0, 0), ("wavefront", 1024, 2, 0),
+                                                  ("wavefront", 256, 1, 3)])
+def test_terrain_windows_match_oracle(hip_ctx, terrain, form, chunk, sort, tail):
     pt, windows = terrain
-    print("terrain parity: %s, leaf batch %d, sorted bounces %d, tail after %d" % (form, leaf, sort, tail), flush=True)
-    hip_ctx.pt_set_tuning(pt, leaf_batch=leaf, sort_bounces=sort, tail_after=tail)
+    print("terrain parity: %s, chunk %d, sorted bounces %d, tail after %d" % (form, chunk, sort, tail), flush=True)
+    hip_ctx.pt_set_tuning(pt, queue_chunk=chunk, sort_bounces=sort, tail_after=tail)
     mode = hip.PT_MEGAKERNEL if form == "megakernel" else hip.PT_WAVEFRONT
     hip_ctx.pt_set_mode(pt, mode, form == "wavefront")
     hip_ctx.pt_reset(pt)

@@ -54,26 +54,27 @@ def test_wavefront_matches_oracle_cornell(hip_ctx, oracle):
 
 def test_wavefront_instanced_and_every_tuning(hip_ctx):
     """Instance level (TLAS traversal in the queue kernels) under every
-    trace block / stack depth and two chunk sizes, plus reset and continue."""
+    trace block / stack depth, three chunk sizes, sorted bounces and tails, plus
+    reset and continue. refillBudget and leafBatch select no code: they are
+    checked, kept and returned."""
     c = P.cornell_instanced(32)
     print("wavefront instanced, tuning sweep", flush=True)
     pt, sc = P.gpu_pt_instanced(hip_ctx, c)
     hip_ctx.pt_iterate(pt, 2)
     ref = hip_ctx.pt_target(pt)
     hip_ctx.pt_set_mode(pt, hip.PT_WAVEFRONT, True)
-    shapes = [(64, 8), (64, 16), (128, 8), (128, 16), (256, 8), (256, 16), (256, 24)]
-    for (block, depth), leaf in [(sh, 1) for sh in shapes] + [(sh, 8) for sh in shapes]:
-        for chunk, sort, refill, tail in ((64, 0, 0, 0), (1024, 3, 0, 1), (256, 0, 16, 3), (256, 2, 3, 2)):
+    for block, depth in [(64, 8), (64, 16), (128, 8), (128, 16), (256, 8), (256, 16), (256, 24)]:
+        for chunk, sort, refill, leaf, tail in ((64, 0, 0, 1, 0), (1024, 3, 0, 8, 1), (256, 0, 16, 1, 3),
+                                                (256, 2, 3, 8, 2)):
             hip_ctx.pt_set_tuning(pt, block, depth, chunk, sort, refill, leaf, tail)
             hip_ctx.pt_reset(pt)
             hip_ctx.pt_iterate(pt, 1)
             hip_ctx.pt_iterate(pt, 1)
             got = hip_ctx.pt_target(pt)
-            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (block, depth, leaf, chunk, sort, refill,
-                                                                              tail)
+            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (block, depth, chunk, sort, tail)
     assert hip_ctx.pt_get_tuning(pt) == dict(traceBlock=256, stackDepth=24, queueChunk=256, sortBounces=2,
                                              refillBudget=3, leafBatch=8, tailAfter=2)
-    # the megakernel with 8 triangles of a leaf loaded ahead
+    # the megakernel under a tuning of the wavefront
     hip_ctx.pt_set_mode(pt, hip.PT_MEGAKERNEL)
     hip_ctx.pt_reset(pt)
     hip_ctx.pt_iterate(pt, 2)
@@ -82,14 +83,32 @@ def test_wavefront_instanced_and_every_tuning(hip_ctx):
         hip_ctx.pt_set_tuning(pt, 256, 16, 256, 0, 0, 4)
 
 
+@pytest.mark.parametrize("chunk", [64, 256, 1024])
+def test_wavefront_queues_past_the_waves(hip_ctx, chunk):
+    """1.4M paths: the queues of the first bounces hold more than four chunks a
+    wave, so that chunks come from the counter instead of being dealt out, the
+    later ones fewer."""
+    c = S.cornell_box(8, 16, 1301, 1100)
+    print("wavefront 1301x1100, chunk %d" % chunk, flush=True)
+    pt = P.gpu_pt(hip_ctx, c, seed=3, max_path_length=4, nee_count=1)
+    hip_ctx.pt_iterate(pt, 1)
+    ref = hip_ctx.pt_target(pt)
+    hip_ctx.pt_set_mode(pt, hip.PT_WAVEFRONT)
+    hip_ctx.pt_set_tuning(pt, queue_chunk=chunk)
+    hip_ctx.pt_reset(pt)
+    hip_ctx.pt_iterate(pt, 1)
+    assert np.array_equal(hip_ctx.pt_target(pt).view(np.uint32), ref.view(np.uint32))
+
+
 def test_autotune_picks_a_shape_and_resets(hip_ctx):
     c = P.cornell(8, 16, 32)
     pt = P.gpu_pt(hip_ctx, c)
     hip_ctx.pt_set_mode(pt, hip.PT_WAVEFRONT, True)
+    hip_ctx.pt_set_tuning(pt, refill_budget=16, leaf_batch=8)
     best, ms = hip_ctx.pt_autotune(pt, 1)
     print("autotune best %s %.3f ms" % (best, ms), flush=True)
     assert ms > 0 and best["queueChunk"] in (256, 1024) and best["sortBounces"] in (0, 1, 2)
-    assert best["refillBudget"] in (0, 16, 32)
+    assert best["refillBudget"] == 16 and best["leafBatch"] == 8  # the caller's, unchanged
     assert hip_ctx.pt_iteration(pt) == -1
     hip_ctx.pt_iterate(pt, 2)
     a = hip_ctx.pt_target(pt)
@@ -124,10 +143,11 @@ def _with_stack(c, levels=160):
     return out
 
 
-def test_leaf_batch_on_long_leaves(hip_ctx, oracle):
-    """Leaves of up to hundreds of triangles (partial batches of 8, any-hit
-    shadow rays that stop inside a batch, ties between identical triangles):
-    megakernel and wavefront with leaf batch 1 and 8 give the oracle's bits."""
+def test_long_leaves(hip_ctx, oracle):
+    """Leaves of the reference's BVH of up to hundreds of triangles, which the
+    traversal hierarchy cuts into parts (held leaves whose records are loaded one
+    ahead, any-hit shadow rays that stop inside one, ties between identical
+    triangles): megakernel and wavefront give the oracle's bits."""
     c = _with_stack(P.cornell(8, 16, 48))
     print("long leaves: %d triangles" % len(c["tris"]), flush=True)
     lod = hip_ctx.lod_create(c["verts"], c["tris"])
@@ -144,10 +164,10 @@ def test_leaf_batch_on_long_leaves(hip_ctx, oracle):
     assert counts.max() >= 64
     ps = P.oracle_pt_scene(oracle, c, hip_ctx.pt_light_tree(pt))
     o_rad, o_hit, _ = oracle.pt_render(ps, 1, 0, 6, 2, 3)
-    for mode, leaf in ((hip.PT_MEGAKERNEL, 1), (hip.PT_MEGAKERNEL, 8), (hip.PT_WAVEFRONT, 8), (hip.PT_WAVEFRONT, 1)):
+    for mode in (hip.PT_MEGAKERNEL, hip.PT_WAVEFRONT):
         hip_ctx.pt_set_mode(pt, mode, False)
-        hip_ctx.pt_set_tuning(pt, 128, 8, 256, 0, 0, leaf)
+        hip_ctx.pt_set_tuning(pt, 128, 8, 256)
         hip_ctx.pt_reset(pt)
         hip_ctx.pt_iterate(pt, 3)
-        assert np.array_equal(hip_ctx.pt_target(pt, hip.TARGET_HIT_ID), o_hit), (mode, leaf)
-        assert np.array_equal(hip_ctx.pt_target(pt).view(np.uint32), o_rad.view(np.uint32)), (mode, leaf)
+        assert np.array_equal(hip_ctx.pt_target(pt, hip.TARGET_HIT_ID), o_hit), mode
+        assert np.array_equal(hip_ctx.pt_target(pt).view(np.uint32), o_rad.view(np.uint32)), mode

@@ -79,6 +79,41 @@ def test_wide_traversal_matches_oracle(hip_ctx, oracle, name, limit):
         assert np.array_equal(hip_ctx.trace_any(sc, rays), oracle.trace_any(oscene, rays))
 
 
+def test_full_stack(hip_ctx, oracle):
+    """45 instances that halve one axis after the other towards the origin, a
+    chain of the instance level: rays to the origin enter the inner side first
+    and leave two entries a level behind, more than the 64 of the wide stack, so
+    they are handed to the reference traversal. Others stay below."""
+    v, t = S.random_triangle_soup(300, seed=8, mu=-1.5)
+    v = np.clip(v, 0.0, 1.0).astype(np.float32)
+    v[:6] = [[0, 0, 0], [1, 1, 1], [1, 0, 1], [0, 1, 0], [1, 0, 0], [0, 1, 1]]
+    s = np.ones(3)
+    w = []
+    for k in range(45):
+        w.append(np.array([1 / s[0], 0, 0, 0, 0, 1 / s[1], 0, 0, 0, 0, 1 / s[2], 0], np.float32))
+        s[k % 3] *= 0.5
+    lod = hip_ctx.lod_create(v, t)
+    hip_ctx.lbvh_build(lod)
+    il = np.zeros(45, np.int32)
+    sc = hip_ctx.scene_create(np.full(45, lod, np.int32), np.stack(w))
+    oscene, _ = U.oracle_scene(oracle, [(v, t)], il, np.stack(w))
+    rng = np.random.default_rng(4)
+    n = 6000
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, 0:3] = rng.uniform(-1.0, -0.1, (n, 3))
+    d = rng.uniform(0, 1e-6, (n, 3)) - rays[:, 0:3]
+    d[n // 2:] += rng.uniform(0, 0.6, (n - n // 2, 3))
+    rays[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays[:, 3] = S.MAX_SCENE_SIZE
+    print("full stack", flush=True)
+    gt, gi, gp, gb, st = hip_ctx.trace_closest(sc, rays)
+    ot, oi, op, ob = oracle.trace_closest(oscene, rays)
+    assert (st == 0).all() and (oi >= 0).sum() > 1000
+    assert np.array_equal(gi, oi) and np.array_equal(gp, op)
+    assert np.array_equal(gt.view(np.uint32), ot.view(np.uint32))
+    assert np.array_equal(hip_ctx.trace_any(sc, rays), oracle.trace_any(oscene, rays))
+
+
 @pytest.mark.parametrize("shift", [0.0, 0.3, 7.7])
 @pytest.mark.parametrize("instances", [1, 2])
 def test_coinciding_surfaces(hip_ctx, oracle, instances, shift):
