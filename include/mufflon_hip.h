@@ -375,9 +375,10 @@ typedef struct mfh_wavefront_tuning {
     int32_t stackDepth;
     int32_t queueChunk;
     int32_t sortBounces;
-    int32_t refillBudget; /* 0 .. 4096 and */
-    int32_t leafBatch;    /* 1 or 8: accepted and returned by mfh_pt_get_tuning; the traversal has one
-                             form, which loads a leaf's next primitive while it tests one */
+    int32_t refillBudget; /* 0 .. 4096, and */
+    int32_t leafBatch;    /* 1 or 8: both are checked, kept and returned by mfh_pt_get_tuning and select
+                             nothing; the traversal has one form, which loads a leaf's next primitive
+                             while it tests one */
     int32_t tailAfter;    /* 0: one launch per stage and bounce; k > 0: after the extension rays of
                              bounce k one launch finishes every remaining path (megakernel-style,
                              same bits), so the last bounces of a few long paths do not cost three

@@ -39,9 +39,9 @@ constexpr int kPtThreads = kPtTile * kPtTile;
 // lane and one launch per iteration: Cornell box 256x256, 16 iterations 22.3
 // -> 10.6 ms; terrain of 2.1M triangles and 2048 instances, 1280x720, 4
 // iterations 31.5 -> 24.5 ms; one iteration of a 200x151 room 0.82 -> 0.55 ms
-// (over binary nodes; 8.4, 20.3 and 0.43 ms over the wide ones).
-// What bounds it now is the traversal's chain of dependent loads (80 % of a
-// wave's time; about 1500 cycles a node or triangle step in the Cornell box).
+// (over binary nodes; 8.7, 19.9 and 0.45 ms over the wide ones).
+// What bounds it now is the traversal's chain of dependent loads: in the Cornell
+// box the vector units are busy 48 % of the time, with 8 % of the lanes active.
 //
 // The shadow ray of a vertex is traced after the walk from it (the random
 // numbers of both are drawn before, in the order of pt_sample): through that
@@ -165,10 +165,11 @@ void launch_pt_init_rng(u64* rngs, int num, int seed, hipStream_t stream) {
     MFH_HIP(hipGetLastError());
 }
 
-// Fewest lanes of a wave that take pixels (Cornell box 256x256, 64 / 32 / 16
-// lanes: 14.1 / 12.7 / 10.6 ms; 200x151 room, 64 / 32 / 16 / 8: 0.72 / 0.63 /
-// 0.57 / 0.55 ms; the terrain image, which fills the chip, 24.5 / 34.4 / 47.5;
-// all over binary nodes).
+// Fewest lanes of a wave that take pixels (64 / 32 / 16 / 8: Cornell box 256x256,
+// 16 iterations, 11.8 / 10.7 / 8.9 / 8.7 ms, the last with 16 lanes as well by the
+// rule below; one iteration of a 200x151 room 0.57 / 0.53 / 0.50 / 0.45 ms. The
+// light tracer's Cornell box is fastest at 32: 12.2 / 11.6 / 14.1 / 14.0. The
+// terrain image fills the chip and takes 64).
 constexpr int kMinLanes = 8;
 
 int path_work(const void* fn, int slots, int iterations, LaunchQueue& queue, int numCUs, PathWork& W) {

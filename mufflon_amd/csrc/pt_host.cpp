@@ -85,7 +85,8 @@ void release_wavefront(PathTracer& t) {
     t.wfMaxLen = t.wfNee = -1;
 }
 
-// Paths of one megakernel launch, at most (a fraction of a second on a large scene).
+// Paths of one megakernel launch, at most (the terrain of 10M triangles at 1920x1080,
+// 313 Mpaths/s: 0.21 s).
 constexpr int64_t kMaxLaunchPaths = 1 << 26;
 
 // Queue chunks the autotuners try.

@@ -11,10 +11,10 @@ constexpr int kCountThreads = 256;
 
 // Persistent waves over the rays (trace_queue). kAny: stop at the first
 // accepted hit. kSingle: the scene has one instance (no instance level).
-// kMixed: the scene's LoDs hold quads or spheres. kTies: see Trav. Waves per SIMD: what the
-// persistent traversal needs itself (89 and 127 VGPRs; one wave more a SIMD
-// spills in the loop: 1M-triangle trace 1.75 instead of 1.65 ms, instanced
-// 1.64 instead of 0.92 ms). The called reference traversal would take 150.
+// kMixed: the scene's LoDs hold quads or spheres. kTies: see Trav. Waves per
+// SIMD: what the persistent traversal needs itself (up to 96 and 128 VGPRs; one
+// wave more a SIMD spills in the loop: 1M-triangle trace with its build 2.48
+// instead of 2.13 ms, instanced 1.65 instead of 0.92 ms).
 template <bool kAny, bool kSingle, bool kMixed, bool kTies>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kSingle ? 5 : 4))) void k_trace(
     TraceParams p, const float4* __restrict__ rays, int n, float4* __restrict__ hits, float2* __restrict__ bary,

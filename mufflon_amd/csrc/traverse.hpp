@@ -487,9 +487,13 @@ __device__ __forceinline__ TraceHit reference_ray(const TraceParams& p, V3 wo, V
 }
 
 // A ray in an object's space for the wide nodes: the margin (in distance along
-// the ray, per axis) covers the rounding of a quantized plane's distance and
-// of the full-precision slab test it stands for, each below 2^-23 (|origin| +
-// |coordinate|) / |direction|.
+// the ray, per axis) covers the rounding of a quantized plane's distance and of
+// the full-precision slab test it stands for. In units of 2^-23 (|origin| +
+// |coordinate|) / |direction| the slab test has three roundings, below 1; the
+// quantized plane one half each for the node's origin less the ray's, for the fma
+// that offsets it, for the last fma, and up to 1 for the scale times a byte (the
+// grid spans twice |coordinate| where the node does): 2.5. Together 3.5 of the 4
+// that the margin has, so it cannot be halved.
 struct WideRay {
     V3 o, inv, eps;
 };
@@ -629,10 +633,11 @@ __device__ __forceinline__ ObjectData object_data(const DevLod& lod) {
 // the caller can hand new rays to the lanes that are done. kSingle: one
 // instance (else the instance level, or one instance found at run time).
 //
-// (1M-triangle mesh, 2.1M camera and 2.1M incoherent rays: 2.96 ms with a ray
-// per lane over binary nodes, 2.15 over wide nodes, 1.65 with the lanes handed
-// new rays: 22 -> 39 % of the lanes active. What bounds it now is instruction
-// issue, 70 % of the time, at that utilization.)
+// (1M-triangle mesh, 2.1M camera and 2.1M incoherent rays: 2.98 ms with a ray
+// per lane over binary nodes, 1.88 over wide nodes with the lanes handed new
+// rays: 24 -> 40 % of the lanes active. What bounds it now: the vector units are
+// busy 80 % of the time at that utilization, and the L2 misses stream at the rate
+// of a large copy, 4.7 TB/s.)
 //
 // A turn of run() takes the lanes between objects to their next one (over the
 // binary nodes of the instances, in the reference's order), and the lanes
@@ -1066,8 +1071,8 @@ __device__ __forceinline__ void trace_queue(WaveQueue& q, int* lstack, Params pa
                 V3 o, d;
                 float tmax;
                 load(entry, o, d, tmax);
-                store(entry, binary_ray<T::kAnyHit, false, kInstances, T::kMixedLods>(params(entry), o, d, tmax,
-                                                                                     typename T::Binary{lstack, 0, false}));
+                const typename T::Binary stack{lstack, 0, false};
+                store(entry, binary_ray<T::kAnyHit, false, kInstances, T::kMixedLods>(params(entry), o, d, tmax, stack));
                 entry = -1;
             }
             continue;

@@ -575,7 +575,7 @@ class HipContext:
 
     def pt_set_tuning(self, pt, trace_block=256, stack_depth=16, queue_chunk=256, sort_bounces=0, refill_budget=0,
                       leaf_batch=1, tail_after=0):
-        """Wavefront launch shape; refill_budget and leaf_batch are recorded and change nothing;
+        """Wavefront launch shape; refill_budget and leaf_batch are kept and select nothing;
         tail_after > 0 finishes every path in one launch after that bounce."""
         r = np.zeros(1, TUNING_DTYPE)
         r["traceBlock"], r["stackDepth"], r["queueChunk"] = trace_block, stack_depth, queue_chunk
